@@ -34,8 +34,10 @@ __global__ __launch_bounds__(BS, 5) void k_batch(BatchTable bt, const float* __r
                                               const float* __restrict__ seed, uint32_t* __restrict__ out_idx,
                                               float* __restrict__ out_dist, uint32_t* __restrict__ err)
 {
-    __shared__ uint32_t stk[SSZ * BS];
-    __shared__ EdgeLds elds[BS / 64];
+    // closest point: a pool per wave; closest silhouette: a stack per lane
+    constexpr uint32_t POOL_WORDS = 2 * 32 * SSZ + WaveLds::FIXED;
+    __shared__ __align__(16) uint32_t stk[KIND == 0 ? POOL_WORDS * (BS / 64) : SSZ * BS];
+    __shared__ EdgeLds elds[KIND == 0 ? 1 : BS / 64];
     const uint32_t lane = threadIdx.x & 63;
     bool ovf = false;
     Counts cnt;
@@ -60,21 +62,29 @@ __global__ __launch_bounds__(BS, 5) void k_batch(BatchTable bt, const float* __r
         const uint32_t q1 = min(q0 + bt.qpw, bt.qoff[m + 1]);
         for (uint32_t base = q0; base < q1; base += 64) {
             const uint32_t slot = base + lane;
-            if (slot >= q1)
+            const bool valid = slot < q1;
+            if (KIND != 0 && !valid)
                 continue;
-            const uint32_t qi = bt.perm ? bt.perm[slot] : slot;
-            const v3 p = load_point<3>(q, qi);
+            const uint32_t qi = valid ? (bt.perm ? bt.perm[slot] : slot) : 0u;
+            const v3 p = valid ? load_point<3>(q, qi) : mk(0.0f, 0.0f, 0.0f);
             float best = F_INF;
             uint32_t bi = INVALID;
             if (KIND == 0) {
-                cp_query<BS, SSZ, false, 3>(tv, p, stk + threadIdx.x, best, bi, cnt, ovf);
+                WaveLds W(stk + (threadIdx.x / 64) * POOL_WORDS, 32 * SSZ);
+                if (valid)
+                    W.start(lane, p);
+                cp_wave<false, 3>(tv, min(64u, q1 - base), W, cnt, ovf);
+                if (!valid)
+                    continue;
+                unpack_best(W.best[lane], best, bi);
                 best = dm::sqrt_(best);
             } else {
                 float cap = SEEDED ? seed[qi] : F_INF;
                 if (!(cap >= 0.0f))
                     cap = F_INF;
                 sil_query<BS, SSZ, false, 3, SEEDED, true>(tv, p, flip != 0, cap, stk + threadIdx.x,
-                                                           &elds[threadIdx.x / 64], best, bi, cnt, ovf);
+                                                           &elds[KIND == 0 ? 0 : threadIdx.x / 64], best, bi, cnt,
+                                                           ovf);
             }
             if (out_idx)
                 out_idx[qi] = bi;

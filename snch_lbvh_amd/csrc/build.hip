@@ -878,15 +878,17 @@ struct MeshIds {
     }
 };
 
-// leaf run of an internal child covering at most leaf_size leaves
-__device__ __forceinline__ uint32_t run_of(const MeshIds& id, uint32_t node, const uint2* __restrict__ range,
-                                           uint32_t leaf_size)
+// an internal child's reference, with its leaf count when that is at most
+// leaf_size (a leaf run); a leaf's sorted position otherwise
+__device__ __forceinline__ uint32_t child_ref(const MeshIds& id, uint32_t node, const uint2* __restrict__ range,
+                                              uint32_t leaf_size)
 {
+    const uint32_t ref = id.ref(node);
     if (leaf_size <= 1 || !id.internal(node))
-        return INVALID;
+        return ref;
     const uint2 rg = range[node];
     const uint32_t cnt = rg.y - rg.x + 1;
-    return cnt <= leaf_size ? ((cnt - 1) << RUN_SHIFT) | (rg.x - id.off) : INVALID;
+    return cnt <= leaf_size ? ref | (cnt << RUN_SHIFT) : ref;
 }
 
 // the parent box and cone of two children (bvh.cuh:520-604), and the records
@@ -909,11 +911,9 @@ __device__ __forceinline__ void refit_write(const MeshIds& id, uint32_t p, uint2
     }
     const uint32_t r = p - id.off; // internal record: (off - m) + (p - nb)
     tnode[4 * r + 0] = make_float4(lb.lo.x, lb.lo.y, lb.lo.z, lb.hi.x);
-    tnode[4 * r + 1] = make_float4(lb.hi.y, lb.hi.z, rb.lo.x, rb.lo.y);
-    tnode[4 * r + 2] = make_float4(rb.lo.z, rb.hi.x, rb.hi.y, rb.hi.z);
-    tnode[4 * r + 3] = make_float4(__uint_as_float(id.ref(ch.x)), __uint_as_float(id.ref(ch.y)),
-                                   __uint_as_float(run_of(id, ch.x, range, leaf_size)),
-                                   __uint_as_float(run_of(id, ch.y, range, leaf_size)));
+    tnode[4 * r + 1] = make_float4(lb.hi.y, lb.hi.z, __uint_as_float(child_ref(id, ch.x, range, leaf_size)), 0.0f);
+    tnode[4 * r + 2] = make_float4(rb.lo.x, rb.lo.y, rb.lo.z, rb.hi.x);
+    tnode[4 * r + 3] = make_float4(rb.hi.y, rb.hi.z, __uint_as_float(child_ref(id, ch.y, range, leaf_size)), 0.0f);
     tcone[4 * r + 0] = make_float4(lc.axis.x, lc.axis.y, lc.axis.z, lc.half_angle);
     tcone[4 * r + 1] = make_float4(rc.axis.x, rc.axis.y, rc.axis.z, rc.half_angle);
     tcone[4 * r + 2] = make_float4(lc.radius, rc.radius, 0.0f, 0.0f);

@@ -190,6 +190,8 @@ snch::TreeView snch_scene::view(uint32_t m) const
     t.tcone = tcone.as<float4>() + 4 * (size_t)(off - m);
     // the trig-free cone test is conservative only with the enclosing radius
     t.flags = (dim == 3 && !(build_flags & SNCH_BUILD_REFERENCE_RADIUS)) ? TREE_FAST_CONE : 0u;
+    if (leaf_size > 1)
+        t.flags |= TREE_RUNS;
     uint32_t vd = 0;
     const float d2 = m < mesh_diag2.size() ? mesh_diag2[m] : 0.0f;
     std::memcpy(&vd, &d2, sizeof(vd));
@@ -440,6 +442,26 @@ snch_scene::~snch_scene()
 }
 
 namespace {
+// the device copies of the meshes' views after a build with this leaf size
+hipError_t refresh_views(snch_scene* s, uint32_t leaf)
+{
+    s->leaf_size = leaf;
+    std::vector<TreeView> views(s->n_meshes);
+    for (uint32_t m = 0; m < s->n_meshes; ++m)
+        views[m] = s->view(m);
+    const hipError_t e = s->batch.views.ensure(sizeof(TreeView) * views.size());
+    return e != hipSuccess ? e : hipMemcpy(s->batch.views.p, views.data(), sizeof(TreeView) * views.size(),
+                                           hipMemcpyHostToDevice);
+}
+
+// build_tree and the views of its tree (hipMemcpy waits for the copy, not for
+// the build: both use device memory that the build does not touch)
+hipError_t rebuild(snch_scene* s, uint32_t flags, uint32_t leaf, hipStream_t st)
+{
+    const hipError_t e = build_tree(s, flags, leaf, st);
+    return e != hipSuccess ? e : refresh_views(s, leaf);
+}
+
 // capture build_tree once into a graph (on a private stream); false when
 // capture or instantiation fails, and the caller builds eagerly
 bool capture_build(snch_scene* s, uint32_t flags, uint32_t leaf, hipStream_t st)
@@ -547,17 +569,8 @@ int snch_scene_build(snch_scene* s, const snch_build_opts* opts, void* stream)
     if (const int rc = check_device_errors("snch_scene_build"))
         return rc;
     s->build_flags = flags;
-    {
-        std::vector<TreeView> views(s->n_meshes);
-        for (uint32_t m = 0; m < s->n_meshes; ++m)
-            views[m] = s->view(m);
-        SNCH_HIP(s->batch.views.ensure(sizeof(TreeView) * views.size()), "snch_scene_build: views");
-        SNCH_HIP(hipMemcpy(s->batch.views.p, views.data(), sizeof(TreeView) * views.size(), hipMemcpyHostToDevice),
-                 "snch_scene_build: views");
-    }
+    SNCH_HIP(refresh_views(s, leaf), "snch_scene_build: views");
     s->built = true;
-    s->build_flags = flags;
-    s->leaf_size = leaf;
     ++s->build_gen;
     s->last_build_ms = ms;
     return SNCH_OK;
@@ -638,7 +651,7 @@ int snch_closest_point_ex(const snch_scene* s, const float* q, uint32_t n, uint3
         SNCH_HIP(query_order(s->view(), (int)s->dim, q, n, s->qscratch, st, &perm), "snch_closest_point: ordering");
     }
     SNCH_HIP(launch_closest_point(s->view(), (int)s->dim, q, n, out_idx, out_dist, block, depth, perm,
-                                  opts ? opts->stats : nullptr, st),
+                                  opts ? opts->stats : nullptr, s->n_cu(), st),
              "snch_closest_point");
     if (own_order)
         SNCH_HIP(scratch_end(s, st), "snch_closest_point: event");
@@ -908,7 +921,7 @@ int snch_batch_autotune(snch_scene* s, uint32_t kind, const float* q, const uint
     // the others held at their best so far
     const uint32_t flags = s->build_flags;
     float best_ms = 0.0f;
-    if ((err = build_tree(s, flags, 1, st)) == hipSuccess)
+    if ((err = rebuild(s, flags, 1, st)) == hipSuccess)
         err = measure(cur, &best_ms);
     cur.ms_default = best_ms;
     cur.n_tried = 1;
@@ -920,7 +933,7 @@ int snch_batch_autotune(snch_scene* s, uint32_t kind, const float* q, const uint
         float ms = 0.0f;
         snch_tune_result c = cur;
         c.leaf_size = L;
-        if ((err = build_tree(s, flags, L, st)) == hipSuccess && (err = measure(c, &ms)) == hipSuccess) {
+        if ((err = rebuild(s, flags, L, st)) == hipSuccess && (err = measure(c, &ms)) == hipSuccess) {
             ++cur.n_tried;
             if (ms < best_ms) {
                 best_ms = ms;
@@ -929,7 +942,7 @@ int snch_batch_autotune(snch_scene* s, uint32_t kind, const float* q, const uint
         }
     }
     if (err == hipSuccess)
-        err = build_tree(s, flags, cur.leaf_size, st);
+        err = rebuild(s, flags, cur.leaf_size, st);
     for (int axis = 0; axis < 3 && err == hipSuccess; ++axis) {
         const uint32_t* vals = axis == 0 ? blocks : axis == 1 ? depths : qpws;
         const int nv = axis == 2 ? 3 : 4;
@@ -958,7 +971,6 @@ int snch_batch_autotune(snch_scene* s, uint32_t kind, const float* q, const uint
         err = hipStreamSynchronize(st);
     if (err != hipSuccess)
         return hip_fail(err, "snch_batch_autotune");
-    s->leaf_size = cur.leaf_size;
     ++s->build_gen;
     cur.ms = best_ms;
     *out = cur;
@@ -1069,11 +1081,12 @@ int snch_scene_export_mesh(const snch_scene* s, uint32_t mesh, uint32_t* nodes, 
             const float* t = &tn[16 * (size_t)r];
             const float* c = &tc[16 * (size_t)r];
             uint32_t ref[2];
-            std::memcpy(ref, t + 12, sizeof(ref));
+            std::memcpy(&ref[0], t + 6, sizeof(uint32_t));
+            std::memcpy(&ref[1], t + 14, sizeof(uint32_t));
             const float llo[3] = {t[0], t[1], t[2]}, lhi[3] = {t[3], t[4], t[5]};
-            const float rlo[3] = {t[6], t[7], t[8]}, rhi[3] = {t[9], t[10], t[11]};
-            const uint32_t node[2] = {(ref[0] & LEAF_BIT) ? (N - 1) + (ref[0] & ~LEAF_BIT) : ref[0],
-                                      (ref[1] & LEAF_BIT) ? (N - 1) + (ref[1] & ~LEAF_BIT) : ref[1]};
+            const float rlo[3] = {t[8], t[9], t[10]}, rhi[3] = {t[11], t[12], t[13]};
+            const uint32_t node[2] = {((ref[0] & LEAF_BIT) ? N - 1 : 0) + (ref[0] & REF_MASK),
+                                      ((ref[1] & LEAF_BIT) ? N - 1 : 0) + (ref[1] & REF_MASK)};
             if (node[0] < NN)
                 put(node[0], llo, lhi, c + 0, c[3], c[8]);
             if (node[1] < NN)

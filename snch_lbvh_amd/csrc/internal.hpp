@@ -54,6 +54,7 @@ struct snch_context {
 
 struct snch_scene {
     snch_context* ctx = nullptr;
+    uint32_t n_cu() const { return ctx && ctx->n_cu > 0 ? (uint32_t)ctx->n_cu : 256u; }
     uint32_t dim = 3;
     uint32_t n_meshes = 1;
     // per-mesh offsets (n_meshes + 1 each): primitives, vertices, silhouette
@@ -141,7 +142,7 @@ size_t query_order_scratch_bytes(uint32_t n);
 hipError_t query_order_in(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* words, hipStream_t st,
                           const uint32_t** perm, uint32_t* err);
 hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* idx, float* dist,
-                                uint32_t block, uint32_t depth, const uint32_t* perm, uint64_t* stats,
+                                uint32_t block, uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t n_cu,
                                 hipStream_t st);
 // seed (nullable): per-query radius.  capped: a hard radius (answers beyond
 // it are not searched; the returned distance is then larger than the

@@ -5,15 +5,17 @@
 // query_device, query.cuh:79-423, and sample_object_in_sphere,
 // sample.cuh:23-92).  Differences in HOW, not WHAT:
 //  * Node layout: one 64-B record per internal node holds both children's
-//    boxes and references; the silhouette query reads a 48-B cone record from
-//    a separate stream, so the closest-point and ray queries never touch it.
-//  * Stack: closest point, closest silhouette and rays keep a short per-lane
-//    stack in LDS (16 packed entries, a column per lane so a wave's 64 lanes
-//    hit distinct banks) with a restart trail (TrailStack): nothing in
-//    private memory; a far child pushed out of the full stack is found again
-//    from the trail.  The generic overlap and line queries, which must emit
-//    hits in the reference's visit order, keep 16 LDS entries over a private
-//    overflow array (the tree depth is at most 64, so it never loses one).
+//    boxes and references, 32 B each; the silhouette query reads a cone record
+//    from a separate stream, so the closest-point and ray queries never touch
+//    it.
+//  * The closest-point search runs a wave's queries from one pool of pending
+//    nodes in LDS (wave_search.hpp).  Rays keep a short per-lane stack in LDS
+//    (16 packed entries, a column per lane so a wave's 64 lanes hit distinct
+//    banks) with a restart trail (TrailStack): nothing in private memory; a
+//    far child pushed out of the full stack is found again from the trail.
+//    The generic overlap and line queries, which must emit hits in the
+//    reference's visit order, keep 16 LDS entries over a private overflow
+//    array (the tree depth is at most 64, so it never loses one).
 //  * Order: the nearer child is descended first and the farther is pushed,
 //    and a child is skipped when its lower bound exceeds the best answer so
 //    far.  The reference's own pruning predicates (minmaxdist for closest
@@ -35,31 +37,40 @@ namespace {
 constexpr int OVF = 64; // private overflow entries per lane (generic queries)
 
 // ------------------------------------------------------------ closest point
-template <int BS, bool STATS, int DIM, int SSZ>
-__global__ __launch_bounds__(BS) void k_closest_point(TreeView t, const float* __restrict__ q, uint32_t n,
-                                                      uint32_t* __restrict__ out_idx, float* __restrict__ out_dist,
-                                                      const uint32_t* __restrict__ perm, uint32_t* __restrict__ err,
-                                                      unsigned long long* stats)
+// One wave per chunk of qpw queries.  qpw = 64: consecutive queries of the
+// visiting order.  qpw < 64 (a launch that 64 per wave would leave too few
+// waves for): every n_waves-th query, so that costly neighbours (the centre
+// of a sphere) land in different waves.
+template <bool STATS, int DIM>
+__global__ __launch_bounds__(512, 6) void k_closest_point(TreeView t, const float* __restrict__ q, uint32_t n,
+                                                          uint32_t qpw, uint32_t cap, uint32_t* __restrict__ out_idx,
+                                                          float* __restrict__ out_dist,
+                                                          const uint32_t* __restrict__ perm,
+                                                          uint32_t* __restrict__ err, unsigned long long* stats)
 {
-    __shared__ uint32_t stk[SSZ * BS];
-    const uint32_t slot = xcd_remap(blockIdx.x, gridDim.x) * BS + threadIdx.x;
-    Counts cnt;
+    extern __shared__ __align__(16) uint32_t smem[];
+    const uint32_t lane = threadIdx.x & 63, wpb = blockDim.x >> 6, w = threadIdx.x >> 6;
+    WaveLds W(smem + w * (2 * cap + WaveLds::FIXED), cap);
     if (t.n_dev)
         n = min(n, *t.n_dev);
-    if (slot >= n) {
-        if (STATS)
-            flush_counts(cnt, stats);
-        return;
-    }
-    const uint32_t qi = perm ? min(perm[slot], n - 1) : slot;
-    float best;
-    uint32_t best_idx;
+    const uint32_t chunk = uniform(xcd_remap(blockIdx.x, gridDim.x) * wpb + w), n_waves = gridDim.x * wpb;
+    const uint32_t slot = qpw < 64u ? lane * n_waves + chunk : chunk * 64u + lane;
+    const bool valid = lane < qpw && slot < n;
+    const uint32_t qi = valid ? (perm ? min(perm[slot], n - 1) : slot) : 0u;
+    if (valid)
+        W.start(lane, load_point<DIM>(q, qi));
     bool ovf = false;
-    cp_query<BS, SSZ, STATS, DIM>(t, load_point<DIM>(q, qi), stk + threadIdx.x, best, best_idx, cnt, ovf);
+    Counts cnt;
+    cp_wave<STATS, DIM>(t, (uint32_t)__popcll(__ballot(valid)), W, cnt, ovf);
     if (ovf && err)
         atomicOr(err, 1u);
-    out_idx[qi] = best_idx;
-    out_dist[qi] = dm::sqrt_(best);
+    if (valid) {
+        float best;
+        uint32_t best_idx;
+        unpack_best(W.best[lane], best, best_idx);
+        out_idx[qi] = best_idx;
+        out_dist[qi] = dm::sqrt_(best);
+    }
     if (STATS)
         flush_counts(cnt, stats);
 }
@@ -133,7 +144,7 @@ __global__ __launch_bounds__(BS) void k_ray(TreeView t, const float* __restrict_
             const bool Lh = bL && Ld <= tbest;
             const bool Rh = bR && Rd <= tbest;
             uint32_t lf, lc, rf, rc;
-            const bool lLeaf = as_leaf(nr.lref, nr.lrun, lf, lc), rLeaf = as_leaf(nr.rref, nr.rrun, rf, rc);
+            const bool lLeaf = as_leaf(nr.lref, 0u, lf, lc), rLeaf = as_leaf(nr.rref, 1u, rf, rc);
             // nearer child first, as query.cuh:136-149
             const bool rfirst = Lh && Rh && Rd < Ld;
             if (rfirst) {
@@ -399,15 +410,15 @@ __global__ __launch_bounds__(BS) void k_generic(TreeView t, const float* __restr
             const NodeRec nr = load_node(t.tnode, st.pop());
             if (hit_box(nr.L)) {
                 if (nr.lref & LEAF_BIT)
-                    emit(nr.lref & ~LEAF_BIT);
+                    emit(nr.lref & REF_MASK);
                 else
-                    st.push(nr.lref);
+                    st.push(nr.lref & REF_MASK);
             }
             if (hit_box(nr.R)) {
                 if (nr.rref & LEAF_BIT)
-                    emit(nr.rref & ~LEAF_BIT);
+                    emit(nr.rref & REF_MASK);
                 else
-                    st.push(nr.rref);
+                    st.push(nr.rref & REF_MASK);
             }
         }
         if (st.overflow && err)
@@ -479,41 +490,31 @@ hipError_t query_order_in(const TreeView& t, int dim, const float* q, uint32_t n
     return hipGetLastError();
 }
 
-template <int BS, int DIM, int SSZ>
-static void launch_cp_cfg(const TreeView& t, const float* q, uint32_t n, uint32_t* idx, float* dist,
-                          const uint32_t* perm, unsigned long long* stats, hipStream_t st)
+// queries per wave of a launch of n: 64, or fewer when that leaves resident
+// waves without work
+static uint32_t queries_per_wave(uint32_t n, uint32_t resident_waves)
 {
-    if (stats)
-        hipLaunchKernelGGL((k_closest_point<BS, true, DIM, SSZ>), dim3(nblocks(n, BS)), dim3(BS), 0, st, t, q, n, idx,
-                           dist, perm, traversal_error_word(), stats);
-    else
-        hipLaunchKernelGGL((k_closest_point<BS, false, DIM, SSZ>), dim3(nblocks(n, BS)), dim3(BS), 0, st, t, q, n,
-                           idx, dist, perm, traversal_error_word(), stats);
-}
-
-template <int BS, int DIM>
-static void launch_cp_bs(const TreeView& t, const float* q, uint32_t n, uint32_t* idx, float* dist, uint32_t depth,
-                         const uint32_t* perm, unsigned long long* stats, hipStream_t st)
-{
-    if (DIM == 3 && depth == 8)
-        launch_cp_cfg<BS, DIM, 8>(t, q, n, idx, dist, perm, stats, st);
-    else
-        launch_cp_cfg<BS, DIM, 16>(t, q, n, idx, dist, perm, stats, st);
+    return std::min(64u, std::max(1u, nblocks(n, std::max(resident_waves, 1u))));
 }
 
 hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* idx, float* dist,
-                                uint32_t block, uint32_t depth, const uint32_t* perm, uint64_t* stats, hipStream_t st)
+                                uint32_t block, uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t n_cu,
+                                hipStream_t st)
 {
     if (n == 0)
         return hipSuccess;
     auto* sp = reinterpret_cast<unsigned long long*>(stats);
+    const uint32_t wpb = block / 64, cap = 32 * depth;
+    const size_t lds = sizeof(uint32_t) * wpb * wave_lds_words(depth);
+    const uint32_t qpw = t.n_dev ? 64u : queries_per_wave(n, n_cu * (uint32_t)(LDS_PER_CU / lds) * wpb);
+    const dim3 g(nblocks(nblocks(n, qpw), wpb)), b(block);
     SNCH_DISPATCH_DIM(dim, {
-        switch (block) {
-        case 128: launch_cp_bs<128, DIM>(t, q, n, idx, dist, depth, perm, sp, st); break;
-        case 256: launch_cp_bs<256, DIM>(t, q, n, idx, dist, depth, perm, sp, st); break;
-        case 512: launch_cp_bs<512, DIM>(t, q, n, idx, dist, depth, perm, sp, st); break;
-        default: launch_cp_bs<64, DIM>(t, q, n, idx, dist, depth, perm, sp, st); break;
-        }
+        if (stats)
+            hipLaunchKernelGGL((k_closest_point<true, DIM>), g, b, lds, st, t, q, n, qpw, cap, idx, dist, perm,
+                               traversal_error_word(), sp);
+        else
+            hipLaunchKernelGGL((k_closest_point<false, DIM>), g, b, lds, st, t, q, n, qpw, cap, idx, dist, perm,
+                               traversal_error_word(), sp);
     });
     return hipGetLastError();
 }

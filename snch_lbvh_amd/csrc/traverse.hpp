@@ -16,39 +16,47 @@ struct Counts {
 
 struct NodeRec {
     box3 L, R;
-    uint32_t lref, rref, lrun, rrun;
+    uint32_t lref, rref;
 };
 
 __device__ __forceinline__ NodeRec load_node(const float4* __restrict__ tnode, uint32_t i)
 {
-    const float4 a = tnode[4 * i], b = tnode[4 * i + 1], c = tnode[4 * i + 2], r = tnode[4 * i + 3];
+    const float4 a = tnode[4 * i], b = tnode[4 * i + 1], c = tnode[4 * i + 2], d = tnode[4 * i + 3];
     NodeRec n;
     n.L.lo = mk(a.x, a.y, a.z);
     n.L.hi = mk(a.w, b.x, b.y);
-    n.R.lo = mk(b.z, b.w, c.x);
-    n.R.hi = mk(c.y, c.z, c.w);
-    n.lref = __float_as_uint(r.x);
-    n.rref = __float_as_uint(r.y);
-    n.lrun = __float_as_uint(r.z);
-    n.rrun = __float_as_uint(r.w);
+    n.lref = __float_as_uint(b.z);
+    n.R.lo = mk(c.x, c.y, c.z);
+    n.R.hi = mk(c.w, d.x, d.y);
+    n.rref = __float_as_uint(d.z);
     return n;
 }
 
-// a child the traversal treats as a leaf: a true leaf, or a run of sorted
-// leaves [first, first + count) under an internal node (leaf size > 1)
-__device__ __forceinline__ bool as_leaf(uint32_t ref, uint32_t run, uint32_t& first, uint32_t& count)
+// one child of a node (side 0: left, 1: right)
+struct ChildRec {
+    box3 box;
+    uint32_t ref;
+};
+__device__ __forceinline__ ChildRec load_child(const float4* __restrict__ tnode, uint32_t i, uint32_t side)
 {
-    if (ref & LEAF_BIT) {
-        first = ref & ~LEAF_BIT;
-        count = 1;
-        return true;
-    }
-    if (run != INVALID) {
-        first = run & RUN_FIRST_MASK;
-        count = (run >> RUN_SHIFT) + 1;
-        return true;
-    }
-    return false;
+    const float4 a = tnode[4 * i + 2 * side], b = tnode[4 * i + 2 * side + 1];
+    ChildRec c;
+    c.box.lo = mk(a.x, a.y, a.z);
+    c.box.hi = mk(a.w, b.x, b.y);
+    c.ref = __float_as_uint(b.z);
+    return c;
+}
+
+// a child the traversal treats as a leaf: a true leaf, or a run of sorted
+// leaves [first, first + count) under an internal node (leaf size > 1).  An
+// internal left child (side 0) is numbered by its last leaf, a right one by
+// its first (Karras: the children of a split at g are nodes g and g + 1).
+__device__ __forceinline__ bool as_leaf(uint32_t ref, uint32_t side, uint32_t& first, uint32_t& count)
+{
+    const uint32_t id = ref & REF_MASK, run = (ref >> RUN_SHIFT) & RUN_BITS;
+    count = run ? run : 1u;
+    first = run && side == 0u ? id + 1u - run : id;
+    return (ref & LEAF_BIT) || run;
 }
 
 __device__ __forceinline__ box3 ldbox2(const float4* nb, uint32_t n)
@@ -159,7 +167,7 @@ __device__ __forceinline__ void sample_one(const TreeView& t, const float4* __re
     uint32_t ref = t.n_leaves == 1 ? LEAF_BIT : 0u;
     for (int depth = 0; depth < 96; ++depth) { // a single descent: at most the tree depth
         if (ref & LEAF_BIT) {
-            const uint32_t j = ref & ~LEAF_BIT;
+            const uint32_t j = ref & REF_MASK;
             if (j >= t.n_leaves)
                 break;
             const float4 a = t.tleaf[3 * j], b = t.tleaf[3 * j + 1], d = t.tleaf[3 * j + 2];
@@ -171,9 +179,10 @@ __device__ __forceinline__ void sample_one(const TreeView& t, const float4* __re
             }
             break;
         }
-        if (ref >= t.n_leaves - 1)
+        const uint32_t node = ref & REF_MASK;
+        if (node >= t.n_leaves - 1)
             break;
-        const NodeRec nr = load_node(t.tnode, ref);
+        const NodeRec nr = load_node(t.tnode, node);
         const float Lw = box_sphere(nr.L, c, r)
                              ? (DIM == 3 ? green_weight(c, box_centroid(nr.L)) : green_weight2d(c, box_centroid(nr.L)))
                              : 0.0f;
@@ -236,7 +245,7 @@ __device__ inline void dev_nearest(const TreeView& t, v3 p, float& best, uint32_
         const float Lmm = box_minmaxdist(nr.L, p), Rmm = box_minmaxdist(nr.R, p);
         const bool cL = Lmd <= Rmm, cR = Rmd <= Lmm; // query.cuh:279, :297
         uint32_t lf, lc, rf, rc;
-        const bool lLeaf = as_leaf(nr.lref, nr.lrun, lf, lc), rLeaf = as_leaf(nr.rref, nr.rrun, rf, rc);
+        const bool lLeaf = as_leaf(nr.lref, 0u, lf, lc), rLeaf = as_leaf(nr.rref, 1u, rf, rc);
         if (cL && lLeaf && Lmd <= best)
             for (uint32_t k = 0; k < lc; ++k)
                 cp_leaf<DIM>(t, lf + k, p, best, best_idx);
@@ -307,7 +316,7 @@ __device__ inline void dev_nearest_silhouette(const TreeView& t, v3 p, bool flip
             }
         }
         uint32_t lf, lc, rf, rc;
-        const bool lLeaf = as_leaf(nr.lref, nr.lrun, lf, lc), rLeaf = as_leaf(nr.rref, nr.rrun, rf, rc);
+        const bool lLeaf = as_leaf(nr.lref, 0u, lf, lc), rLeaf = as_leaf(nr.rref, 1u, rf, rc);
         if (hL && lLeaf)
             for (uint32_t k = 0; k < lc; ++k)
                 sil_leaf<DIM>(t, lf + k, p, flip, best, best_e, cnt);
@@ -389,7 +398,7 @@ __device__ inline bool dev_ray(const TreeView& t, v3 ro, v3 rd, float max_dist, 
         const bool Lh = box_ray(nr.L, ro, inv, max_dist, Ld) && Ld <= tbest;
         const bool Rh = box_ray(nr.R, ro, inv, max_dist, Rd) && Rd <= tbest;
         uint32_t lf, lc, rf, rc;
-        const bool lLeaf = as_leaf(nr.lref, nr.lrun, lf, lc), rLeaf = as_leaf(nr.rref, nr.rrun, rf, rc);
+        const bool lLeaf = as_leaf(nr.lref, 0u, lf, lc), rLeaf = as_leaf(nr.rref, 1u, rf, rc);
         const bool rfirst = Lh && Rh && Rd < Ld; // nearer child first, as query.cuh:136-149
         if (rfirst) {
             if (Rh && rLeaf)

@@ -11,18 +11,16 @@ namespace snch {
 // ---------------------------------------------------------------------------
 // HBM layout of a built tree (N leaves, N-1 internal nodes, E silhouette edges)
 //
-//   tnode[i]  4 x float4 = 64 B per internal node i (64-B aligned): the boxes
-//             of BOTH children plus their references, so one visit is one
-//             64-B load:
-//               [0] L.lo.x L.lo.y L.lo.z L.hi.x
-//               [1] L.hi.y L.hi.z R.lo.x R.lo.y
-//               [2] R.lo.z R.hi.x R.hi.y R.hi.z
-//               [3] ref(L) ref(R) run(L) run(R)
-//             ref(c) = c for an internal child, LEAF_BIT | j for the leaf in
-//             sorted position j.  run(c) = INVALID, or, when the tree is
-//             built with leaf size k > 1 and internal child c covers at most
-//             k leaves, (count - 1) << 27 | first: the traversal queries then
-//             treat c as one leaf holding sorted leaves [first, first + count).
+//   tnode[i]  4 x float4 = 64 B per internal node i (64-B aligned): 32 B for
+//             each child, so one visit is one 64-B line, and a pair of lanes
+//             reads one child each:
+//               [0] L.lo.x L.lo.y L.lo.z L.hi.x  [1] L.hi.y L.hi.z ref(L) 0
+//               [2] R.lo.x R.lo.y R.lo.z R.hi.x  [3] R.hi.y R.hi.z ref(R) 0
+//             ref(c): bits 0-23 the internal child's id, or with LEAF_BIT the
+//             sorted position of the leaf.  Bits 24-27 are 0, or, when the
+//             tree is built with leaf size k > 1 and internal child c covers
+//             at most k leaves, their count: the traversal queries then treat
+//             c as one leaf holding that run of sorted leaves (as_leaf).
 //   tcone[i]  4 x float4 = 64 B per internal node: the children's normal
 //             cones, read only by the silhouette query:
 //               [0] L.axis L.half_angle  [1] R.axis R.half_angle
@@ -45,16 +43,17 @@ namespace snch {
 // the batch of one, with every offset zero.  Records hold mesh-local ids.
 // ---------------------------------------------------------------------------
 constexpr uint32_t LEAF_BIT = 0x80000000u;
-constexpr uint32_t RUN_SHIFT = 27;
-constexpr uint32_t RUN_FIRST_MASK = (1u << RUN_SHIFT) - 1u;
+constexpr uint32_t REF_MASK = 0x00FFFFFFu;
+constexpr uint32_t RUN_SHIFT = 24, RUN_BITS = 15u;
 constexpr uint32_t MAX_LEAF_SIZE = 8;
-constexpr uint32_t MAX_MESH_PRIMS = 1u << 24; // node ids fit the 24-bit field of a packed stack entry
+constexpr uint32_t MAX_MESH_PRIMS = 1u << 24; // node ids fit the 24-bit fields of child references and pending-node entries
 
 struct MeshDesc {
     uint32_t off, n, eoff, nb;
 };
 
 constexpr uint32_t TREE_FAST_CONE = 1u; // TreeView::flags: cone_overlap_fast may replace cone_overlap
+constexpr uint32_t TREE_RUNS = 2u;      // children may be leaf runs (built with leaf size > 1)
 
 struct TreeView {
     uint32_t n_leaves;

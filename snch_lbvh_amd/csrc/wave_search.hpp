@@ -13,13 +13,17 @@ namespace snch {
 
 namespace {
 
-constexpr int SS = 16; // default LDS stack entries per lane
+constexpr int SS = 16; // LDS stack entries per lane (rays)
+constexpr uint32_t LDS_PER_CU = 160 * 1024;
 
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb)
 {
     const uint32_t X = 8, q = nb / X, r = nb % X, x = b % X, k = b / X;
     return x * q + (x < r ? x : r) + k;
 }
+
+// wave-uniform copy of lane 0's value (a scalar register)
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // A short stack with a restart trail (Laine 2010, "Restart trail for
 // stackless BVH traversal"), for searches whose pruning bound only tightens:
@@ -72,6 +76,12 @@ struct TrailStack {
         const uint32_t q = v > qbase ? min(v - qbase, 255u) : 0u;
         return (n << 8) | q;
     }
+    // the lower bound stored in an entry
+    __device__ __forceinline__ float key(uint32_t e) const
+    {
+        const uint32_t q = e & 255u;
+        return q ? __uint_as_float((q + qbase) << 20) : 0.0f;
+    }
     __device__ __forceinline__ void push(uint32_t n, float d, uint32_t k)
     {
         lds[(top % SSZ) * BS] = enc(n, d);
@@ -87,8 +97,7 @@ struct TrailStack {
         --top;
         const uint32_t e = lds[(top % SSZ) * BS];
         n = e >> 8;
-        const uint32_t q = e & 255u;
-        d = q ? __uint_as_float((q + qbase) << 20) : 0.0f;
+        d = key(e);
         const uint32_t k = 63u - (uint32_t)__clzll(M);
         const uint64_t kb = 1ull << k;
         M &= ~kb;
@@ -160,79 +169,314 @@ __device__ __forceinline__ void flush_counts(const Counts& c, unsigned long long
     }
 }
 
+// ------------------------------------------------------------ pooled search
+// One wave answers up to 64 queries from a pool of pending nodes in LDS.  An
+// item is (query slot, internal node) with the lower bound it was pushed
+// with; a step pops the last 32 items, one pair of lanes each, and each lane
+// tests one child of its item.  Surviving internal children are pushed, near
+// ones on top, and surviving leaves go to a buffer that the wave evaluates 64
+// at a time.  Each query's best answer and pruning bound live in LDS and are
+// updated by atomic minima on (distance bits, id).  Against a stack per lane (one query per lane, the
+// wave as slow as its slowest lane, a lane as slow as its chain of dependent
+// loads) every lane has work until the wave's last query ends, a node's two
+// children share one 64-B line per pair of lanes, and leaf code runs on full
+// waves.  Queries enter as the pool runs low: POOL_ADD at a time keeps few
+// queries, and so few pending nodes, in flight (all 64 at once fill the pool
+// and leave it popping one item at a time: 218 instead of 33 ms on the case
+// below, with one lane per item; 4 or 16 at a time 33.5 and 34.6).
+//
+// Closest point, one lane per query with a stack -> pool: 2^22 queries on
+// 2^20 triangles 46 -> 26 ms (VALU issue 0.78 of the SIMD cycles, 582 nodes
+// per query), 65,536 on 20,480 triangles 2.1 -> 0.18 ms, 1,000 on 20,480
+// triangles 0.83 -> 0.03 ms (there a launch lasted as long as the longest
+// chain of dependent loads, about 2 us a node).
+//
+// The answer is that of the search one lane would make alone, near child
+// first, each node's leaves at once, which skips a box as soon as its lower
+// bound exceeds the best distance so far (lane_nearest below).  Where no
+// rounding interferes that is the smallest (distance, id) of all leaves,
+// whatever the order.  But a leaf's computed distance can lie below its box's
+// computed lower bound by a few units in the last place of the coordinates
+// ("hidden" leaves): among candidates that close, what the lone search finds
+// first decides.  So the pool prunes with bounds widened by more than that
+// rounding, which leaves no such candidate out, and where a hidden leaf has
+// the smallest distance the lane repeats the search alone, from the widened
+// bound (a few dozen nodes).
+constexpr uint32_t POOL_ADD = 8;
+constexpr uint32_t LEAF_CAP = 128; // leaf buffer entries: below 64 before a step, which adds at most 64
+
+// smaller is better: the distance, ties to the smaller id (distances are not negative)
+__device__ __forceinline__ unsigned long long pack_best(float d, uint32_t id)
+{
+    return ((unsigned long long)__float_as_uint(d) << 32) | id;
+}
+__device__ __forceinline__ void unpack_best(unsigned long long v, float& d, uint32_t& id)
+{
+    d = __uint_as_float((uint32_t)(v >> 32));
+    id = (uint32_t)v;
+}
+// lanes of mask below this one
+__device__ __forceinline__ uint32_t rank_in(uint64_t mask)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+// the value of the other lane of this lane's pair (lane ^ 1)
+__device__ __forceinline__ float pair_other(float v)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0xB1, 0xF, 0xF, true));
+}
+
+// LDS of one wave, carved from the block's dynamic LDS: cap pool items (2
+// words each: slot << 24 | node, key), the leaf buffer (2 words per entry:
+// slot << 24 | leaf, key), and per query slot its answer, point, widened
+// (squared) bound and the smallest distance of a hidden leaf
+struct WaveLds {
+    unsigned long long* best;
+    uint32_t *pool, *leaf, *bound, *hidden;
+    float* q; // x, y, z rows of 64
+    uint32_t cap;
+    static constexpr uint32_t FIXED = 128 + 2 * LEAF_CAP + 128 + 192; // words besides the pool
+    __device__ __forceinline__ WaveLds(uint32_t* base, uint32_t cap_)
+    {
+        best = reinterpret_cast<unsigned long long*>(base);
+        pool = base + 128;
+        leaf = pool + 2 * cap_;
+        bound = leaf + 2 * LEAF_CAP;
+        hidden = bound + 64;
+        q = reinterpret_cast<float*>(hidden + 64);
+        cap = cap_;
+    }
+    __device__ __forceinline__ v3 point(uint32_t s) const { return mk(q[s], q[64 + s], q[128 + s]); }
+    __device__ __forceinline__ void start(uint32_t s, v3 p)
+    {
+        q[s] = p.x;
+        q[64 + s] = p.y;
+        q[128 + s] = p.z;
+        best[s] = pack_best(F_INF, INVALID);
+        bound[s] = hidden[s] = __float_as_uint(F_INF);
+    }
+};
+// a distance widened by more than the rounding of any distance to the scene
+// from p (scale: the scene's largest coordinate; in 2D also the offset of the
+// boxes), squared
+template <int DIM>
+__device__ __forceinline__ float widened(float d, v3 p, float scale)
+{
+    const float delta = (DIM == 3 ? 5e-7f : 2.0f * BVH_OFFSET) +
+                        1e-6f * fmx(scale, fmx(dm::fabs_(p.x), fmx(dm::fabs_(p.y), dm::fabs_(p.z))));
+    const float u = d * 1.000002f + delta;
+    return u * u;
+}
+__device__ __forceinline__ float scene_scale(const TreeView& t)
+{
+    const box3 b = ldbox2(t.nbox, 0);
+    return fmx(fmx(fmx(dm::fabs_(b.lo.x), dm::fabs_(b.hi.x)), fmx(dm::fabs_(b.lo.y), dm::fabs_(b.hi.y))),
+               fmx(dm::fabs_(b.lo.z), dm::fabs_(b.hi.z)));
+}
+// words of dynamic LDS of a wave with `depth` pool items per lane pair
+inline uint32_t wave_lds_words(uint32_t depth) { return 2 * 32 * depth + WaveLds::FIXED; }
+
+// append (a, key) of the lanes with `yes` to a list of two-word entries (the
+// callers' sizes never exceed the list: pool_take, LEAF_CAP)
+__device__ __forceinline__ void list_push(uint32_t* list, uint32_t& size, bool yes, uint32_t a, float key)
+{
+    const uint64_t m = __builtin_amdgcn_ballot_w64(yes);
+    const uint32_t at = size + rank_in(m);
+    if (yes) {
+        list[2 * at] = a;
+        list[2 * at + 1] = __float_as_uint(key);
+    }
+    size += (uint32_t)__popcll(m);
+}
+
+// how many items to pop so that their children fit: 32, fewer near the
+// pool's end, and one at a time in its reserve of 64 (a depth-first search of
+// one item needs at most one place per tree level)
+__device__ __forceinline__ uint32_t pool_take(uint32_t size, uint32_t cap)
+{
+    const uint32_t room = cap - 64, k = min(32u, size);
+    return size + k <= room ? k : size < room ? min(k, room - size) : 1u;
+}
+
 // ------------------------------------------------------------ closest point
 
-// query_device(nearest) (query.cuh:238-318) for one query point; best is the
-// squared distance
-template <int BS, int SSZ, bool STATS, int DIM>
-__device__ __forceinline__ void cp_query(const TreeView& t, v3 p, uint32_t* stk_col, float& best,
-                                         uint32_t& best_idx, Counts& cnt, bool& overflow)
+// query_device(nearest) (query.cuh:238-318) by one lane: near child first,
+// each node's leaves at once, with only nodes within the squared distance w.
+// st: 128 words of LDS (a stack of 64 nodes and keys: a path of a Karras tree
+// holds at most 64 internal nodes).
+template <int DIM>
+__device__ inline void lane_nearest(const TreeView& t, v3 p, float w, uint32_t* st, float& best, uint32_t& best_idx)
 {
     best = F_INF;
     best_idx = INVALID;
-    if (t.n_leaves == 1) {
-        cp_leaf<DIM>(t, 0, p, best, best_idx);
-        return;
-    }
-    TrailStack<BS, SSZ> st;
-    st.init(stk_col, t.qbase);
-    uint32_t node = 0;
-    // a pass visits each internal node at most once, restarts add the paths
-    // above lost far children; the cap and the range checks only guard
-    // against a malformed tree (hitting the cap is reported as an overflow)
-    const uint32_t cap_iters = 8 * t.n_leaves + 8192;
-    uint32_t it = 0;
-    for (; it < cap_iters && node < t.n_leaves - 1; ++it) {
+    uint32_t sp = 0, node = 0;
+    for (uint32_t it = 0; it < 2 * t.n_leaves + 64 && node < t.n_leaves - 1; ++it) {
         const NodeRec nr = load_node(t.tnode, node);
         const float Lmd = box_mindist(nr.L, p), Rmd = box_mindist(nr.R, p);
         const float Lmm = box_minmaxdist(nr.L, p), Rmm = box_minmaxdist(nr.R, p);
         const bool cL = Lmd <= Rmm, cR = Rmd <= Lmm; // query.cuh:279, :297
         uint32_t lf, lc, rf, rc;
-        const bool lLeaf = as_leaf(nr.lref, nr.lrun, lf, lc), rLeaf = as_leaf(nr.rref, nr.rrun, rf, rc);
-        if (STATS) {
-            cnt.node += 1;
-            cnt.box += 2;
-        }
-        if (cL && lLeaf && Lmd <= best) {
-            if (STATS)
-                cnt.leaf += lc;
+        const bool lLeaf = as_leaf(nr.lref, 0u, lf, lc), rLeaf = as_leaf(nr.rref, 1u, rf, rc);
+        if (cL && lLeaf && Lmd <= fmn(best, w))
             for (uint32_t k = 0; k < lc; ++k)
                 cp_leaf<DIM>(t, lf + k, p, best, best_idx);
-        }
-        if (cR && rLeaf && Rmd <= best) {
-            if (STATS)
-                cnt.leaf += rc;
+        if (cR && rLeaf && Rmd <= fmn(best, w))
             for (uint32_t k = 0; k < rc; ++k)
                 cp_leaf<DIM>(t, rf + k, p, best, best_idx);
-        }
-        const bool gL = cL && !lLeaf && Lmd <= best;
-        const bool gR = cR && !rLeaf && Rmd <= best;
-        if ((gL || gR) && st.lv >= 63u) {
-            overflow = true; // deeper than a Karras tree can be
-            break;
-        }
+        const float b = fmn(best, w);
+        const bool gL = cL && !lLeaf && Lmd <= b, gR = cR && !rLeaf && Rmd <= b;
         const bool lfirst = Lmd <= Rmd;
-        if (st.descend(lfirst ? gL : gR, lfirst ? gR : gL, lfirst ? nr.lref : nr.rref, lfirst ? nr.rref : nr.lref,
-                       lfirst ? Rmd : Lmd, node))
+        if (gL && gR && sp < 64u) {
+            st[2 * sp] = lfirst ? nr.rref : nr.lref;
+            st[2 * sp + 1] = __float_as_uint(lfirst ? Rmd : Lmd);
+            ++sp;
+        }
+        if (gL || gR) {
+            node = gL && (lfirst || !gR) ? nr.lref : nr.rref;
             continue;
+        }
         bool found = false;
-        while (st.M) {
-            uint32_t nn;
-            float dd;
-            st.pop(nn, dd);
-            if (dd <= best) { // query.cuh:259
-                node = nn;
-                found = true;
-                break;
+        while (sp > 0 && !found) {
+            --sp;
+            node = st[2 * sp];
+            found = __uint_as_float(st[2 * sp + 1]) <= b; // query.cuh:259
+        }
+        if (!found)
+            break;
+    }
+}
+
+// evaluates the last (up to 64) leaves of the wave's buffer; returns how many are left
+template <bool STATS, int DIM>
+__device__ __forceinline__ uint32_t cp_leaves(const TreeView& t, WaveLds& W, uint32_t nleaf, float scale, Counts& cnt)
+{
+    const uint32_t lane = threadIdx.x & 63, k = min(64u, nleaf);
+    nleaf -= k;
+    if (lane < k) {
+        const uint32_t w = W.leaf[2 * (nleaf + lane)], slot = w >> 24;
+        const float key = __uint_as_float(W.leaf[2 * (nleaf + lane) + 1]), b = __uint_as_float(W.bound[slot]);
+        if (key <= b) {
+            if (STATS)
+                cnt.leaf += 1;
+            const v3 p = W.point(slot);
+            float d = F_INF;
+            uint32_t id = INVALID;
+            cp_leaf<DIM>(t, w & REF_MASK, p, d, id);
+            if (id != INVALID && d <= b) {
+                atomicMin(&W.best[slot], pack_best(d, id));
+                atomicMin(&W.bound[slot], __float_as_uint(widened<DIM>(HwMath::sqrt(d), p, scale)));
+                if (key > d)
+                    atomicMin(&W.hidden[slot], __float_as_uint(d));
             }
         }
-        if (found)
-            continue;
-        if (!st.restart())
-            break;
-        node = 0;
     }
-    overflow = overflow || it >= cap_iters;
+    return nleaf;
+}
+
+// query_device(nearest) (query.cuh:238-318) for the points in slots [0, nq)
+// of a wave (WaveLds::start): W.best receives (squared distance, index).  Run
+// by the whole wave.  Every box has geometry on (in 2D, within BVH_OFFSET of)
+// each of its faces, so its minmaxdist bounds the answer from above: besides
+// the reference's test against the sibling (query.cuh:279, :297) it lowers
+// the query's bound before any leaf is reached.
+template <bool STATS, int DIM>
+__device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds& W, Counts& cnt, bool& overflow)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    if (t.n_leaves == 1) {
+        if (lane < nq) {
+            float d = F_INF;
+            uint32_t id = INVALID;
+            cp_leaf<DIM>(t, 0, W.point(lane), d, id);
+            W.best[lane] = pack_best(d, id);
+        }
+        return;
+    }
+    const float scale = scene_scale(t);
+    uint32_t size = 0, nleaf = 0, next = 0;
+    // every iteration pops a node of some query (each at most once) or
+    // evaluates leaves; the bound only guards against a malformed tree
+    const uint32_t cap_iters = 128u * t.n_leaves + 65536u;
+    for (uint32_t it = 0;; ++it) {
+        const bool fed = next >= nq;
+        if (nleaf >= 64u || (nleaf > 0u && fed && size < 32u)) {
+            nleaf = cp_leaves<STATS, DIM>(t, W, nleaf, scale, cnt);
+            continue;
+        }
+        if (size == 0u && fed)
+            break;
+        if (it >= cap_iters) {
+            overflow = true;
+            break;
+        }
+        if (size < 32u && !fed) {
+            const uint32_t add = min(POOL_ADD, nq - next);
+            list_push(W.pool, size, lane < add, (next + lane) << 24, 0.0f);
+            next += add;
+        }
+        const uint32_t k = pool_take(size, W.cap), side = lane & 1u;
+        size -= k;
+        uint32_t slot = 0, ref = 0;
+        float md = F_INF, mm = F_INF, b = 0.0f;
+        bool live = false;
+        v3 p = mk(0.0f, 0.0f, 0.0f);
+        if ((lane >> 1) < k) {
+            const uint32_t at = size + (lane >> 1), w = W.pool[2 * at], node = w & REF_MASK;
+            slot = w >> 24;
+            b = __uint_as_float(W.bound[slot]);
+            live = __uint_as_float(W.pool[2 * at + 1]) <= b && node < t.n_leaves - 1;
+            if (live) {
+                p = W.point(slot);
+                const ChildRec c = load_child(t.tnode, node, side);
+                ref = c.ref;
+                md = box_mindist(c.box, p);
+                mm = box_minmaxdist_fast(c.box, p);
+                if (STATS) {
+                    cnt.node += side;
+                    cnt.box += 1;
+                }
+            }
+        }
+        const float mo = pair_other(mm), m2 = fmn(mm, mo);
+        if (live && m2 < b) {
+            const float u = widened<DIM>(HwMath::sqrt(m2), p, scale);
+            if (u < b) {
+                if (side)
+                    atomicMin(&W.bound[slot], __float_as_uint(u));
+                b = u;
+            }
+        }
+        uint32_t first, count;
+        const bool go = live && md <= mo && md <= b, leaf = as_leaf(ref, side, first, count);
+        const float other = pair_other(md);
+        const bool lt = md < other, eq = md == other, near = lt || (eq && !side);
+        list_push(W.pool, size, go && !leaf && !near, (slot << 24) | (ref & REF_MASK), md);
+        list_push(W.pool, size, go && !leaf && near, (slot << 24) | (ref & REF_MASK), md);
+        list_push(W.leaf, nleaf, go && leaf, (slot << 24) | first, md);
+        for (uint32_t j = 1; (t.flags & TREE_RUNS) && __ballot(go && leaf && j < count); ++j) {
+            if (nleaf >= 64u)
+                nleaf = cp_leaves<STATS, DIM>(t, W, nleaf, scale, cnt);
+            list_push(W.leaf, nleaf, go && leaf && j < count, (slot << 24) | (first + j), md);
+        }
+    }
+    // the pool is empty: its memory holds the stacks of the lone searches
+    bool alone = false;
+    if (lane < nq) {
+        const uint32_t d = (uint32_t)(W.best[lane] >> 32);
+        alone = d < __float_as_uint(F_INF) && W.hidden[lane] == d;
+    }
+    for (uint64_t todo = __ballot(alone); todo; todo = __ballot(alone)) {
+        const uint32_t r = rank_in(todo);
+        if (alone && r < W.cap / 64u) {
+            const v3 p = W.point(lane);
+            float d;
+            uint32_t id;
+            lane_nearest<DIM>(t, p, widened<DIM>(HwMath::sqrt(__uint_as_float(W.bound[lane])), p, scale),
+                              W.pool + 128 * r, d, id);
+            W.best[lane] = pack_best(d, id);
+            alone = false;
+        }
+    }
 }
 
 // ------------------------------------------------------------ silhouette
@@ -415,8 +659,8 @@ __device__ __forceinline__ void sil_query(const TreeView& t, v3 p, bool flip, fl
             }
             lref = nr.lref;
             rref = nr.rref;
-            lLeaf = as_leaf(nr.lref, nr.lrun, lf, lc);
-            rLeaf = as_leaf(nr.rref, nr.rrun, rf, rc);
+            lLeaf = as_leaf(nr.lref, 0u, lf, lc);
+            rLeaf = as_leaf(nr.rref, 1u, rf, rc);
             leaves = (hL && lLeaf) || (hR && rLeaf);
             decide = !leaves;
         }
@@ -480,9 +724,6 @@ __device__ __forceinline__ void sil_query(const TreeView& t, v3 p, bool flip, fl
     }
     overflow = overflow || it >= cap_iters;
 }
-
-// wave-uniform copy of lane 0's value (a scalar register)
-__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // the next 64-query chunk of nchunks for a one-wave block of a persistent
 // launch: its own XCD's contiguous range first (x0: the block's XCD), then

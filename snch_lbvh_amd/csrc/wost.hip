@@ -319,7 +319,7 @@ hipError_t enqueue_steps(snch_wost* s, uint32_t max_steps, float eps, uint64_t s
         hipLaunchKernelGGL(k_apply_order, dim3(nb), dim3(256), 0, st, s->w, cur, cap,
                            in_alt ? s->oidx_alt.as<uint32_t>() : s->oidx.as<uint32_t>());
         hipLaunchKernelGGL(k_gather, dim3(nb), dim3(256), 0, st, s->w, cur, cap);
-        if ((e = launch_closest_point(vd, 3, s->w.qpos, cap, s->w.cp_idx, s->w.cp_dist, 64, 16, nullptr, nullptr, st)) != hipSuccess)
+        if ((e = launch_closest_point(vd, 3, s->w.qpos, cap, s->w.cp_idx, s->w.cp_dist, 64, 16, nullptr, nullptr, n_cu, st)) != hipSuccess)
             return e;
         // the silhouette within the star radius bound (the closest-point
         // distance) on a persistent launch: capped searches vary widely in length

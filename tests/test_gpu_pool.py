@@ -1,0 +1,58 @@
+"""The pooled wave searches at the edges of their launch shapes: answers do not
+depend on how many queries share a wave, on the pool's size or on leaf runs,
+also where a mesh far from the origin makes box bounds and distances round
+differently (many candidates within a few units in the last place)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _meshes():
+    from snch_lbvh_amd import workloads as W
+
+    V, F = W.icosphere(3, 0.02, seed=1)
+    B, sides, caps = W.slab_box(12)  # axis-aligned, coplanar triangles
+    return {
+        "ico": (V, F),
+        "ico_far": (V + np.float32([96.0, -40.0, 7.0]), F),
+        "box_far": (B + np.float32([24.0, 3.0, 0.0]), np.concatenate([sides, caps])),
+        "two": (V[F[:2].ravel()], np.arange(6, dtype=np.int32).reshape(2, 3)),
+    }
+
+
+def _points(V, n, seed):
+    from snch_lbvh_amd import workloads as W
+
+    lo, hi = W.padded_box(V, 0.3)
+    q = W.uniform_points(n, lo, hi, seed)
+    # exact ties: points straight above vertices and on them
+    r = np.random.default_rng(seed)
+    at = V[r.integers(0, len(V), n // 8)]
+    q[: n // 16] = at[: n // 16] * np.float32([1, 1, 1]) + np.float32([0, 0, 0.25])
+    q[n // 16: n // 8] = at[n // 16: n // 8]
+    return q[r.permutation(n)]
+
+
+@pytest.mark.parametrize("name", ["ico", "ico_far", "box_far", "two"])
+@pytest.mark.parametrize("leaf_size", [1, 3, 8])
+def test_closest_point_does_not_depend_on_the_launch(name, leaf_size):
+    import oracle
+    import snch_lbvh_amd as S
+
+    V, F = _meshes()[name]
+    q = _points(V, 70000, 11)
+    sc = S.Scene(V, F).build_bvh(leaf_size=leaf_size)
+    i0, d0 = (x.cpu().numpy() for x in sc.closest_point(q))  # 64 queries a wave, Morton order
+    for n in (1, 2, 8, 9, 63, 64, 65, 1000):
+        i1, d1 = (x.cpu().numpy() for x in sc.closest_point(q[:n]))
+        np.testing.assert_array_equal(d1, d0[:n])
+        np.testing.assert_array_equal(i1, i0[:n])
+    for kw in ({"block_size": 512}, {"block_size": 128, "stack_depth": 8}, {"coherent": 2}):
+        i1, d1 = (x.cpu().numpy() for x in sc.closest_point(q, **kw))
+        np.testing.assert_array_equal(d1, d0)
+        np.testing.assert_array_equal(i1, i0)
+    # FP32 rounding of a distance between points of this size: a few units in
+    # the last place of the coordinates
+    ref = oracle.bf_closest_point(V, F, q[:2000])[1]
+    assert np.abs(d0[:2000] - ref).max() <= 8 * np.spacing(np.abs(q).max())
