@@ -63,11 +63,8 @@ typedef struct snch_build_opts {
 
 /* Traversal tuning (chosen by the autotuner; defaults are safe) */
 typedef struct snch_query_opts {
-    uint32_t block_size; /* threads per block: 64, 128, 256 or 512; 0 = default (64).  The
-                            closest silhouette without a seed (or with a hard cap) runs, at
-                            block size 64 and stack depth 16, as a persistent launch whose
-                            wavefronts take 64-query chunks; other shapes launch one block
-                            per chunk.  Outputs are the same. */
+    uint32_t block_size; /* threads per block: 64, 128, 256 or 512; 0 = default (64).  Outputs
+                            are the same. */
     uint32_t coherent;   /* visiting order: 0 = Morton order of the query points when
                             n >= SNCH_ORDER_MIN_QUERIES, 1 = always Morton order,
                             2 = input order.  Results are written in input order and
@@ -77,20 +74,17 @@ typedef struct snch_query_opts {
                             visited, cone records read (silhouette query only) */
     const uint32_t *order; /* optional DEVICE permutation of [0, n) (e.g. from
                               snch_query_order): the visiting order; overrides coherent */
-    uint32_t stack_depth;      /* LDS stack entries per lane: closest point 8 or 16 (0 = 16),
-                                  closest silhouette (3D) and batched queries 8, 16, 24 or
-                                  32 (0 = 16) */
+    uint32_t stack_depth;      /* LDS of a wavefront's pool of pending nodes, 40 nodes per unit:
+                                  closest point 8 or 16 (0 = 16), closest silhouette (3D) and
+                                  batched queries 8, 16, 24 or 32 (0 = 16).  Outputs are the same. */
     uint32_t queries_per_wave; /* batched queries: queries a wavefront takes from the work
                                   queue at a time, a multiple of 64 up to 4096 (0 = 64) */
     uint32_t seed_is_cap;      /* closest silhouette: 1 = seed_radius is a hard search radius
                                   (the answer is exact when it lies within the radius; otherwise
                                   the returned distance exceeds the radius, possibly +inf) */
-    uint32_t seed_retry;       /* closest silhouette with seed_radius (not a cap): 0 = queries not
-                                  settled within their radius are queued (one queue per XCD) and
-                                  searched again 64 at a time by whole wavefronts of the same
-                                  persistent launch (default;
-                                  block size 64 and stack depth 16 only), 1 = each is searched again
-                                  at once by its own lane.  Outputs are the same. */
+    uint32_t seed_retry;       /* kept for callers that set it; no effect: queries not settled
+                                  within their seed radius are searched again by the same
+                                  wavefront, all its lanes at once */
 } snch_query_opts;
 
 const char *snch_last_error(void);

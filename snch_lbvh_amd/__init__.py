@@ -299,9 +299,8 @@ class Scene:
         """query_device(nearest_silhouette) (query.cuh:325-423) over q (n x dim).
         seed_radius: optional per-query pruning radius (a learned bound); the
         outputs equal the unseeded call's.  Queries not settled within it are
-        re-queued for whole wavefronts of the same launch, or with
-        seed_in_place searched again at once by their own lane.  seed_is_cap
-        makes the radius a hard search radius."""
+        searched again by the same wavefront (seed_in_place changes nothing).
+        seed_is_cap makes the radius a hard search radius."""
         import torch
 
         q = _dev_f32(q, self.dim, self.device)

@@ -26,69 +26,56 @@ struct BatchTable {
     uint32_t n_sched, total_chunks, qpw;
 };
 
-// SEEDED (closest silhouette): seed[qi] is the query's pruning radius (a
-// learned bound); the search within it is exact, a query not settled there
-// searches again from the root, so results equal the unseeded ones
-template <int BS, int SSZ, int KIND, bool SEEDED>
-__global__ __launch_bounds__(BS, 5) void k_batch(BatchTable bt, const float* __restrict__ q, int flip,
-                                              const float* __restrict__ seed, uint32_t* __restrict__ out_idx,
-                                              float* __restrict__ out_dist, uint32_t* __restrict__ err)
+// KIND 0: closest point.  1: closest silhouette.  2: closest silhouette with
+// a per-query pruning hint seed[qi]; results equal the unseeded ones
+template <int KIND>
+__global__ __launch_bounds__(512, 6) void k_batch(BatchTable bt, uint32_t cap, const float* __restrict__ q, int flip,
+                                                  const float* __restrict__ seed, uint32_t* __restrict__ out_idx,
+                                                  float* __restrict__ out_dist, uint32_t* __restrict__ err)
 {
-    // closest point: a pool per wave; closest silhouette: a stack per lane
-    constexpr uint32_t POOL_WORDS = 2 * 32 * SSZ + WaveLds::FIXED;
-    __shared__ __align__(16) uint32_t stk[KIND == 0 ? POOL_WORDS * (BS / 64) : SSZ * BS];
-    __shared__ EdgeLds elds[KIND == 0 ? 1 : BS / 64];
+    extern __shared__ __align__(16) uint32_t smem[];
     const uint32_t lane = threadIdx.x & 63;
+    WaveLds W(smem + (threadIdx.x >> 6) * wave_lds_words(cap), cap);
     bool ovf = false;
     Counts cnt;
     for (uint32_t guard = 0; guard < bt.total_chunks + 1; ++guard) {
         uint32_t c = 0;
         if (lane == 0)
             c = atomicAdd(bt.counter, 1u);
-        c = __shfl(c, 0, 64);
+        c = uniform(c);
         if (c >= bt.total_chunks)
             break;
         uint32_t lo = 0, hi = bt.n_sched; // last entry with cstart <= c
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
-            if (bt.cstart[mid] <= c)
+            if (uniform(bt.cstart[mid]) <= c)
                 lo = mid;
             else
                 hi = mid;
         }
-        const uint32_t m = bt.sched[lo];
+        const uint32_t m = uniform(bt.sched[lo]);
         const TreeView tv = bt.views[m];
-        const uint32_t q0 = bt.qoff[m] + (c - bt.cstart[lo]) * bt.qpw;
-        const uint32_t q1 = min(q0 + bt.qpw, bt.qoff[m + 1]);
+        const uint32_t q0 = uniform(bt.qoff[m]) + (c - uniform(bt.cstart[lo])) * bt.qpw;
+        const uint32_t q1 = min(q0 + bt.qpw, uniform(bt.qoff[m + 1]));
         for (uint32_t base = q0; base < q1; base += 64) {
             const uint32_t slot = base + lane;
             const bool valid = slot < q1;
-            if (KIND != 0 && !valid)
-                continue;
             const uint32_t qi = valid ? (bt.perm ? bt.perm[slot] : slot) : 0u;
-            const v3 p = valid ? load_point<3>(q, qi) : mk(0.0f, 0.0f, 0.0f);
-            float best = F_INF;
-            uint32_t bi = INVALID;
-            if (KIND == 0) {
-                WaveLds W(stk + (threadIdx.x / 64) * POOL_WORDS, 32 * SSZ);
-                if (valid)
-                    W.start(lane, p);
+            if (valid)
+                W.start(lane, load_point<3>(q, qi));
+            if (KIND == 0)
                 cp_wave<false, 3>(tv, min(64u, q1 - base), W, cnt, ovf);
-                if (!valid)
-                    continue;
+            else
+                sil_wave<false, 3, KIND - 1>(tv, __ballot(valid), flip != 0, KIND == 2 && valid ? seed[qi] : F_INF, W,
+                                             cnt, ovf);
+            if (valid) {
+                float best;
+                uint32_t bi;
                 unpack_best(W.best[lane], best, bi);
-                best = dm::sqrt_(best);
-            } else {
-                float cap = SEEDED ? seed[qi] : F_INF;
-                if (!(cap >= 0.0f))
-                    cap = F_INF;
-                sil_query<BS, SSZ, false, 3, SEEDED, true>(tv, p, flip != 0, cap, stk + threadIdx.x,
-                                                           &elds[KIND == 0 ? 0 : threadIdx.x / 64], best, bi, cnt,
-                                                           ovf);
+                if (out_idx)
+                    out_idx[qi] = bi;
+                out_dist[qi] = KIND == 0 ? dm::sqrt_(best) : best;
             }
-            if (out_idx)
-                out_idx[qi] = bi;
-            out_dist[qi] = best;
         }
     }
     if (ovf && err)
@@ -132,48 +119,6 @@ __global__ __launch_bounds__(256) void k_query_mesh(const uint32_t* __restrict__
 }
 
 } // namespace
-
-template <int BS, int SSZ, int KIND, bool SEEDED>
-static hipError_t launch_batch_cfg(const BatchTable& bt, const float* q, int flip, const float* seed,
-                                   uint32_t* out_idx, float* out_dist, uint32_t n_cu, hipStream_t st)
-{
-    int per_cu = 0;
-    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_batch<BS, SSZ, KIND, SEEDED>, BS, 0);
-    if (e != hipSuccess)
-        return e;
-    const uint32_t waves = n_cu * (uint32_t)std::max(per_cu, 1) * (BS / 64);
-    // no more waves than chunks
-    const uint32_t grid = std::max(1u, std::min(n_cu * (uint32_t)std::max(per_cu, 1),
-                                                (std::min(waves, bt.total_chunks) + BS / 64 - 1) / (BS / 64)));
-    hipLaunchKernelGGL((k_batch<BS, SSZ, KIND, SEEDED>), dim3(grid), dim3(BS), 0, st, bt, q, flip, seed, out_idx,
-                       out_dist, traversal_error_word());
-    return hipGetLastError();
-}
-
-template <int BS, int KIND, bool SEEDED>
-static hipError_t launch_batch_bs(const BatchTable& bt, uint32_t ssz, const float* q, int flip, const float* seed,
-                                  uint32_t* out_idx, float* out_dist, uint32_t n_cu, hipStream_t st)
-{
-    switch (ssz) {
-    case 8: return launch_batch_cfg<BS, 8, KIND, SEEDED>(bt, q, flip, seed, out_idx, out_dist, n_cu, st);
-    case 24: return launch_batch_cfg<BS, 24, KIND, SEEDED>(bt, q, flip, seed, out_idx, out_dist, n_cu, st);
-    case 32: return launch_batch_cfg<BS, 32, KIND, SEEDED>(bt, q, flip, seed, out_idx, out_dist, n_cu, st);
-    default: return launch_batch_cfg<BS, 16, KIND, SEEDED>(bt, q, flip, seed, out_idx, out_dist, n_cu, st);
-    }
-}
-
-template <int KIND, bool SEEDED>
-static hipError_t launch_batch_kind(const BatchTable& bt, uint32_t bs, uint32_t ssz, const float* q, int flip,
-                                    const float* seed, uint32_t* out_idx, float* out_dist, uint32_t n_cu,
-                                    hipStream_t st)
-{
-    switch (bs) {
-    case 64: return launch_batch_bs<64, KIND, SEEDED>(bt, ssz, q, flip, seed, out_idx, out_dist, n_cu, st);
-    case 128: return launch_batch_bs<128, KIND, SEEDED>(bt, ssz, q, flip, seed, out_idx, out_dist, n_cu, st);
-    case 512: return launch_batch_bs<512, KIND, SEEDED>(bt, ssz, q, flip, seed, out_idx, out_dist, n_cu, st);
-    default: return launch_batch_bs<256, KIND, SEEDED>(bt, ssz, q, flip, seed, out_idx, out_dist, n_cu, st);
-    }
-}
 
 hipError_t launch_batch(const snch_scene* s, int kind, const float* q, const uint32_t* q_off_host, int flip,
                         uint32_t* out_idx, float* out_dist, const BatchConfig& cfg, hipStream_t st,
@@ -251,15 +196,21 @@ hipError_t launch_batch(const snch_scene* s, int kind, const float* q, const uin
         bt.perm = in_alt ? w.idx_alt.as<uint32_t>() : w.idx.as<uint32_t>();
     }
     hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(1), 0, st, bt.counter);
-    const uint32_t n_cu = s->ctx && s->ctx->n_cu > 0 ? (uint32_t)s->ctx->n_cu : 256u;
+    // as many waves as are resident, and no more than chunks
+    const uint32_t wpb = cfg.block_size / 64, cap = pool_cap(cfg.stack_depth);
+    const size_t lds = sizeof(uint32_t) * wpb * wave_lds_words(cap);
+    const uint32_t per_cu = std::max(1u, std::min((uint32_t)(LDS_PER_CU / lds), 24u / wpb));
+    const dim3 g(std::max(1u, std::min(s->n_cu() * per_cu, nblocks(total, wpb)))), blk(cfg.block_size);
+#define SNCH_BATCH(K_)                                                                                               \
+    hipLaunchKernelGGL((k_batch<K_>), g, blk, lds, st, bt, cap, q, flip, seed, out_idx, out_dist, traversal_error_word())
     if (kind == 0)
-        return launch_batch_kind<0, false>(bt, cfg.block_size, cfg.stack_depth, q, flip, nullptr, out_idx, out_dist,
-                                           n_cu, st);
-    if (seed)
-        return launch_batch_kind<1, true>(bt, cfg.block_size, cfg.stack_depth, q, flip, seed, out_idx, out_dist, n_cu,
-                                          st);
-    return launch_batch_kind<1, false>(bt, cfg.block_size, cfg.stack_depth, q, flip, nullptr, out_idx, out_dist, n_cu,
-                                       st);
+        SNCH_BATCH(0);
+    else if (seed)
+        SNCH_BATCH(2);
+    else
+        SNCH_BATCH(1);
+#undef SNCH_BATCH
+    return hipGetLastError();
 }
 
 } // namespace snch

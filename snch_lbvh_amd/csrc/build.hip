@@ -915,21 +915,23 @@ __device__ __forceinline__ void refit_write(const MeshIds& id, uint32_t p, uint2
     tnode[4 * r + 2] = make_float4(rb.lo.x, rb.lo.y, rb.lo.z, rb.hi.x);
     tnode[4 * r + 3] = make_float4(rb.hi.y, rb.hi.z, __uint_as_float(child_ref(id, ch.y, range, leaf_size)), 0.0f);
     tcone[4 * r + 0] = make_float4(lc.axis.x, lc.axis.y, lc.axis.z, lc.half_angle);
-    tcone[4 * r + 1] = make_float4(rc.axis.x, rc.axis.y, rc.axis.z, rc.half_angle);
-    tcone[4 * r + 2] = make_float4(lc.radius, rc.radius, 0.0f, 0.0f);
-    // tcone[4 r + 3] (sin, cos of the half angles) is filled by tcone_trig
-    // once the merges are done: off the chain of dependent merges
+    tcone[4 * r + 2] = make_float4(rc.axis.x, rc.axis.y, rc.axis.z, rc.half_angle);
+    // the sines and cosines (the halves before these) are filled by
+    // tcone_trig once the merges are done: off the chain of dependent merges
+    reinterpret_cast<float2*>(tcone)[8 * r + 3] = make_float2(lc.radius, 0.0f);
+    reinterpret_cast<float2*>(tcone)[8 * r + 7] = make_float2(rc.radius, 0.0f);
 }
 
 // sin and cos of both children's half angles of internal record r, read
-// back from the record's first two entries
+// back from the record
 __device__ __forceinline__ void tcone_trig(float4* __restrict__ tcone, uint32_t r)
 {
-    const float hl = tcone[4 * r + 0].w, hr = tcone[4 * r + 1].w;
+    const float hl = tcone[4 * r + 0].w, hr = tcone[4 * r + 2].w;
     float ls, lcs, rs, rcs;
     dm::sincosf_(hl, &ls, &lcs);
     dm::sincosf_(hr, &rs, &rcs);
-    tcone[4 * r + 3] = make_float4(ls, lcs, rs, rcs);
+    reinterpret_cast<float2*>(tcone)[8 * r + 2] = make_float2(ls, lcs);
+    reinterpret_cast<float2*>(tcone)[8 * r + 6] = make_float2(rs, rcs);
 }
 
 // box + cone of live nodes in LDS, structure of arrays over RT slots.  A node

@@ -646,15 +646,13 @@ int snch_closest_point_ex(const snch_scene* s, const float* q, uint32_t n, uint3
     SNCH_CHECK_ARG(depth == 8 || depth == 16, "snch_closest_point: stack_depth must be 8 or 16");
     const uint32_t* perm = opts ? opts->order : nullptr;
     const bool own_order = !perm && want_order(opts, n);
-    if (own_order) {
-        SNCH_HIP(scratch_begin(s, st), "snch_closest_point: stream wait");
-        SNCH_HIP(query_order(s->view(), (int)s->dim, q, n, s->qscratch, st, &perm), "snch_closest_point: ordering");
-    }
-    SNCH_HIP(launch_closest_point(s->view(), (int)s->dim, q, n, out_idx, out_dist, block, depth, perm,
-                                  opts ? opts->stats : nullptr, s->n_cu(), st),
-             "snch_closest_point");
+    SNCH_HIP(scratch_begin(s, st), "snch_closest_point: stream wait");
     if (own_order)
-        SNCH_HIP(scratch_end(s, st), "snch_closest_point: event");
+        SNCH_HIP(query_order(s->view(), (int)s->dim, q, n, s->qscratch, st, &perm), "snch_closest_point: ordering");
+    SNCH_HIP(launch_closest_point(s->view(), (int)s->dim, q, n, out_idx, out_dist, block, depth, perm,
+                                  opts ? opts->stats : nullptr, nullptr, s->n_cu(), st),
+             "snch_closest_point");
+    SNCH_HIP(scratch_end(s, st), "snch_closest_point: event");
     return SNCH_OK;
 }
 
@@ -679,38 +677,16 @@ int snch_closest_silhouette_ex(const snch_scene* s, const float* q, uint32_t n, 
     const uint32_t* perm = opts ? opts->order : nullptr;
     const bool own_order = !perm && want_order(opts, n);
     const bool capped = opts && opts->seed_is_cap;
-    // a seed radius, not a hard cap: unsettled queries are re-queued for whole
-    // waves unless asked to search again in place (default launch shape only)
-    const bool requeue = seed && !capped && n > 0 && !(opts && opts->seed_retry == 1) && block == 64 && depth == 16;
-    // no seed or a hard cap: a persistent launch taking 64-query chunks (default launch shape)
-    const bool persist = (!seed || capped) && n > 0 && block == 64 && depth == 16;
-    if (own_order || requeue || persist)
-        SNCH_HIP(scratch_begin(s, st), "snch_closest_silhouette: stream wait");
+    SNCH_HIP(scratch_begin(s, st), "snch_closest_silhouette: stream wait");
     if (own_order)
         SNCH_HIP(query_order(s->view(), (int)s->dim, q, n, s->qscratch, st, &perm),
                  "snch_closest_silhouette: ordering");
-    if (persist) {
-        SNCH_HIP(s->rq_ctr.ensure(sizeof(uint32_t) * 32), "snch_closest_silhouette: allocation");
-        const uint32_t n_cu = s->ctx && s->ctx->n_cu > 0 ? (uint32_t)s->ctx->n_cu : 256u;
-        SNCH_HIP(launch_closest_silhouette_persist(s->view(), (int)s->dim, q, n, flip, seed, out_sil, out_dist,
-                                                   perm, opts ? opts->stats : nullptr, s->rq_ctr.as<uint32_t>(), n_cu,
-                                                   st),
-                 "snch_closest_silhouette");
-    } else if (requeue) {
-        SNCH_HIP(s->rq_ctr.ensure(sizeof(uint32_t) * 32), "snch_closest_silhouette: allocation");
-        SNCH_HIP(s->rq_queue.ensure(sizeof(uint32_t) * 8 * (size_t)n), "snch_closest_silhouette: allocation");
-        const uint32_t n_cu = s->ctx && s->ctx->n_cu > 0 ? (uint32_t)s->ctx->n_cu : 256u;
-        SNCH_HIP(launch_closest_silhouette_requeue(s->view(), (int)s->dim, q, n, flip, seed, out_sil, out_dist, perm,
-                                                   opts ? opts->stats : nullptr, s->rq_ctr.as<uint32_t>(),
-                                                   s->rq_queue.as<uint32_t>(), n_cu, st),
-                 "snch_closest_silhouette");
-    } else {
-        SNCH_HIP(launch_closest_silhouette(s->view(), (int)s->dim, q, n, flip, seed, capped, out_sil, out_dist,
-                                           block, depth, perm, opts ? opts->stats : nullptr, st),
-                 "snch_closest_silhouette");
-    }
-    if (own_order || requeue || persist)
-        SNCH_HIP(scratch_end(s, st), "snch_closest_silhouette: event");
+    SNCH_HIP(s->chunk_ctr.ensure(sizeof(uint32_t) * 32), "snch_closest_silhouette: allocation");
+    SNCH_HIP(launch_closest_silhouette(s->view(), (int)s->dim, q, n, flip, seed, capped, out_sil, out_dist, block,
+                                       depth, perm, opts ? opts->stats : nullptr, s->chunk_ctr.as<uint32_t>(),
+                                       s->n_cu(), st),
+             "snch_closest_silhouette");
+    SNCH_HIP(scratch_end(s, st), "snch_closest_silhouette: event");
     return SNCH_OK;
 }
 
@@ -1088,9 +1064,9 @@ int snch_scene_export_mesh(const snch_scene* s, uint32_t mesh, uint32_t* nodes, 
             const uint32_t node[2] = {((ref[0] & LEAF_BIT) ? N - 1 : 0) + (ref[0] & REF_MASK),
                                       ((ref[1] & LEAF_BIT) ? N - 1 : 0) + (ref[1] & REF_MASK)};
             if (node[0] < NN)
-                put(node[0], llo, lhi, c + 0, c[3], c[8]);
+                put(node[0], llo, lhi, c + 0, c[3], c[6]);
             if (node[1] < NN)
-                put(node[1], rlo, rhi, c + 4, c[7], c[9]);
+                put(node[1], rlo, rhi, c + 8, c[11], c[14]);
         }
     }
     return SNCH_OK;

@@ -79,7 +79,7 @@ struct snch_scene {
     snch::DeviceBuffer tnode, tcone, tleaf, tedge, nbox, ncone;
     snch::BuildScratch scratch;
     mutable snch::QueryScratch qscratch; // used by const query entry points
-    mutable snch::DeviceBuffer rq_ctr, rq_queue; // re-queued seeded search (counters, queue)
+    mutable snch::DeviceBuffer chunk_ctr; // chunk counters of a persistent silhouette launch
     mutable snch::BatchState batch;
     bool built = false;
     bool sorted_in_alt = false; // sorted codes/indices live in scratch.codes_alt/idx_alt
@@ -141,33 +141,22 @@ hipError_t query_order(const TreeView& t, int dim, const float* q, uint32_t n, Q
 size_t query_order_scratch_bytes(uint32_t n);
 hipError_t query_order_in(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* words, hipStream_t st,
                           const uint32_t** perm, uint32_t* err);
+// ctr (nullable; 8 words, rewritten at launch by a kernel: graph capture is
+// fine): lets a large launch be persistent, and is needed where the number of
+// queries is on the device (t.n_dev)
 hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* idx, float* dist,
-                                uint32_t block, uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t n_cu,
-                                hipStream_t st);
+                                uint32_t block, uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t* ctr,
+                                uint32_t n_cu, hipStream_t st);
 // seed (nullable): per-query radius.  capped: a hard radius (answers beyond
 // it are not searched; the returned distance is then larger than the
 // radius, possibly +inf).  Otherwise a hint: queries not settled within it
 // continue without it; results equal the unseeded search.
-// err (nullable): the sticky overflow word to report to (default: the current
-// device's, traversal_error_word())
+// ctr: as above.  err (nullable): the sticky overflow word to report to
+// (default: the current device's, traversal_error_word())
 hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q, uint32_t n, int flip,
                                      const float* seed, bool capped, uint32_t* sil, float* dist, uint32_t block,
-                                     uint32_t depth, const uint32_t* perm, uint64_t* stats, hipStream_t st,
-                                     uint32_t* err = nullptr);
-// seeded search with unsettled queries re-queued for whole waves (ctr: 24
-// words, queue: 8 n words; both rewritten at launch)
-hipError_t launch_closest_silhouette_requeue(const TreeView& t, int dim, const float* q, uint32_t n, int flip,
-                                             const float* seed, uint32_t* sil, float* dist, const uint32_t* perm,
-                                             uint64_t* stats, uint32_t* ctr, uint32_t* queue, uint32_t n_cu,
-                                             hipStream_t st, uint32_t* err = nullptr);
-// the search on a persistent launch taking 64-query chunks: plain (seed
-// null) or within the radius seed[qi] only (a hard cap); over the first
-// min(n, *t.n_dev) queries when the count is on the device (capped only).
-// ctr: 24 words, rewritten at launch (by a kernel: graph capture is fine)
-hipError_t launch_closest_silhouette_persist(const TreeView& t, int dim, const float* q, uint32_t n, int flip,
-                                             const float* seed, uint32_t* sil, float* dist, const uint32_t* perm,
-                                             uint64_t* stats, uint32_t* ctr, uint32_t n_cu, hipStream_t st,
-                                             uint32_t* err = nullptr);
+                                     uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t* ctr,
+                                     uint32_t n_cu, hipStream_t st, uint32_t* err = nullptr);
 hipError_t launch_ray(const TreeView& t, int dim, const float* o, const float* d, const float* tmax, uint32_t n,
                       int any_hit, uint8_t* hit, float* tout, float* uv, uint32_t* idx, uint64_t* stats,
                       hipStream_t st);

@@ -101,7 +101,7 @@ extern "C" int snch_closest_silhouette_noalloc(const snch_scene* s, const float*
         e = query_order_in(t, (int)s->dim, q, n, c->noalloc_scratch, st, &perm, c->err_word + 1);
     if (e == hipSuccess)
         e = launch_closest_silhouette(t, (int)s->dim, q, n, flip, seed, false, out_sil, out_dist, 64, 16, perm,
-                                      nullptr, st, c->err_word);
+                                      nullptr, nullptr, s->n_cu(), st, c->err_word);
     if (e != hipSuccess)
         return hip_fail(e, "snch_closest_silhouette_noalloc");
     return SNCH_OK;

@@ -37,40 +37,37 @@ namespace {
 constexpr int OVF = 64; // private overflow entries per lane (generic queries)
 
 // ------------------------------------------------------------ closest point
-// One wave per chunk of qpw queries.  qpw = 64: consecutive queries of the
-// visiting order.  qpw < 64 (a launch that 64 per wave would leave too few
-// waves for): every n_waves-th query, so that costly neighbours (the centre
-// of a sphere) land in different waves.
 template <bool STATS, int DIM>
 __global__ __launch_bounds__(512, 6) void k_closest_point(TreeView t, const float* __restrict__ q, uint32_t n,
                                                           uint32_t qpw, uint32_t cap, uint32_t* __restrict__ out_idx,
                                                           float* __restrict__ out_dist,
-                                                          const uint32_t* __restrict__ perm,
+                                                          const uint32_t* __restrict__ perm, uint32_t* ctr,
                                                           uint32_t* __restrict__ err, unsigned long long* stats)
 {
     extern __shared__ __align__(16) uint32_t smem[];
-    const uint32_t lane = threadIdx.x & 63, wpb = blockDim.x >> 6, w = threadIdx.x >> 6;
-    WaveLds W(smem + w * (2 * cap + WaveLds::FIXED), cap);
+    const uint32_t lane = threadIdx.x & 63;
+    WaveLds W(smem + (threadIdx.x >> 6) * wave_lds_words(cap), cap);
     if (t.n_dev)
         n = min(n, *t.n_dev);
-    const uint32_t chunk = uniform(xcd_remap(blockIdx.x, gridDim.x) * wpb + w), n_waves = gridDim.x * wpb;
-    const uint32_t slot = qpw < 64u ? lane * n_waves + chunk : chunk * 64u + lane;
-    const bool valid = lane < qpw && slot < n;
-    const uint32_t qi = valid ? (perm ? min(perm[slot], n - 1) : slot) : 0u;
-    if (valid)
-        W.start(lane, load_point<DIM>(q, qi));
+    if (qpw == 0u)
+        qpw = queries_per_wave(n, gridDim.x * (blockDim.x >> 6));
     bool ovf = false;
     Counts cnt;
-    cp_wave<STATS, DIM>(t, (uint32_t)__popcll(__ballot(valid)), W, cnt, ovf);
+    for_chunks(n, qpw, ctr, [&](uint32_t slot, bool valid) {
+        const uint32_t qi = valid ? (perm ? min(perm[slot], n - 1) : slot) : 0u;
+        if (valid)
+            W.start(lane, load_point<DIM>(q, qi));
+        cp_wave<STATS, DIM>(t, (uint32_t)__popcll(__ballot(valid)), W, cnt, ovf);
+        if (valid) {
+            float best;
+            uint32_t best_idx;
+            unpack_best(W.best[lane], best, best_idx);
+            out_idx[qi] = best_idx;
+            out_dist[qi] = dm::sqrt_(best);
+        }
+    });
     if (ovf && err)
         atomicOr(err, 1u);
-    if (valid) {
-        float best;
-        uint32_t best_idx;
-        unpack_best(W.best[lane], best, best_idx);
-        out_idx[qi] = best_idx;
-        out_dist[qi] = dm::sqrt_(best);
-    }
     if (STATS)
         flush_counts(cnt, stats);
 }
@@ -490,31 +487,30 @@ hipError_t query_order_in(const TreeView& t, int dim, const float* q, uint32_t n
     return hipGetLastError();
 }
 
-// queries per wave of a launch of n: 64, or fewer when that leaves resident
-// waves without work
-static uint32_t queries_per_wave(uint32_t n, uint32_t resident_waves)
+__global__ void k_clear_chunks(uint32_t* __restrict__ ctr)
 {
-    return std::min(64u, std::max(1u, nblocks(n, std::max(resident_waves, 1u))));
+    if (threadIdx.x < CHUNK_CTR_WORDS)
+        ctr[threadIdx.x] = 0u;
 }
 
 hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* idx, float* dist,
-                                uint32_t block, uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t n_cu,
-                                hipStream_t st)
+                                uint32_t block, uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t* ctr,
+                                uint32_t n_cu, hipStream_t st)
 {
     if (n == 0)
         return hipSuccess;
     auto* sp = reinterpret_cast<unsigned long long*>(stats);
-    const uint32_t wpb = block / 64, cap = 32 * depth;
-    const size_t lds = sizeof(uint32_t) * wpb * wave_lds_words(depth);
-    const uint32_t qpw = t.n_dev ? 64u : queries_per_wave(n, n_cu * (uint32_t)(LDS_PER_CU / lds) * wpb);
-    const dim3 g(nblocks(nblocks(n, qpw), wpb)), b(block);
+    const SearchGrid g = search_grid(n, block, depth, false, n_cu, 6, ctr != nullptr, t.n_dev != nullptr);
+    uint32_t* c = g.persist ? ctr : nullptr;
+    if (c)
+        hipLaunchKernelGGL(k_clear_chunks, dim3(1), dim3(64), 0, st, c);
     SNCH_DISPATCH_DIM(dim, {
         if (stats)
-            hipLaunchKernelGGL((k_closest_point<true, DIM>), g, b, lds, st, t, q, n, qpw, cap, idx, dist, perm,
-                               traversal_error_word(), sp);
+            hipLaunchKernelGGL((k_closest_point<true, DIM>), g.grid, g.block, g.lds, st, t, q, n, g.qpw,
+                               pool_cap(depth), idx, dist, perm, c, traversal_error_word(), sp);
         else
-            hipLaunchKernelGGL((k_closest_point<false, DIM>), g, b, lds, st, t, q, n, qpw, cap, idx, dist, perm,
-                               traversal_error_word(), sp);
+            hipLaunchKernelGGL((k_closest_point<false, DIM>), g.grid, g.block, g.lds, st, t, q, n, g.qpw,
+                               pool_cap(depth), idx, dist, perm, c, traversal_error_word(), sp);
     });
     return hipGetLastError();
 }

@@ -47,6 +47,17 @@ __device__ __forceinline__ ChildRec load_child(const float4* __restrict__ tnode,
     return c;
 }
 
+// one child's cone, and the sine and cosine of its half angle
+struct ConeRec {
+    v3 axis;
+    float half_angle, sin_ha, cos_ha, radius;
+};
+__device__ __forceinline__ ConeRec load_cone(const float4* __restrict__ tcone, uint32_t i, uint32_t side)
+{
+    const float4 a = tcone[4 * i + 2 * side], b = tcone[4 * i + 2 * side + 1];
+    return ConeRec{mk(a.x, a.y, a.z), a.w, b.x, b.y, b.z};
+}
+
 // a child the traversal treats as a leaf: a true leaf, or a run of sorted
 // leaves [first, first + count) under an internal node (leaf size > 1).  An
 // internal left child (side 0) is numbered by its last leaf, a right one by
@@ -151,6 +162,17 @@ __device__ __forceinline__ bool overlap_dim(const float4& C, float radius, v3 p,
 {
     return DIM == 3 ? cone_overlap(mk(C.x, C.y, C.z), C.w, radius, p, b, md)
                     : cone_overlap2d(mk(C.x, C.y, 0.0f), C.w, radius, p, b, md);
+}
+
+// the cone test of a child whose box lies at squared distance md (query.cuh:366-367)
+template <int DIM>
+__device__ __forceinline__ bool cone_hit(const TreeView& t, const ConeRec& c, v3 p, const box3& b, float md)
+{
+    if (!cone_valid(c.half_angle))
+        return false;
+    if (DIM == 3 && (t.flags & TREE_FAST_CONE))
+        return cone_overlap_fast(c.axis, c.half_angle, c.sin_ha, c.cos_ha, c.radius, p, b, md);
+    return overlap_dim<DIM>(make_float4(c.axis.x, c.axis.y, c.axis.z, c.half_angle), c.radius, p, b, md);
 }
 
 // SampleTriangleInSphere for one sphere (sample.cuh:23-92): the reference's
@@ -301,20 +323,8 @@ __device__ inline void dev_nearest_silhouette(const TreeView& t, v3 p, bool flip
         const NodeRec nr = load_node(t.tnode, node);
         const float Lmd = box_mindist(nr.L, p), Rmd = box_mindist(nr.R, p);
         const float b2 = best * best;
-        bool hL = Lmd <= b2, hR = Rmd <= b2;
-        if (hL || hR) { // query.cuh:366-367
-            const float4 CL = t.tcone[4 * node], CR = t.tcone[4 * node + 1], Cr = t.tcone[4 * node + 2];
-            if (DIM == 3 && (t.flags & TREE_FAST_CONE)) {
-                const float4 SC = t.tcone[4 * node + 3];
-                hL = hL && cone_valid(CL.w) &&
-                     cone_overlap_fast(mk(CL.x, CL.y, CL.z), CL.w, SC.x, SC.y, Cr.x, p, nr.L, Lmd);
-                hR = hR && cone_valid(CR.w) &&
-                     cone_overlap_fast(mk(CR.x, CR.y, CR.z), CR.w, SC.z, SC.w, Cr.y, p, nr.R, Rmd);
-            } else {
-                hL = hL && cone_valid(CL.w) && overlap_dim<DIM>(CL, Cr.x, p, nr.L, Lmd);
-                hR = hR && cone_valid(CR.w) && overlap_dim<DIM>(CR, Cr.y, p, nr.R, Rmd);
-            }
-        }
+        const bool hL = Lmd <= b2 && cone_hit<DIM>(t, load_cone(t.tcone, node, 0u), p, nr.L, Lmd);
+        const bool hR = Rmd <= b2 && cone_hit<DIM>(t, load_cone(t.tcone, node, 1u), p, nr.R, Rmd);
         uint32_t lf, lc, rf, rc;
         const bool lLeaf = as_leaf(nr.lref, 0u, lf, lc), rLeaf = as_leaf(nr.rref, 1u, rf, rc);
         if (hL && lLeaf)

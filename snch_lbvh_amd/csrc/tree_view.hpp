@@ -22,10 +22,9 @@ namespace snch {
 //             at most k leaves, their count: the traversal queries then treat
 //             c as one leaf holding that run of sorted leaves (as_leaf).
 //   tcone[i]  4 x float4 = 64 B per internal node: the children's normal
-//             cones, read only by the silhouette query:
-//               [0] L.axis L.half_angle  [1] R.axis R.half_angle
-//               [2] L.radius R.radius 0 0
-//               [3] sin, cos of L.half_angle, sin, cos of R.half_angle
+//             cones, 32 B each, read only by the silhouette query:
+//               [0] L.axis L.half_angle  [1] sin, cos of L.half_angle, L.radius, 0
+//               [2] R.axis R.half_angle  [3] sin, cos of R.half_angle, R.radius, 0
 //   tleaf[j]  3 x float4 = 48 B per leaf, in Morton (sorted) order:
 //               [k] vertex k xyz, w = (original triangle, first owned edge,
 //               owned edge count) for k = 0, 1, 2

@@ -180,16 +180,16 @@ __device__ __forceinline__ void flush_counts(const Counts& c, unsigned long long
 // wave as slow as its slowest lane, a lane as slow as its chain of dependent
 // loads) every lane has work until the wave's last query ends, a node's two
 // children share one 64-B line per pair of lanes, and leaf code runs on full
-// waves.  Queries enter as the pool runs low: POOL_ADD at a time keeps few
-// queries, and so few pending nodes, in flight (all 64 at once fill the pool
-// and leave it popping one item at a time: 218 instead of 33 ms on the case
-// below, with one lane per item; 4 or 16 at a time 33.5 and 34.6).
+// waves.  Queries enter as the pool runs low, POOL_ADD at a time: with all 64
+// in flight at once the pool fills and pops one item at a time.
 //
-// Closest point, one lane per query with a stack -> pool: 2^22 queries on
-// 2^20 triangles 46 -> 26 ms (VALU issue 0.78 of the SIMD cycles, 582 nodes
-// per query), 65,536 on 20,480 triangles 2.1 -> 0.18 ms, 1,000 on 20,480
-// triangles 0.83 -> 0.03 ms (there a launch lasted as long as the longest
-// chain of dependent loads, about 2 us a node).
+// Measured, one lane per query with a stack -> pool.  Closest point: 2^22
+// queries on 2^20 triangles 46 -> 24 ms, 65,536 on 20,480 triangles 2.1 ->
+// 0.18 ms, 1,000 on 20,480 triangles 0.83 -> 0.03 ms (there a launch lasted as
+// long as the longest chain of dependent loads, about 2 us a node).  Closest
+// silhouette: 2^22 on 2^20 triangles 69 -> 36 ms (POOL_ADD 4: 43, 8: 41, 12:
+// 38, 16: 37, 24: 35), 10,007 on 90,000 triangles 4.3 -> 0.18 ms.  Pairs that
+// keep their near child in registers instead of the pool: 50 to 58 ms.
 //
 // The answer is that of the search one lane would make alone, near child
 // first, each node's leaves at once, which skips a box as soon as its lower
@@ -202,18 +202,24 @@ __device__ __forceinline__ void flush_counts(const Counts& c, unsigned long long
 // rounding, which leaves no such candidate out, and where a hidden leaf has
 // the smallest distance the lane repeats the search alone, from the widened
 // bound (a few dozen nodes).
-constexpr uint32_t POOL_ADD = 8;
-constexpr uint32_t LEAF_CAP = 128; // leaf buffer entries: below 64 before a step, which adds at most 64
+constexpr uint32_t POOL_ADD = 20;
+constexpr uint32_t LEAF_RUN = 40;            // leaves that are worth a step of the wave
+constexpr uint32_t LEAF_CAP = LEAF_RUN + 64; // buffer entries: below LEAF_RUN before a step, which adds at most 64
 
-// smaller is better: the distance, ties to the smaller id (distances are not negative)
-__device__ __forceinline__ unsigned long long pack_best(float d, uint32_t id)
+// smaller is better: the distance, then hidden candidates (so that an answer
+// tells whether any attains it), then the smaller id (distances are not
+// negative, ids are below 2^31)
+__device__ __forceinline__ unsigned long long pack_best(float d, uint32_t id, bool hidden = false)
 {
-    return ((unsigned long long)__float_as_uint(d) << 32) | id;
+    return ((unsigned long long)__float_as_uint(d) << 32) | (hidden ? id : id | 0x80000000u);
 }
-__device__ __forceinline__ void unpack_best(unsigned long long v, float& d, uint32_t& id)
+// returns whether the answer is hidden
+__device__ __forceinline__ bool unpack_best(unsigned long long v, float& d, uint32_t& id)
 {
+    const uint32_t w = (uint32_t)v;
     d = __uint_as_float((uint32_t)(v >> 32));
-    id = (uint32_t)v;
+    id = w == INVALID ? INVALID : w & 0x7FFFFFFFu;
+    return (w & 0x80000000u) == 0u;
 }
 // lanes of mask below this one
 __device__ __forceinline__ uint32_t rank_in(uint64_t mask)
@@ -226,26 +232,30 @@ __device__ __forceinline__ float pair_other(float v)
     return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), 0xB1, 0xF, 0xF, true));
 }
 
-// LDS of one wave, carved from the block's dynamic LDS: cap pool items (2
-// words each: slot << 24 | node, key), the leaf buffer (2 words per entry:
-// slot << 24 | leaf, key), and per query slot its answer, point, widened
-// (squared) bound and the smallest distance of a hidden leaf
+// LDS of one wave, carved from the block's dynamic LDS: cap pool items (slot
+// << 24 | node, and the upper half of the float bits of the bound it was
+// pushed with: a lower bound of it), the leaf buffer (2 words per entry: slot
+// << 24 | leaf, bound), and per query slot its answer, point and widened
+// (squared) pruning bound
 struct WaveLds {
     unsigned long long* best;
-    uint32_t *pool, *leaf, *bound, *hidden;
+    uint32_t *pool, *leaf, *bound;
+    uint16_t* pkey;
     float* q; // x, y, z rows of 64
     uint32_t cap;
-    static constexpr uint32_t FIXED = 128 + 2 * LEAF_CAP + 128 + 192; // words besides the pool
+    static constexpr uint32_t FIXED = 128 + 2 * LEAF_CAP + 64 + 192; // words besides the pool (and hard caps)
     __device__ __forceinline__ WaveLds(uint32_t* base, uint32_t cap_)
     {
         best = reinterpret_cast<unsigned long long*>(base);
-        pool = base + 128;
-        leaf = pool + 2 * cap_;
+        leaf = base + 128;
         bound = leaf + 2 * LEAF_CAP;
-        hidden = bound + 64;
-        q = reinterpret_cast<float*>(hidden + 64);
+        q = reinterpret_cast<float*>(bound + 64);
+        pool = base + FIXED;
+        pkey = reinterpret_cast<uint16_t*>(pool + cap_);
         cap = cap_;
     }
+    // squared hard caps, after the pool (hard-capped searches only)
+    __device__ __forceinline__ float* cap2() const { return reinterpret_cast<float*>(pool + cap + cap / 2); }
     __device__ __forceinline__ v3 point(uint32_t s) const { return mk(q[s], q[64 + s], q[128 + s]); }
     __device__ __forceinline__ void start(uint32_t s, v3 p)
     {
@@ -253,7 +263,7 @@ struct WaveLds {
         q[64 + s] = p.y;
         q[128 + s] = p.z;
         best[s] = pack_best(F_INF, INVALID);
-        bound[s] = hidden[s] = __float_as_uint(F_INF);
+        bound[s] = __float_as_uint(F_INF);
     }
 };
 // a distance widened by more than the rounding of any distance to the scene
@@ -273,8 +283,18 @@ __device__ __forceinline__ float scene_scale(const TreeView& t)
     return fmx(fmx(fmx(dm::fabs_(b.lo.x), dm::fabs_(b.hi.x)), fmx(dm::fabs_(b.lo.y), dm::fabs_(b.hi.y))),
                fmx(dm::fabs_(b.lo.z), dm::fabs_(b.hi.z)));
 }
-// words of dynamic LDS of a wave with `depth` pool items per lane pair
-inline uint32_t wave_lds_words(uint32_t depth) { return 2 * 32 * depth + WaveLds::FIXED; }
+// pool items of a wave for a stack depth option: 640 for the default of 16
+// (6.2 KB of LDS per wave: 26 waves on a CU, above the 6 per SIMD that 80 VGPRs
+// allow).  A fuller pool pops
+// fewer items at a time (pool_take): closest silhouette on the torus below,
+// with 8-byte items, 62 ms with 480, 53 with 512, 42 with 640 (5 waves per
+// SIMD), 45 with 800 (4 waves).
+constexpr uint32_t pool_cap(uint32_t depth) { return 40 * depth; }
+// words of dynamic LDS of a wave
+constexpr uint32_t wave_lds_words(uint32_t cap, bool capped = false)
+{
+    return cap + cap / 2 + WaveLds::FIXED + (capped ? 64u : 0u);
+}
 
 // append (a, key) of the lanes with `yes` to a list of two-word entries (the
 // callers' sizes never exceed the list: pool_take, LEAF_CAP)
@@ -287,6 +307,28 @@ __device__ __forceinline__ void list_push(uint32_t* list, uint32_t& size, bool y
         list[2 * at + 1] = __float_as_uint(key);
     }
     size += (uint32_t)__popcll(m);
+}
+
+// the same for pool items
+__device__ __forceinline__ void pool_push(WaveLds& W, uint32_t& size, bool yes, uint32_t a, float key)
+{
+    const uint64_t m = __builtin_amdgcn_ballot_w64(yes);
+    const uint32_t at = size + rank_in(m);
+    if (yes) {
+        W.pool[at] = a;
+        W.pkey[at] = (uint16_t)(__float_as_uint(key) >> 16);
+    }
+    size += (uint32_t)__popcll(m);
+}
+
+// queries waiting to enter (todo: a slot per bit) into the pool, up to
+// POOL_ADD of them
+__device__ __forceinline__ void pool_feed(WaveLds& W, uint32_t& size, uint64_t& todo)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    const bool in = ((todo >> lane) & 1ull) && rank_in(todo) < POOL_ADD;
+    todo &= ~__builtin_amdgcn_ballot_w64(in);
+    pool_push(W, size, in, lane << 24, 0.0f);
 }
 
 // how many items to pop so that their children fit: 32, fewer near the
@@ -363,10 +405,8 @@ __device__ __forceinline__ uint32_t cp_leaves(const TreeView& t, WaveLds& W, uin
             uint32_t id = INVALID;
             cp_leaf<DIM>(t, w & REF_MASK, p, d, id);
             if (id != INVALID && d <= b) {
-                atomicMin(&W.best[slot], pack_best(d, id));
+                atomicMin(&W.best[slot], pack_best(d, id, key > d));
                 atomicMin(&W.bound[slot], __float_as_uint(widened<DIM>(HwMath::sqrt(d), p, scale)));
-                if (key > d)
-                    atomicMin(&W.hidden[slot], __float_as_uint(d));
             }
         }
     }
@@ -393,27 +433,24 @@ __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds&
         return;
     }
     const float scale = scene_scale(t);
-    uint32_t size = 0, nleaf = 0, next = 0;
+    uint32_t size = 0, nleaf = 0;
+    uint64_t todo = __builtin_amdgcn_ballot_w64(lane < nq);
     // every iteration pops a node of some query (each at most once) or
     // evaluates leaves; the bound only guards against a malformed tree
     const uint32_t cap_iters = 128u * t.n_leaves + 65536u;
     for (uint32_t it = 0;; ++it) {
-        const bool fed = next >= nq;
-        if (nleaf >= 64u || (nleaf > 0u && fed && size < 32u)) {
+        if (nleaf >= LEAF_RUN || (nleaf > 0u && todo == 0ull && size < 32u)) {
             nleaf = cp_leaves<STATS, DIM>(t, W, nleaf, scale, cnt);
             continue;
         }
-        if (size == 0u && fed)
+        if (size == 0u && todo == 0ull)
             break;
         if (it >= cap_iters) {
             overflow = true;
             break;
         }
-        if (size < 32u && !fed) {
-            const uint32_t add = min(POOL_ADD, nq - next);
-            list_push(W.pool, size, lane < add, (next + lane) << 24, 0.0f);
-            next += add;
-        }
+        if (size < 32u && todo != 0ull)
+            pool_feed(W, size, todo);
         const uint32_t k = pool_take(size, W.cap), side = lane & 1u;
         size -= k;
         uint32_t slot = 0, ref = 0;
@@ -421,10 +458,10 @@ __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds&
         bool live = false;
         v3 p = mk(0.0f, 0.0f, 0.0f);
         if ((lane >> 1) < k) {
-            const uint32_t at = size + (lane >> 1), w = W.pool[2 * at], node = w & REF_MASK;
+            const uint32_t at = size + (lane >> 1), w = W.pool[at], node = w & REF_MASK;
             slot = w >> 24;
             b = __uint_as_float(W.bound[slot]);
-            live = __uint_as_float(W.pool[2 * at + 1]) <= b && node < t.n_leaves - 1;
+            live = __uint_as_float((uint32_t)W.pkey[at] << 16) <= b && node < t.n_leaves - 1;
             if (live) {
                 p = W.point(slot);
                 const ChildRec c = load_child(t.tnode, node, side);
@@ -450,27 +487,23 @@ __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds&
         const bool go = live && md <= mo && md <= b, leaf = as_leaf(ref, side, first, count);
         const float other = pair_other(md);
         const bool lt = md < other, eq = md == other, near = lt || (eq && !side);
-        list_push(W.pool, size, go && !leaf && !near, (slot << 24) | (ref & REF_MASK), md);
-        list_push(W.pool, size, go && !leaf && near, (slot << 24) | (ref & REF_MASK), md);
+        pool_push(W, size, go && !leaf && !near, (slot << 24) | (ref & REF_MASK), md);
+        pool_push(W, size, go && !leaf && near, (slot << 24) | (ref & REF_MASK), md);
         list_push(W.leaf, nleaf, go && leaf, (slot << 24) | first, md);
         for (uint32_t j = 1; (t.flags & TREE_RUNS) && __ballot(go && leaf && j < count); ++j) {
-            if (nleaf >= 64u)
+            if (nleaf >= LEAF_RUN)
                 nleaf = cp_leaves<STATS, DIM>(t, W, nleaf, scale, cnt);
             list_push(W.leaf, nleaf, go && leaf && j < count, (slot << 24) | (first + j), md);
         }
     }
     // the pool is empty: its memory holds the stacks of the lone searches
-    bool alone = false;
-    if (lane < nq) {
-        const uint32_t d = (uint32_t)(W.best[lane] >> 32);
-        alone = d < __float_as_uint(F_INF) && W.hidden[lane] == d;
-    }
+    float d = F_INF;
+    uint32_t id = INVALID;
+    bool alone = lane < nq && unpack_best(W.best[lane], d, id);
     for (uint64_t todo = __ballot(alone); todo; todo = __ballot(alone)) {
         const uint32_t r = rank_in(todo);
-        if (alone && r < W.cap / 64u) {
+        if (alone && r < W.cap / 128u) {
             const v3 p = W.point(lane);
-            float d;
-            uint32_t id;
             lane_nearest<DIM>(t, p, widened<DIM>(HwMath::sqrt(__uint_as_float(W.bound[lane])), p, scale),
                               W.pool + 128 * r, d, id);
             W.best[lane] = pack_best(d, id);
@@ -481,254 +514,267 @@ __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds&
 
 // ------------------------------------------------------------ silhouette
 
-// Per-wave LDS of the flattened leaf tests: one round of 64 edge slots (the
-// edge, then its distance with the sign bit set when it is not a silhouette),
-// the owner lane of each slot, and each owner's query point and bound.
-struct EdgeLds {
-    uint32_t edge[64];
-    float d[64];
-    uint8_t owner[64];
-    float px[64], py[64], pz[64], bound[64];
-};
-
-// The leaf tests of the lanes with `mine` set, spread over every lane of the
-// wave that runs this (all looping lanes, wave-uniformly): each owner lists
-// the edges of its (at most two) leaves as a run of slots, and in rounds of
-// 64 slots every lane computes the distance and the silhouette test of one,
-// then each owner applies its results in its original edge order, so ties and
-// the reference's early-out at distance 0 (scene.cuh:791) come out as in
-// sil_leaf.  3D, leaves of one primitive each.
-__device__ __forceinline__ void sil_leaves_wave(const TreeView& t, EdgeLds& L, bool mine, uint32_t la, bool ha,
-                                                uint32_t lb, bool hb, v3 p, bool flip, float& best,
-                                                uint32_t& best_e, Counts& cnt)
-{
-    const uint32_t lane = threadIdx.x & 63;
-    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    uint32_t ea = 0, eb = 0, sa = 0, sb = 0;
-    if (mine && ha && la < t.n_leaves) {
-        sa = __float_as_uint(t.tleaf[3 * la + 1].w);
-        ea = __float_as_uint(t.tleaf[3 * la + 2].w);
-    }
-    if (mine && hb && lb < t.n_leaves) {
-        sb = __float_as_uint(t.tleaf[3 * lb + 1].w);
-        eb = __float_as_uint(t.tleaf[3 * lb + 2].w);
-    }
-    ea = min(ea, 3u);
-    eb = min(eb, 3u);
-    const uint32_t my = ea + eb; // 0..6
-    const uint64_t b0 = __ballot(my & 1u), b1 = __ballot(my & 2u), b2 = __ballot(my & 4u);
-    const uint32_t off = (uint32_t)__popcll(b0 & lt) + 2u * (uint32_t)__popcll(b1 & lt) + 4u * (uint32_t)__popcll(b2 & lt);
-    const uint32_t total = (uint32_t)__popcll(b0) + 2u * (uint32_t)__popcll(b1) + 4u * (uint32_t)__popcll(b2);
-    if (mine) {
-        L.px[lane] = p.x;
-        L.py[lane] = p.y;
-        L.pz[lane] = p.z;
-        L.bound[lane] = best;
-        cnt.leaf += (ha ? 1u : 0u) + (hb ? 1u : 0u);
-        cnt.edge += my;
-    }
-    const uint64_t helpers = __ballot(true);
-    const uint32_t hr = (uint32_t)__popcll(helpers & lt), nh = (uint32_t)__popcll(helpers);
-    bool stop = false; // best reached 0: the owner's remaining edges are skipped
-    for (uint32_t base = 0; base < total; base += 64) {
-        // this round's slots [base, base + 64) of every owner
-        for (uint32_t k = 0; mine && k < my; ++k) {
-            const uint32_t sl = off + k;
-            if (sl >= base && sl < base + 64) {
-                L.edge[sl - base] = k < ea ? sa + k : sb + (k - ea);
-                L.owner[sl - base] = (uint8_t)lane;
-            }
-        }
-        // every lane of the wave (LDS operations of one wave complete in order)
-        const uint32_t n_round = min(64u, total - base);
-        for (uint32_t r = hr; r < n_round; r += nh) {
-            const uint32_t e = L.edge[r], o = L.owner[r];
-            const v3 q = mk(L.px[o], L.py[o], L.pz[o]);
-            const float b = L.bound[o], mr2 = b * b;
-            const float4 A = t.tedge[4 * e], B = t.tedge[4 * e + 1];
-            const uint32_t fl = __float_as_uint(B.w);
-            const v3 pa = mk(A.x, A.y, A.z), pb = mk(B.x, B.y, B.z);
-            v3 cp;
-            const float d = closest_point_segment(pa, pb, q, cp);
-            bool sil = (fl & 3u) != 3u; // a boundary edge is always a silhouette
-            if (!sil && d * d <= mr2) {
-                const float4 N0 = t.tedge[4 * e + 2], N1 = t.tedge[4 * e + 3];
-                sil = is_silhouette_edge(pa, pb, mk(N0.x, N0.y, N0.z), mk(N1.x, N1.y, N1.z),
-                                         mk(q.x - cp.x, q.y - cp.y, q.z - cp.z), d, flip);
-            }
-            L.d[r] = sil ? d : -d; // d >= 0: the sign bit carries "not a silhouette"
-        }
-        for (uint32_t k = 0; mine && !stop && k < my; ++k) {
-            const uint32_t sl = off + k;
-            if (sl < base || sl >= base + 64)
-                continue;
-            const float mr2 = best * best;
-            if (!(0.0f < mr2)) {
-                stop = true; // min_radius_squared (0) >= max_radius_squared
-                break;
-            }
-            const float sd = L.d[sl - base];
-            const float d = dm::fabs_(sd);
-            if (d * d > mr2 || dm::signbit_(sd))
-                continue;
-            const uint32_t e = k < ea ? sa + k : sb + (k - ea);
-            const uint32_t id = __float_as_uint(t.tedge[4 * e].w);
-            if (d < best || (d == best && id < best_e)) {
-                best = d;
-                best_e = id;
-            }
-        }
-    }
-}
-
-
-// query_device(nearest_silhouette) (query.cuh:325-423) for one query point.
-// best / best_e receive the answer.  The stack is a TrailStack: SSZ entries
-// in LDS and no private memory.  A finite radius `cap` prunes internal nodes
-// farther than cap as well.  When the search within cap ends with
-// best <= cap, every node that could hold a silhouette at least as close has
-// been visited; otherwise (HINT) it searches again from the root with no cap
-// and the bound found so far, or (hard cap, !HINT) it stops.  With index
-// tie-breaking the answer equals the uncapped search.
-template <int BS, int SSZ, bool STATS, int DIM, bool HINT, bool PARK>
-__device__ __forceinline__ void sil_query(const TreeView& t, v3 p, bool flip, float cap, uint32_t* stk_col,
-                                          EdgeLds* elds, float& best, uint32_t& best_e, Counts& cnt,
-                                          bool& overflow)
+// query_device(nearest_silhouette) (query.cuh:325-423) by one lane: near child
+// first, each node's leaves at once, with only nodes within the squared
+// distance w, and internal nodes within the squared radius cap2.  st: 128
+// words of LDS.
+template <int DIM>
+__device__ inline void lane_silhouette(const TreeView& t, v3 p, bool flip, float w, float cap2, uint32_t* st,
+                                       float& best, uint32_t& best_e)
 {
     best = F_INF;
     best_e = INVALID;
+    Counts cnt;
+    uint32_t sp = 0, node = 0;
+    for (uint32_t it = 0; it < 2 * t.n_leaves + 64 && node < t.n_leaves - 1; ++it) {
+        const NodeRec nr = load_node(t.tnode, node);
+        const float Lmd = box_mindist(nr.L, p), Rmd = box_mindist(nr.R, p), b2 = fmn(best * best, w);
+        const bool hL = Lmd <= b2 && cone_hit<DIM>(t, load_cone(t.tcone, node, 0u), p, nr.L, Lmd);
+        const bool hR = Rmd <= b2 && cone_hit<DIM>(t, load_cone(t.tcone, node, 1u), p, nr.R, Rmd);
+        uint32_t lf, lc, rf, rc;
+        const bool lLeaf = as_leaf(nr.lref, 0u, lf, lc), rLeaf = as_leaf(nr.rref, 1u, rf, rc);
+        if (hL && lLeaf)
+            for (uint32_t k = 0; k < lc; ++k)
+                sil_leaf<DIM>(t, lf + k, p, flip, best, best_e, cnt);
+        if (hR && rLeaf)
+            for (uint32_t k = 0; k < rc; ++k)
+                sil_leaf<DIM>(t, rf + k, p, flip, best, best_e, cnt);
+        const float nb2 = fmn(best * best, w);
+        const bool gL = hL && !lLeaf && Lmd <= nb2 && Lmd <= cap2, gR = hR && !rLeaf && Rmd <= nb2 && Rmd <= cap2;
+        const bool lfirst = Lmd <= Rmd;
+        if (gL && gR && sp < 64u) {
+            st[2 * sp] = lfirst ? nr.rref : nr.lref;
+            st[2 * sp + 1] = __float_as_uint(lfirst ? Rmd : Lmd);
+            ++sp;
+        }
+        if (gL || gR) {
+            node = gL && (lfirst || !gR) ? nr.lref : nr.rref;
+            continue;
+        }
+        bool found = false;
+        while (sp > 0 && !found) {
+            --sp;
+            node = st[2 * sp];
+            found = __uint_as_float(st[2 * sp + 1]) <= nb2; // query.cuh:347
+        }
+        if (!found)
+            break;
+    }
+}
+
+// a silhouette at distance d of a leaf with box bound key becomes a candidate of query `slot`
+template <int DIM>
+__device__ __forceinline__ void sil_found(WaveLds& W, uint32_t slot, v3 p, float scale, float key, float d, uint32_t id)
+{
+    atomicMin(&W.best[slot], pack_best(d, id, key > d * d));
+    atomicMin(&W.bound[slot], __float_as_uint(widened<DIM>(d, p, scale)));
+}
+
+// evaluates the last (up to 64) leaves of the wave's buffer; returns how many
+// are left.  3D: a leaf owns 0..3 edges; the wave lists the edges of all its
+// leaves as slots and tests one per lane in rounds of 64.
+template <bool STATS, int DIM>
+__device__ __forceinline__ uint32_t sil_leaves(const TreeView& t, WaveLds& W, uint32_t nleaf, float scale, bool flip,
+                                               Counts& cnt)
+{
+    const uint32_t lane = threadIdx.x & 63, k = min(64u, nleaf);
+    nleaf -= k;
+    uint32_t w = 0, es = 0, ec = 0;
+    float key = F_INF;
+    bool mine = false;
+    if (lane < k) {
+        w = W.leaf[2 * (nleaf + lane)];
+        key = __uint_as_float(W.leaf[2 * (nleaf + lane) + 1]);
+        mine = key <= __uint_as_float(W.bound[w >> 24]) && (w & REF_MASK) < t.n_leaves;
+    }
+    const uint32_t slot = w >> 24, j = w & REF_MASK;
+    if (STATS && mine)
+        cnt.leaf += 1;
+    if (DIM == 2) {
+        if (mine) {
+            const v3 p = W.point(slot);
+            float d = F_INF;
+            uint32_t id = INVALID;
+            Counts c;
+            sil_leaf<DIM>(t, j, p, flip, d, id, c);
+            if (STATS)
+                cnt.edge += c.edge;
+            if (id != INVALID && d * d <= __uint_as_float(W.bound[slot]))
+                sil_found<DIM>(W, slot, p, scale, key, d, id);
+        }
+        return nleaf;
+    }
+    if (mine) {
+        es = __float_as_uint(t.tleaf[3 * j + 1].w);
+        ec = min(__float_as_uint(t.tleaf[3 * j + 2].w), 3u);
+    }
+    if (STATS)
+        cnt.edge += ec;
+    const uint64_t b0 = __builtin_amdgcn_ballot_w64((ec & 1u) != 0u), b1 = __builtin_amdgcn_ballot_w64((ec & 2u) != 0u);
+    const uint32_t off = rank_in(b0) + 2u * rank_in(b1);
+    const uint32_t total = (uint32_t)__popcll(b0) + 2u * (uint32_t)__popcll(b1);
+    uint32_t* list = W.leaf + 2 * nleaf; // the popped entries' words: owner lane << 26 | edge
+    for (uint32_t base = 0; base < total; base += 64) {
+#pragma unroll
+        for (uint32_t i = 0; i < 3; ++i) {
+            const uint32_t at = off + i - base;
+            if (i < ec && at < 64u)
+                list[at] = (lane << 26) | (es + i);
+        }
+        const bool on = lane < min(64u, total - base);
+        const uint32_t l = on ? list[lane] : 0u, e = l & 0x03FFFFFFu;
+        const uint32_t s = (uint32_t)__shfl((int)slot, (int)(l >> 26), 64);
+        const float kk = __shfl(key, (int)(l >> 26), 64);
+        if (on) {
+            const v3 p = W.point(s);
+            const float b = __uint_as_float(W.bound[s]);
+            const float4 A = t.tedge[4 * e], B = t.tedge[4 * e + 1];
+            const v3 pa = mk(A.x, A.y, A.z), pb = mk(B.x, B.y, B.z);
+            v3 cp;
+            const float d = closest_point_segment(pa, pb, p, cp);
+            if (d * d <= b) {
+                bool sil = (__float_as_uint(B.w) & 3u) != 3u; // a boundary edge is always a silhouette
+                if (!sil) {
+                    const float4 N0 = t.tedge[4 * e + 2], N1 = t.tedge[4 * e + 3];
+                    sil = is_silhouette_edge(pa, pb, mk(N0.x, N0.y, N0.z), mk(N1.x, N1.y, N1.z),
+                                             mk(p.x - cp.x, p.y - cp.y, p.z - cp.z), d, flip);
+                }
+                if (sil)
+                    sil_found<DIM>(W, s, p, scale, kk, d, __float_as_uint(A.w));
+            }
+        }
+    }
+    return nleaf;
+}
+
+// query_device(nearest_silhouette) (query.cuh:325-423) for the queries of a
+// wave, a slot per bit of `all` (WaveLds::start): W.best receives (distance,
+// silhouette id).  Run by the whole wave.
+// MODE 0: plain.  MODE 1: `cap` (per lane) is a hint: the search within it
+// first; a query with no answer there enters again without it (the pool
+// spreads it over all lanes, so the rest of the wave does not wait for one
+// lane).  Outputs equal MODE 0's.  MODE 2: `cap` is hard: internal nodes
+// farther than it are not visited.
+template <bool STATS, int DIM, int MODE>
+__device__ __forceinline__ void sil_wave(const TreeView& t, uint64_t all, bool flip, float cap, WaveLds& W,
+                                         Counts& cnt, bool& overflow)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    const bool valid = (all >> lane) & 1ull;
     if (t.n_leaves == 1) {
-        const box3 b = ldbox2(t.nbox, 0);
-        const float4 c0 = t.ncone[0], c1 = t.ncone[1];
-        if (cone_valid(c0.w) && overlap_dim<DIM>(c0, c1.x, p, b, box_mindist(b, p)))
-            sil_leaf<DIM>(t, 0, p, flip, best, best_e, cnt);
+        if (valid) {
+            const v3 p = W.point(lane);
+            const box3 b = ldbox2(t.nbox, 0);
+            const float4 c0 = t.ncone[0], c1 = t.ncone[1];
+            float d = F_INF;
+            uint32_t id = INVALID;
+            if (cone_valid(c0.w) && overlap_dim<DIM>(c0, c1.x, p, b, box_mindist(b, p)))
+                sil_leaf<DIM>(t, 0, p, flip, d, id, cnt);
+            W.best[lane] = pack_best(d, id);
+        }
         return;
     }
     if (!(cap >= 0.0f))
         cap = F_INF;
-    float cap2 = cap * cap;
-    TrailStack<BS, SSZ> st;
-    st.init(stk_col, t.qbase);
-    uint32_t node = 0;
-    // a pass visits each internal node at most once; restarts add the paths
-    // above lost far children (a few per query); the bound only guards
-    // against an inconsistent tree, and hitting it is reported as an overflow
-    const uint32_t cap_iters = 8 * t.n_leaves + 8192;
-    uint32_t it = 0;
-    // A lane whose node has leaf children to evaluate parks them (phase
-    // `leaves`) until a quarter of the wave's looping lanes, or all of them,
-    // are parked; the parked lanes then evaluate their leaves together and
-    // decide the node's internal children with the bound found, exactly as
-    // if the leaves had been evaluated at once.  The leaf code then runs on
-    // many lanes at a time instead of on the few that reached a leaf (about
-    // 5 of 64 on the 1M-triangle torus: 99.6 -> 89 ms).  Hard-capped searches
-    // (!HINT: short, as in walk on stars) evaluate leaves at once.
-    bool leaves = false;
-    float Lmd = 0.0f, Rmd = 0.0f;
-    bool hL = false, hR = false, lLeaf = false, rLeaf = false;
-    uint32_t lref = 0, rref = 0, lf = 0, lc = 0, rf = 0, rc = 0;
-    for (; it < cap_iters && node < t.n_leaves - 1;) {
-        bool decide = false;
-        if (!leaves) {
-            ++it;
-            const NodeRec nr = load_node(t.tnode, node);
-            Lmd = box_mindist(nr.L, p);
-            Rmd = box_mindist(nr.R, p);
-            const float b2 = best * best;
-            hL = Lmd <= b2;
-            hR = Rmd <= b2;
-            if (STATS) {
-                cnt.node += 1;
-                cnt.box += 2;
-            }
-            if (hL || hR) {
-                if (STATS)
-                    cnt.cone += 1;
-                const float4 CL = t.tcone[4 * node], CR = t.tcone[4 * node + 1], Cr = t.tcone[4 * node + 2];
-                // query.cuh:366-367
-                if (DIM == 3 && (t.flags & TREE_FAST_CONE)) {
-                    const float4 SC = t.tcone[4 * node + 3];
-                    hL = hL && cone_valid(CL.w) &&
-                         cone_overlap_fast(mk(CL.x, CL.y, CL.z), CL.w, SC.x, SC.y, Cr.x, p, nr.L, Lmd);
-                    hR = hR && cone_valid(CR.w) &&
-                         cone_overlap_fast(mk(CR.x, CR.y, CR.z), CR.w, SC.z, SC.w, Cr.y, p, nr.R, Rmd);
-                } else {
-                    hL = hL && cone_valid(CL.w) && overlap_dim<DIM>(CL, Cr.x, p, nr.L, Lmd);
-                    hR = hR && cone_valid(CR.w) && overlap_dim<DIM>(CR, Cr.y, p, nr.R, Rmd);
+    const float scale = scene_scale(t);
+    if (MODE == 1 && valid && cap < F_INF)
+        W.bound[lane] = __float_as_uint(widened<DIM>(cap, W.point(lane), scale));
+    if (MODE == 2 && valid)
+        W.cap2()[lane] = cap * cap;
+    uint32_t size = 0, nleaf = 0;
+    uint64_t todo = all;
+    bool hinted = MODE == 1;
+    // every iteration pops a node of some query (each at most once, twice
+    // with a hint) or evaluates leaves; the bound only guards against a
+    // malformed tree
+    const uint32_t cap_iters = 128u * t.n_leaves + 65536u;
+    for (uint32_t it = 0;; ++it) {
+        if (nleaf >= LEAF_RUN || (nleaf > 0u && todo == 0ull && size < 32u)) {
+            nleaf = sil_leaves<STATS, DIM>(t, W, nleaf, scale, flip, cnt);
+            continue;
+        }
+        if (size == 0u && todo == 0ull) {
+            if (!hinted)
+                break;
+            // the queries without an answer within their hint enter again
+            hinted = false;
+            float d = F_INF;
+            uint32_t id = INVALID;
+            if (valid)
+                unpack_best(W.best[lane], d, id);
+            const bool again = valid && cap < F_INF && !(id != INVALID && d <= cap);
+            if (again)
+                W.bound[lane] = __float_as_uint(id != INVALID ? widened<DIM>(d, W.point(lane), scale) : F_INF);
+            todo = __builtin_amdgcn_ballot_w64(again);
+            continue;
+        }
+        if (it >= cap_iters) {
+            overflow = true;
+            break;
+        }
+        if (size < 32u && todo != 0ull)
+            pool_feed(W, size, todo);
+        const uint32_t k = pool_take(size, W.cap), side = lane & 1u;
+        size -= k;
+        uint32_t slot = 0, ref = 0;
+        float md = F_INF;
+        bool go = false;
+        if ((lane >> 1) < k) {
+            const uint32_t at = size + (lane >> 1), w = W.pool[at], node = w & REF_MASK;
+            slot = w >> 24;
+            const float b = __uint_as_float(W.bound[slot]);
+            if (__uint_as_float((uint32_t)W.pkey[at] << 16) <= b && node < t.n_leaves - 1) {
+                const v3 p = W.point(slot);
+                const ChildRec c = load_child(t.tnode, node, side);
+                const ConeRec cone = load_cone(t.tcone, node, side);
+                ref = c.ref;
+                md = box_mindist(c.box, p);
+                go = md <= b && cone_hit<DIM>(t, cone, p, c.box, md);
+                if (STATS) {
+                    cnt.node += side;
+                    cnt.cone += side;
+                    cnt.box += 1;
                 }
             }
-            lref = nr.lref;
-            rref = nr.rref;
-            lLeaf = as_leaf(nr.lref, 0u, lf, lc);
-            rLeaf = as_leaf(nr.rref, 1u, rf, rc);
-            leaves = (hL && lLeaf) || (hR && rLeaf);
-            decide = !leaves;
         }
-        const uint64_t parked = __ballot(leaves), looping = __ballot(true);
-        if (parked &&
-            (!PARK || 4u * (uint32_t)__popcll(parked) >= (uint32_t)__popcll(looping) || parked == looping)) {
-            // wave-uniform: the parked lanes' leaves are tested now
-            const bool la = hL && lLeaf, ra = hR && rLeaf;
-            const bool runs = __ballot(leaves && ((la && lc > 1) || (ra && rc > 1))) != 0;
-            if (DIM == 3 && elds && !runs) {
-                sil_leaves_wave(t, *elds, leaves, lf, la, rf, ra, p, flip, best, best_e, cnt);
-            } else if (leaves) {
-                if (la)
-                    for (uint32_t k = 0; k < lc; ++k)
-                        sil_leaf<DIM>(t, lf + k, p, flip, best, best_e, cnt);
-                if (ra)
-                    for (uint32_t k = 0; k < rc; ++k)
-                        sil_leaf<DIM>(t, rf + k, p, flip, best, best_e, cnt);
-            }
-            decide = decide || leaves;
-            leaves = false;
+        uint32_t first, count;
+        const bool leaf = as_leaf(ref, side, first, count);
+        const float other = pair_other(md);
+        const bool lt = md < other, eq = md == other, near = lt || (eq && !side);
+        const bool down = go && !leaf && (MODE != 2 || md <= W.cap2()[slot]);
+        pool_push(W, size, down && !near, (slot << 24) | (ref & REF_MASK), md);
+        pool_push(W, size, down && near, (slot << 24) | (ref & REF_MASK), md);
+        list_push(W.leaf, nleaf, go && leaf, (slot << 24) | first, md);
+        for (uint32_t j = 1; (t.flags & TREE_RUNS) && __ballot(go && leaf && j < count); ++j) {
+            if (nleaf >= LEAF_RUN)
+                nleaf = sil_leaves<STATS, DIM>(t, W, nleaf, scale, flip, cnt);
+            list_push(W.leaf, nleaf, go && leaf && j < count, (slot << 24) | (first + j), md);
         }
-        if (!decide)
-            continue;
-        // internal children to descend: within the bound and the cap
-        const float nb2 = best * best;
-        const bool gL = hL && !lLeaf && Lmd <= nb2 && Lmd <= cap2;
-        const bool gR = hR && !rLeaf && Rmd <= nb2 && Rmd <= cap2;
-        if ((gL || gR) && st.lv >= 63u) {
-            overflow = true; // deeper than a Karras tree can be
-            break;
-        }
-        const bool lfirst = Lmd <= Rmd;
-        if (st.descend(lfirst ? gL : gR, lfirst ? gR : gL, lfirst ? lref : rref, lfirst ? rref : lref,
-                       lfirst ? Rmd : Lmd, node))
-            continue;
-        bool found = false;
-        while (st.M) {
-            uint32_t nn;
-            float dd;
-            st.pop(nn, dd);
-            if (dd <= best * best) { // query.cuh:347
-                node = nn;
-                found = true;
-                break;
-            }
-        }
-        if (found)
-            continue;
-        if (st.restart()) {
-            node = 0;
-            continue;
-        }
-        // the search within the cap is over: settled, or (HINT) search again
-        // from the root with no cap and the bound found so far
-        if (cap2 == F_INF || (best_e != INVALID && best <= cap) || !HINT)
-            break;
-        cap2 = F_INF;
-        st.reset();
-        node = 0;
     }
-    overflow = overflow || it >= cap_iters;
+    // hidden answers, and answers at distance 0, where the reference stops at
+    // the first edge it meets (scene.cuh:791): the lone search decides
+    float d = F_INF;
+    uint32_t id = INVALID;
+    const bool hidden = valid && unpack_best(W.best[lane], d, id);
+    bool alone = hidden || (id != INVALID && !(d * d > 0.0f));
+    for (uint64_t left = __ballot(alone); left; left = __ballot(alone)) {
+        const uint32_t r = rank_in(left);
+        if (alone && r < W.cap / 128u) {
+            const v3 p = W.point(lane);
+            lane_silhouette<DIM>(t, p, flip, widened<DIM>(HwMath::sqrt(__uint_as_float(W.bound[lane])), p, scale),
+                                 MODE == 2 ? W.cap2()[lane] : F_INF, W.pool + 128 * r, d, id);
+            W.best[lane] = pack_best(d, id);
+            alone = false;
+        }
+    }
 }
 
-// the next 64-query chunk of nchunks for a one-wave block of a persistent
-// launch: its own XCD's contiguous range first (x0: the block's XCD), then
-// the other XCDs' ranges; xi counts the ranges exhausted (wave-uniform).
-// ctr: [0, 8) the ranges' counters.  INVALID when none is left.
+// ------------------------------------------------------------ launches
+
+// the next chunk of nchunks for a wave of a persistent launch: its XCD's
+// contiguous range first (x0: the block's XCD), then the other XCDs' ranges;
+// xi counts the ranges exhausted (wave-uniform).  ctr: [0, 8) the ranges'
+// counters (zero at launch).  INVALID when none is left.
 __device__ __forceinline__ uint32_t take_chunk(uint32_t* ctr, uint32_t nchunks, uint32_t x0, uint32_t& xi)
 {
     while (xi < 8u) {
@@ -736,7 +782,7 @@ __device__ __forceinline__ uint32_t take_chunk(uint32_t* ctr, uint32_t nchunks, 
         const uint32_t lo = (uint32_t)((uint64_t)nchunks * xx / 8u);
         const uint32_t hi = (uint32_t)((uint64_t)nchunks * (xx + 1u) / 8u);
         uint32_t k = 0;
-        if (threadIdx.x == 0)
+        if ((threadIdx.x & 63u) == 0)
             k = atomicAdd(ctr + xx, 1u);
         k = uniform(k);
         if (k < hi - lo)
@@ -745,8 +791,68 @@ __device__ __forceinline__ uint32_t take_chunk(uint32_t* ctr, uint32_t nchunks, 
     }
     return INVALID;
 }
+constexpr uint32_t CHUNK_CTR_WORDS = 8;
+
+// queries per wave of a launch over n: 64 consecutive ones of the visiting
+// order, or fewer when that would leave resident waves without work
+__host__ __device__ __forceinline__ uint32_t queries_per_wave(uint32_t n, uint32_t waves)
+{
+    const uint32_t w = waves > 0u ? waves : 1u, k = n / w + (n % w ? 1u : 0u);
+    return k < 1u ? 1u : k > 64u ? 64u : k;
+}
+
+// Calls f(slot, valid) with the queries of each chunk of this wave.  Chunks of
+// 64 are consecutive queries of the visiting order; smaller ones take every
+// nchunks-th query, so that costly neighbours (the centre of a sphere) land in
+// different waves.  One chunk per wave where there are waves enough; else
+// (ctr, a persistent launch) the waves take chunks as they get free.
+template <class F>
+__device__ __forceinline__ void for_chunks(uint32_t n, uint32_t qpw, uint32_t* ctr, F f)
+{
+    const uint32_t lane = threadIdx.x & 63, wpb = blockDim.x >> 6, w = threadIdx.x >> 6;
+    const uint32_t waves = gridDim.x * wpb, nchunks = n / qpw + (n % qpw ? 1u : 0u);
+    auto chunk = [&](uint32_t c) {
+        const uint32_t slot = qpw < 64u ? lane * nchunks + c : c * 64u + lane;
+        f(slot, lane < qpw && slot < n);
+    };
+    if (nchunks <= waves || !ctr) {
+        const uint32_t c = uniform(xcd_remap(blockIdx.x, gridDim.x) * wpb + w);
+        if (c < nchunks)
+            chunk(c);
+        return;
+    }
+    uint32_t xi = 0;
+    for (uint32_t c = take_chunk(ctr, nchunks, blockIdx.x % 8u, xi); c != INVALID;
+         c = take_chunk(ctr, nchunks, blockIdx.x % 8u, xi))
+        chunk(c);
+}
 
 inline uint32_t nblocks(uint32_t n, uint32_t bs) { return (n + bs - 1) / bs; }
+
+// grid of a search launch: a wave per chunk, or (persist) as many waves as
+// are resident (lds bytes of LDS and at most `per_simd` waves on a SIMD)
+struct SearchGrid {
+    dim3 grid, block;
+    uint32_t qpw;
+    size_t lds;
+    bool persist;
+};
+inline SearchGrid search_grid(uint32_t n, uint32_t block, uint32_t depth, bool capped, uint32_t n_cu,
+                              uint32_t per_simd, bool may_persist, bool n_on_device)
+{
+    SearchGrid g;
+    const uint32_t wpb = block / 64;
+    g.lds = sizeof(uint32_t) * wpb * wave_lds_words(pool_cap(depth), capped);
+    const uint32_t per_cu = std::max(1u, std::min((uint32_t)(LDS_PER_CU / g.lds), per_simd * 4u / wpb));
+    const uint32_t resident = n_cu * per_cu;
+    g.qpw = n_on_device ? 0u : queries_per_wave(n, resident * wpb); // 0: from the count on the device
+    const uint32_t blocks = nblocks(nblocks(n, g.qpw ? g.qpw : 1u), wpb);
+    g.persist = may_persist && blocks > resident;
+    g.grid = dim3(g.persist ? resident : blocks);
+    g.block = dim3(block);
+    return g;
+}
+
 
 } // namespace
 

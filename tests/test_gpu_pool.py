@@ -56,3 +56,38 @@ def test_closest_point_does_not_depend_on_the_launch(name, leaf_size):
     # the last place of the coordinates
     ref = oracle.bf_closest_point(V, F, q[:2000])[1]
     assert np.abs(d0[:2000] - ref).max() <= 8 * np.spacing(np.abs(q).max())
+
+
+@pytest.mark.parametrize("name", ["ico", "ico_far", "box_far", "two"])
+@pytest.mark.parametrize("leaf_size", [1, 8])
+def test_closest_silhouette_does_not_depend_on_the_launch(name, leaf_size):
+    import snch_lbvh_amd as S
+
+    V, F = _meshes()[name]
+    q = _points(V, 70000, 12)
+    sc = S.Scene(V, F).build_bvh(leaf_size=leaf_size)
+    np_ = lambda r: tuple(x.cpu().numpy() for x in r)  # noqa: E731
+    for flip in (False, True):
+        e0, d0 = np_(sc.closest_silhouette(q, flip=flip))
+        for n in (1, 2, 20, 21, 63, 64, 65, 1000):
+            e1, d1 = np_(sc.closest_silhouette(q[:n], flip=flip))
+            np.testing.assert_array_equal(d1, d0[:n])
+            np.testing.assert_array_equal(e1, e0[:n])
+        for kw in ({"block_size": 512}, {"block_size": 128, "stack_depth": 8}, {"stack_depth": 32}, {"coherent": 2}):
+            e1, d1 = np_(sc.closest_silhouette(q, flip=flip, **kw))
+            np.testing.assert_array_equal(d1, d0)
+            np.testing.assert_array_equal(e1, e0)
+        # hints too small, about right, too large, zero and none
+        r = np.random.default_rng(3)
+        seed = np.where(np.isfinite(d0), d0, 1.0) * r.choice([0.0, 0.5, 1.0, 1.25, np.inf], len(d0))
+        for n in (65, len(q)):
+            e1, d1 = np_(sc.closest_silhouette(q[:n], flip=flip, seed_radius=seed[:n].astype(np.float32)))
+            np.testing.assert_array_equal(d1, d0[:n])
+            np.testing.assert_array_equal(e1, e0[:n])
+        # a hard cap: the answer where it lies within, else something farther
+        cap = (np.where(np.isfinite(d0), d0, 1.0) * r.choice([0.5, 1.25], len(d0))).astype(np.float32)
+        e1, d1 = np_(sc.closest_silhouette(q, flip=flip, seed_radius=cap, seed_is_cap=True))
+        within = d0 <= cap
+        np.testing.assert_array_equal(d1[within], d0[within])
+        np.testing.assert_array_equal(e1[within], e0[within])
+        assert np.all(d1[~within] > cap[~within])
