@@ -157,9 +157,9 @@ hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q,
                                      const float* seed, bool capped, uint32_t* sil, float* dist, uint32_t block,
                                      uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t* ctr,
                                      uint32_t n_cu, hipStream_t st, uint32_t* err = nullptr);
-hipError_t launch_ray(const TreeView& t, int dim, const float* o, const float* d, const float* tmax, uint32_t n,
-                      int any_hit, uint8_t* hit, float* tout, float* uv, uint32_t* idx, uint64_t* stats,
-                      hipStream_t st);
+hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* o, const float* d,
+                      const float* tmax, uint32_t n, int any_hit, uint8_t* hit, float* tout, float* uv, uint32_t* idx,
+                      uint64_t* stats, uint32_t* ctr, uint32_t n_cu, hipStream_t st);
 hipError_t launch_sample(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* c,
                          const float* r, const float* u, uint32_t n, int32_t* idx, float* pdf, float* pt,
                          hipStream_t st);

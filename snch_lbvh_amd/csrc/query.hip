@@ -8,14 +8,11 @@
 //    boxes and references, 32 B each; the silhouette query reads a cone record
 //    from a separate stream, so the closest-point and ray queries never touch
 //    it.
-//  * The closest-point search runs a wave's queries from one pool of pending
-//    nodes in LDS (wave_search.hpp).  Rays keep a short per-lane stack in LDS
-//    (16 packed entries, a column per lane so a wave's 64 lanes hit distinct
-//    banks) with a restart trail (TrailStack): nothing in private memory; a
-//    far child pushed out of the full stack is found again from the trail.
-//    The generic overlap and line queries, which must emit hits in the
-//    reference's visit order, keep 16 LDS entries over a private overflow
-//    array (the tree depth is at most 64, so it never loses one).
+//  * The searches run a wave's queries from one pool of pending nodes in LDS
+//    (wave_search.hpp).  The generic overlap and line queries, which must emit
+//    hits in the reference's visit order, keep 16 LDS entries per lane over a
+//    private overflow array (the tree depth is at most 64, so it never loses
+//    one).
 //  * Order: the nearer child is descended first and the farther is pushed,
 //    and a child is skipped when its lower bound exceeds the best answer so
 //    far.  The reference's own pruning predicates (minmaxdist for closest
@@ -34,6 +31,7 @@ namespace snch {
 
 namespace {
 
+constexpr int SS = 16;  // LDS stack entries per lane (generic queries)
 constexpr int OVF = 64; // private overflow entries per lane (generic queries)
 
 // ------------------------------------------------------------ closest point
@@ -73,145 +71,75 @@ __global__ __launch_bounds__(512, 6) void k_closest_point(TreeView t, const floa
 }
 
 // ------------------------------------------------------------ ray
-template <int BS, bool STATS, int DIM>
-__global__ __launch_bounds__(BS) void k_ray(TreeView t, const float* __restrict__ o, const float* __restrict__ d,
-                                            const float* __restrict__ tmax, uint32_t n, int any_hit,
-                                            uint8_t* __restrict__ out_hit, float* __restrict__ out_t,
-                                            float* __restrict__ out_uv, uint32_t* __restrict__ out_idx,
-                                            uint32_t* __restrict__ err, unsigned long long* stats)
+// out_uv: the hit's barycentrics (2D: the segment parameter), from the hit
+// test of the triangle found
+template <bool STATS, int DIM, bool ANY>
+__global__ __launch_bounds__(64, 6) void k_ray(TreeView t, const float4* __restrict__ V, const int32_t* __restrict__ F,
+                                               const float* __restrict__ o, const float* __restrict__ d,
+                                               const float* __restrict__ tmax, uint32_t n, uint32_t qpw,
+                                               uint8_t* __restrict__ out_hit, float* __restrict__ out_t,
+                                               float* __restrict__ out_uv, uint32_t* __restrict__ out_idx,
+                                               uint32_t* ctr, uint32_t* __restrict__ err, unsigned long long* stats)
 {
-    __shared__ uint32_t stk[SS * BS];
-    const uint32_t qi = xcd_remap(blockIdx.x, gridDim.x) * BS + threadIdx.x;
-    Counts cnt;
+    __shared__ __align__(16) uint32_t smem[RayLds::WORDS];
+    const uint32_t lane = threadIdx.x & 63;
+    RayLds W(smem);
     if (t.n_dev)
         n = min(n, *t.n_dev);
-    if (qi >= n) {
-        if (STATS)
-            flush_counts(cnt, stats);
-        return;
-    }
-    const v3 ro = load_point<DIM>(o, qi);
-    const v3 rd = load_point<DIM>(d, qi);
-    const v3 inv = mk(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z); // aabb.cuh:308-311 (2D: z slab inert)
-    const float max_dist = tmax ? tmax[qi] : F_INF;
-    float tbest = F_INF, bu = 0.0f, bv = 0.0f;
-    uint32_t bidx = INVALID;
-    bool found = false;
-    auto leaf = [&](uint32_t j) {
-        if (j >= t.n_leaves)
+    if (qpw == 0u)
+        qpw = queries_per_wave(n, gridDim.x);
+    bool ovf = false;
+    Counts cnt;
+    for_chunks(n, qpw, ctr, [&](uint32_t qi, bool valid) {
+        float max_dist = F_INF;
+        v3 ro = mk(0.0f, 0.0f, 0.0f), rd = ro;
+        if (valid) {
+            ro = load_point<DIM>(o, qi);
+            rd = load_point<DIM>(d, qi);
+            if (tmax)
+                max_dist = tmax[qi];
+            // aabb.cuh:308-311 (2D: z slab inert)
+            W.start(lane, ro, rd, mk(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z), max_dist);
+        }
+        ray_wave<STATS, DIM, ANY>(t, __ballot(valid), max_dist, W, cnt, ovf);
+        if (!valid)
             return;
-        if (STATS)
-            cnt.leaf += 1;
-        const float4 a = t.tleaf[3 * j], b = t.tleaf[3 * j + 1];
-        float th, uh, vh = 0.0f;
-        const uint32_t o = __float_as_uint(a.w);
-        bool h;
-        if (DIM == 3) {
-            const float4 c = t.tleaf[3 * j + 2];
-            h = ray_triangle(ro, rd, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), mk(c.x, c.y, c.z), th, uh, vh);
-        } else {
-            h = ray_segment(ro, rd, mk(a.x, a.y, 0.0f), mk(b.x, b.y, 0.0f), th, uh);
-        }
-        if (h && th < max_dist && (th < tbest || (th == tbest && o < bidx))) { // query.cuh:115
-            tbest = th;
-            bu = uh;
-            bv = vh;
-            bidx = o;
-            found = true;
-        }
-    };
-    if (t.n_leaves == 1) {
-        leaf(0);
-    } else {
-        // the closest hit only shrinks, so the restart-trail stack applies
-        TrailStack<BS, SS> st;
-        st.init(stk + threadIdx.x, t.qbase);
-        uint32_t node = 0;
-        const uint32_t cap_iters = 8 * t.n_leaves + 8192;
-        uint32_t it = 0;
-        bool deep = false;
-        for (; it < cap_iters && node < t.n_leaves - 1; ++it) {
-            const NodeRec nr = load_node(t.tnode, node);
-            float Ld = F_INF, Rd = F_INF;
-            if (STATS) {
-                cnt.node += 1;
-                cnt.box += 2;
-            }
-            const bool bL = box_ray(nr.L, ro, inv, max_dist, Ld), bR = box_ray(nr.R, ro, inv, max_dist, Rd);
-            const bool Lh = bL && Ld <= tbest;
-            const bool Rh = bR && Rd <= tbest;
-            uint32_t lf, lc, rf, rc;
-            const bool lLeaf = as_leaf(nr.lref, 0u, lf, lc), rLeaf = as_leaf(nr.rref, 1u, rf, rc);
-            // nearer child first, as query.cuh:136-149
-            const bool rfirst = Lh && Rh && Rd < Ld;
-            if (rfirst) {
-                if (Rh && rLeaf)
-                    for (uint32_t k = 0; k < rc; ++k)
-                        leaf(rf + k);
-                if (Lh && lLeaf && Ld <= tbest)
-                    for (uint32_t k = 0; k < lc; ++k)
-                        leaf(lf + k);
+        float tbest;
+        uint32_t idx;
+        unpack_best(W.best[lane], tbest, idx);
+        const bool found = idx != INVALID;
+        if (out_hit)
+            out_hit[qi] = found ? 1 : 0;
+        if (ANY)
+            return;
+        float u = 0.0f, v = 0.0f;
+        if (found && (out_uv || out_t)) {
+            const v3 o2 = W.origin(lane), d2 = W.dir(lane);
+            if (DIM == 3) {
+                const float4 a = V[F[3 * idx]], b = V[F[3 * idx + 1]], c = V[F[3 * idx + 2]];
+                ray_triangle(o2, d2, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), mk(c.x, c.y, c.z), tbest, u, v);
             } else {
-                if (Lh && lLeaf)
-                    for (uint32_t k = 0; k < lc; ++k)
-                        leaf(lf + k);
-                if (Rh && rLeaf && Rd <= tbest)
-                    for (uint32_t k = 0; k < rc; ++k)
-                        leaf(rf + k);
+                const float4 a = V[F[2 * idx]], b = V[F[2 * idx + 1]];
+                ray_segment(o2, d2, mk(a.x, a.y, 0.0f), mk(b.x, b.y, 0.0f), tbest, u);
             }
-            if (any_hit && found)
-                break;
-            const bool gL = Lh && !lLeaf && Ld <= tbest;
-            const bool gR = Rh && !rLeaf && Rd <= tbest;
-            if ((gL || gR) && st.lv >= 63u) {
-                deep = true; // deeper than a Karras tree can be
-                break;
-            }
-            // near and far by geometry alone (a box the ray misses is far), so
-            // every pass orders a node's children alike; with both boxes hit
-            // this is query.cuh:136-149's order
-            const bool lnear = bL && (!bR || !(Rd < Ld));
-            if (st.descend(lnear ? gL : gR, lnear ? gR : gL, lnear ? nr.lref : nr.rref, lnear ? nr.rref : nr.lref,
-                           lnear ? Rd : Ld, node))
-                continue;
-            bool more = false;
-            while (st.M) {
-                uint32_t nn;
-                float dd;
-                st.pop(nn, dd);
-                if (dd <= tbest) { // query.cuh:106
-                    node = nn;
-                    more = true;
-                    break;
-                }
-            }
-            if (more)
-                continue;
-            if (!st.restart())
-                break;
-            node = 0;
         }
-        if ((deep || it >= cap_iters) && err)
-            atomicOr(err, 1u);
-    }
-    if (out_hit)
-        out_hit[qi] = found ? 1 : 0;
+        if (out_t)
+            out_t[qi] = tbest;
+        if (out_uv) {
+            if (DIM == 3) {
+                out_uv[2 * qi] = u;
+                out_uv[2 * qi + 1] = v;
+            } else {
+                out_uv[qi] = u; // segment parameter s
+            }
+        }
+        if (out_idx)
+            out_idx[qi] = idx;
+    });
+    if (ovf && err)
+        atomicOr(err, 1u);
     if (STATS)
         flush_counts(cnt, stats);
-    if (any_hit)
-        return;
-    if (out_t)
-        out_t[qi] = tbest;
-    if (out_uv) {
-        if (DIM == 3) {
-            out_uv[2 * qi] = bu;
-            out_uv[2 * qi + 1] = bv;
-        } else {
-            out_uv[qi] = bu; // segment parameter s
-        }
-    }
-    if (out_idx)
-        out_idx[qi] = bidx;
 }
 
 // ------------------------------------------------------------ sampling
@@ -500,7 +428,7 @@ hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint
     if (n == 0)
         return hipSuccess;
     auto* sp = reinterpret_cast<unsigned long long*>(stats);
-    const SearchGrid g = search_grid(n, block, depth, false, n_cu, 6, ctr != nullptr, t.n_dev != nullptr);
+    const SearchGrid g = search_grid(n, block, wave_lds_words(pool_cap(depth)), n_cu, 6, ctr != nullptr, t.n_dev != nullptr);
     uint32_t* c = g.persist ? ctr : nullptr;
     if (c)
         hipLaunchKernelGGL(k_clear_chunks, dim3(1), dim3(64), 0, st, c);
@@ -515,21 +443,33 @@ hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint
     return hipGetLastError();
 }
 
-hipError_t launch_ray(const TreeView& t, int dim, const float* o, const float* d, const float* tmax, uint32_t n,
-                      int any_hit, uint8_t* hit, float* tout, float* uv, uint32_t* idx, uint64_t* stats,
-                      hipStream_t st)
+hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* o, const float* d,
+                      const float* tmax, uint32_t n, int any_hit, uint8_t* hit, float* tout, float* uv, uint32_t* idx,
+                      uint64_t* stats, uint32_t* ctr, uint32_t n_cu, hipStream_t st)
 {
     if (n == 0)
         return hipSuccess;
     auto* sp = reinterpret_cast<unsigned long long*>(stats);
+    const SearchGrid g = search_grid(n, 64, RayLds::WORDS, n_cu, 6, ctr != nullptr, t.n_dev != nullptr);
+    uint32_t* c = g.persist ? ctr : nullptr;
+    if (c)
+        hipLaunchKernelGGL(k_clear_chunks, dim3(1), dim3(64), 0, st, c);
+#define SNCH_RAY(S_, A_)                                                                                             \
+    hipLaunchKernelGGL((k_ray<S_, DIM, A_>), g.grid, g.block, 0, st, t, V, F, o, d, tmax, n, g.qpw, hit, tout, uv, idx, \
+                       c, traversal_error_word(), sp)
     SNCH_DISPATCH_DIM(dim, {
-        if (stats)
-            hipLaunchKernelGGL((k_ray<256, true, DIM>), dim3(nblocks(n, 256)), dim3(256), 0, st, t, o, d, tmax, n,
-                               any_hit, hit, tout, uv, idx, traversal_error_word(), sp);
-        else
-            hipLaunchKernelGGL((k_ray<256, false, DIM>), dim3(nblocks(n, 256)), dim3(256), 0, st, t, o, d, tmax, n,
-                               any_hit, hit, tout, uv, idx, traversal_error_word(), sp);
+        if (any_hit) {
+            if (stats)
+                SNCH_RAY(true, true);
+            else
+                SNCH_RAY(false, true);
+        } else if (stats) {
+            SNCH_RAY(true, false);
+        } else {
+            SNCH_RAY(false, false);
+        }
     });
+#undef SNCH_RAY
     return hipGetLastError();
 }
 

@@ -68,7 +68,7 @@ hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q,
     if (!err)
         err = traversal_error_word();
     const bool hard = seed && capped;
-    const SearchGrid g = search_grid(n, block, depth, hard, n_cu, 6, ctr != nullptr, t.n_dev != nullptr);
+    const SearchGrid g = search_grid(n, block, wave_lds_words(pool_cap(depth), hard), n_cu, 6, ctr != nullptr, t.n_dev != nullptr);
     uint32_t* c = g.persist ? ctr : nullptr;
     if (c)
         hipLaunchKernelGGL(k_clear_sil_chunks, dim3(1), dim3(64), 0, st, c);

@@ -1,6 +1,6 @@
 // Searches shared by the query kernels (query.hip, silhouette.hip, batch.hip):
-// the restart-trail stack, closest point and closest silhouette for the lanes
-// of a wave, and the chunks of a persistent launch.  Device code.
+// closest point, closest silhouette and rays of a wave from one pool of pending
+// nodes, and the chunks of a persistent launch.  Device code.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -13,7 +13,6 @@ namespace snch {
 
 namespace {
 
-constexpr int SS = 16; // LDS stack entries per lane (rays)
 constexpr uint32_t LDS_PER_CU = 160 * 1024;
 
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb)
@@ -24,133 +23,6 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t nb)
 
 // wave-uniform copy of lane 0's value (a scalar register)
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-
-// A short stack with a restart trail (Laine 2010, "Restart trail for
-// stackless BVH traversal"), for searches whose pruning bound only tightens:
-// SSZ 4-B entries in a circular LDS column, and nothing in private memory.
-// An entry is node << 8 | q for trees of at most 2^24 leaves (internal node
-// ids < 2^24); q is an 8-bit lower bound of the key (a non-negative squared
-// distance): the key's float bits >> 20 (exponent and 3 mantissa bits, the
-// key truncated to 8 steps per octave) minus a base chosen per tree so that
-// the 255 levels span 31 octaves below the squared scene diagonal; keys
-// below that range store 0 (decoded as 0), keys above saturate at 255, so
-// the decoded value never exceeds the key and a popped entry is never
-// skipped wrongly.  A push onto a full stack overwrites the oldest
-// entry (the shallowest level); the lost far children are found again
-// through the trail and revisited from the root.  Per lane, one bit per tree
-// level (root 0; a path holds at most 64 internal nodes):
-//   T  at this level the near child is finished and the far child taken;
-//   S  at this level only one child was descended (nothing left behind);
-//   M  the levels whose far child sits in the stack (levels grow from the
-//      stack's bottom to its top, so the top entry's level is M's highest).
-// A level of the current path with neither T nor S set, and not in M, left
-// its far child behind; when the stack runs empty the deepest such level j
-// gets T and the search restarts from the root: levels above j follow the
-// trail (T: far child; else near, re-pushing a surviving far child), and
-// level j takes its far child.  Children survive only if they pass the
-// pruning tests, which can only fail more often as the bound tightens, so a
-// subtree left by the trail holds nothing new.
-template <int BS, int SSZ>
-struct TrailStack {
-    uint32_t* lds;
-    uint32_t top; // position of the next push (mod SSZ)
-    uint32_t qbase;
-    uint64_t T, S, M;
-    uint32_t lv; // level of the current node
-
-    __device__ __forceinline__ void init(uint32_t* base, uint32_t qb)
-    {
-        lds = base;
-        qbase = qb;
-        reset();
-    }
-    __device__ __forceinline__ void reset()
-    {
-        top = 0;
-        T = S = M = 0ull;
-        lv = 0;
-    }
-    __device__ __forceinline__ uint32_t enc(uint32_t n, float d) const
-    {
-        const uint32_t v = __float_as_uint(d) >> 20;
-        const uint32_t q = v > qbase ? min(v - qbase, 255u) : 0u;
-        return (n << 8) | q;
-    }
-    // the lower bound stored in an entry
-    __device__ __forceinline__ float key(uint32_t e) const
-    {
-        const uint32_t q = e & 255u;
-        return q ? __uint_as_float((q + qbase) << 20) : 0.0f;
-    }
-    __device__ __forceinline__ void push(uint32_t n, float d, uint32_t k)
-    {
-        lds[(top % SSZ) * BS] = enc(n, d);
-        ++top;
-        if (__popcll(M) >= SSZ)
-            M &= M - 1ull; // the oldest entry was just overwritten
-        M |= 1ull << k;
-    }
-    // pop the top entry (M != 0): its node and decoded key; the current
-    // path ends at its level, whose near child is finished
-    __device__ __forceinline__ void pop(uint32_t& n, float& d)
-    {
-        --top;
-        const uint32_t e = lds[(top % SSZ) * BS];
-        n = e >> 8;
-        d = key(e);
-        const uint32_t k = 63u - (uint32_t)__clzll(M);
-        const uint64_t kb = 1ull << k;
-        M &= ~kb;
-        T = (T & (kb - 1ull)) | kb;
-        S &= kb - 1ull;
-        lv = k;
-    }
-    // the stack is empty: restart from the root for the deepest level of the
-    // current path that left its far child behind; false when there is none
-    __device__ __forceinline__ bool restart()
-    {
-        const uint64_t path = lv >= 63u ? ~1ull : ((2ull << lv) - 1ull) & ~1ull; // levels 1..lv
-        const uint64_t Z = ~(T | S) & path;
-        if (!Z)
-            return false;
-        const uint32_t j = 63u - (uint32_t)__clzll(Z);
-        const uint64_t jb = 1ull << j;
-        T = (T & (jb - 1ull)) | jb;
-        S &= jb - 1ull;
-        top = 0;
-        lv = 0;
-        return true;
-    }
-    // choose the child to descend from the current node (children at level
-    // lv + 1), given which of the near (N) and far (F) children survive;
-    // false: nothing to descend
-    __device__ __forceinline__ bool descend(bool gN, bool gF, uint32_t nN, uint32_t nF, float dF, uint32_t& node)
-    {
-        if (!gN && !gF)
-            return false;
-        const uint32_t k = lv + 1u; // at most 63: the caller stops deeper paths
-        const uint64_t kb = 1ull << k;
-        if (T & kb) { // near finished before: the far child, if it survives
-            if (!gF)
-                return false;
-            node = nF;
-        } else if (gN && gF) {
-            push(nF, dF, k);
-            node = nN;
-        } else if (gN) {
-            S |= kb;
-            node = nN;
-        } else if (gF) { // off the trail: the near child no longer survives
-            T = (T & (kb - 1ull)) | kb;
-            S &= kb - 1ull;
-            node = nF;
-        } else {
-            return false;
-        }
-        lv = k;
-        return true;
-    }
-};
 
 // per-query visit counters (Counts), summed over the wave before one atomic per wave
 __device__ __forceinline__ void flush_counts(const Counts& c, unsigned long long* stats)
@@ -310,7 +182,8 @@ __device__ __forceinline__ void list_push(uint32_t* list, uint32_t& size, bool y
 }
 
 // the same for pool items
-__device__ __forceinline__ void pool_push(WaveLds& W, uint32_t& size, bool yes, uint32_t a, float key)
+template <class L>
+__device__ __forceinline__ void pool_push(L& W, uint32_t& size, bool yes, uint32_t a, float key)
 {
     const uint64_t m = __builtin_amdgcn_ballot_w64(yes);
     const uint32_t at = size + rank_in(m);
@@ -321,12 +194,13 @@ __device__ __forceinline__ void pool_push(WaveLds& W, uint32_t& size, bool yes, 
     size += (uint32_t)__popcll(m);
 }
 
-// queries waiting to enter (todo: a slot per bit) into the pool, up to
-// POOL_ADD of them
-__device__ __forceinline__ void pool_feed(WaveLds& W, uint32_t& size, uint64_t& todo)
+// queries waiting to enter (todo: a slot per bit) into the pool, up to `add`
+// of them
+template <class L>
+__device__ __forceinline__ void pool_feed(L& W, uint32_t& size, uint64_t& todo, uint32_t add)
 {
     const uint32_t lane = threadIdx.x & 63;
-    const bool in = ((todo >> lane) & 1ull) && rank_in(todo) < POOL_ADD;
+    const bool in = ((todo >> lane) & 1ull) && rank_in(todo) < add;
     todo &= ~__builtin_amdgcn_ballot_w64(in);
     pool_push(W, size, in, lane << 24, 0.0f);
 }
@@ -450,7 +324,7 @@ __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds&
             break;
         }
         if (size < 32u && todo != 0ull)
-            pool_feed(W, size, todo);
+            pool_feed(W, size, todo, POOL_ADD);
         const uint32_t k = pool_take(size, W.cap), side = lane & 1u;
         size -= k;
         uint32_t slot = 0, ref = 0;
@@ -713,7 +587,7 @@ __device__ __forceinline__ void sil_wave(const TreeView& t, uint64_t all, bool f
             break;
         }
         if (size < 32u && todo != 0ull)
-            pool_feed(W, size, todo);
+            pool_feed(W, size, todo, POOL_ADD);
         const uint32_t k = pool_take(size, W.cap), side = lane & 1u;
         size -= k;
         uint32_t slot = 0, ref = 0;
@@ -764,6 +638,246 @@ __device__ __forceinline__ void sil_wave(const TreeView& t, uint64_t all, bool f
             lane_silhouette<DIM>(t, p, flip, widened<DIM>(HwMath::sqrt(__uint_as_float(W.bound[lane])), p, scale),
                                  MODE == 2 ? W.cap2()[lane] : F_INF, W.pool + 128 * r, d, id);
             W.best[lane] = pack_best(d, id);
+            alone = false;
+        }
+    }
+}
+
+// ------------------------------------------------------------ rays
+
+// LDS of a wave's rays: as WaveLds, with the origin, the reciprocal and the
+// direction per query slot.  A ray visits few nodes (20 on the 1M-triangle
+// torus), so all 64 of a wave enter at once and a smaller pool does.
+constexpr uint32_t RAY_LEAF_RUN = 24, RAY_ADD = 32;
+struct RayLds {
+    unsigned long long* best; // (t, triangle)
+    uint32_t *pool, *leaf, *bound;
+    uint16_t* pkey;
+    float* q; // origin, reciprocal direction, direction: 9 rows of 64
+    uint32_t cap;
+    static constexpr uint32_t CAP = 384;
+    static constexpr uint32_t WORDS = 128 + 2 * LEAF_CAP + 64 + 576 + CAP + CAP / 2;
+    __device__ __forceinline__ explicit RayLds(uint32_t* base)
+    {
+        best = reinterpret_cast<unsigned long long*>(base);
+        leaf = base + 128;
+        bound = leaf + 2 * LEAF_CAP;
+        q = reinterpret_cast<float*>(bound + 64);
+        pool = bound + 640;
+        pkey = reinterpret_cast<uint16_t*>(pool + CAP);
+        cap = CAP;
+    }
+    __device__ __forceinline__ v3 row3(uint32_t r, uint32_t s) const
+    {
+        return mk(q[64 * r + s], q[64 * r + 64 + s], q[64 * r + 128 + s]);
+    }
+    __device__ __forceinline__ v3 origin(uint32_t s) const { return row3(0, s); }
+    __device__ __forceinline__ v3 inv(uint32_t s) const { return row3(3, s); }
+    __device__ __forceinline__ v3 dir(uint32_t s) const { return row3(6, s); }
+    __device__ __forceinline__ void start(uint32_t s, v3 o, v3 d, v3 i, float max_dist)
+    {
+        const v3 a[3] = {o, i, d};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            q[64 * (3 * k) + s] = a[k].x;
+            q[64 * (3 * k + 1) + s] = a[k].y;
+            q[64 * (3 * k + 2) + s] = a[k].z;
+        }
+        best[s] = pack_best(F_INF, INVALID);
+        bound[s] = __float_as_uint(max_dist);
+    }
+};
+static_assert(RayLds::WORDS % 2 == 0, "8-byte aligned answers");
+
+// the scene's hit test of the leaf at sorted position j: t, (u, v) and the original index
+template <int DIM>
+__device__ __forceinline__ bool ray_leaf(const TreeView& t, uint32_t j, v3 ro, v3 rd, float& th, float& uh, float& vh,
+                                         uint32_t& id)
+{
+    if (j >= t.n_leaves)
+        return false;
+    const float4 a = t.tleaf[3 * j], b = t.tleaf[3 * j + 1];
+    id = __float_as_uint(a.w);
+    vh = 0.0f;
+    if (DIM == 3) {
+        const float4 c = t.tleaf[3 * j + 2];
+        return ray_triangle(ro, rd, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), mk(c.x, c.y, c.z), th, uh, vh);
+    }
+    return ray_segment(ro, rd, mk(a.x, a.y, 0.0f), mk(b.x, b.y, 0.0f), th, uh);
+}
+
+// query_device(ray_intersect) (query.cuh:79-169) by one lane: near child
+// first, a node's leaves at once in that order.  st: 128 words of LDS.
+template <int DIM>
+__device__ inline void lane_ray(const TreeView& t, v3 ro, v3 rd, v3 inv, float max_dist, uint32_t* st, float& tbest,
+                                uint32_t& bidx)
+{
+    tbest = F_INF;
+    bidx = INVALID;
+    auto leaf = [&](uint32_t j) {
+        float th, uh, vh;
+        uint32_t id;
+        if (ray_leaf<DIM>(t, j, ro, rd, th, uh, vh, id) && th < max_dist && (th < tbest || (th == tbest && id < bidx))) {
+            tbest = th;
+            bidx = id;
+        }
+    };
+    uint32_t sp = 0, node = 0;
+    for (uint32_t it = 0; it < 2 * t.n_leaves + 64 && node < t.n_leaves - 1; ++it) {
+        const NodeRec nr = load_node(t.tnode, node);
+        float Ld = F_INF, Rd = F_INF;
+        const bool bL = box_ray(nr.L, ro, inv, max_dist, Ld), bR = box_ray(nr.R, ro, inv, max_dist, Rd);
+        const bool Lh = bL && Ld <= tbest, Rh = bR && Rd <= tbest;
+        uint32_t lf, lc, rf, rc;
+        const bool lLeaf = as_leaf(nr.lref, 0u, lf, lc), rLeaf = as_leaf(nr.rref, 1u, rf, rc);
+        const bool rfirst = Lh && Rh && Rd < Ld; // nearer child first, as query.cuh:136-149
+        if (rfirst) {
+            if (Rh && rLeaf)
+                for (uint32_t k = 0; k < rc; ++k)
+                    leaf(rf + k);
+            if (Lh && lLeaf && Ld <= tbest)
+                for (uint32_t k = 0; k < lc; ++k)
+                    leaf(lf + k);
+        } else {
+            if (Lh && lLeaf)
+                for (uint32_t k = 0; k < lc; ++k)
+                    leaf(lf + k);
+            if (Rh && rLeaf && Rd <= tbest)
+                for (uint32_t k = 0; k < rc; ++k)
+                    leaf(rf + k);
+        }
+        const bool gL = Lh && !lLeaf && Ld <= tbest, gR = Rh && !rLeaf && Rd <= tbest;
+        const bool lnear = bL && (!bR || !(Rd < Ld));
+        if (gL && gR && sp < 64u) {
+            st[2 * sp] = lnear ? nr.rref : nr.lref;
+            st[2 * sp + 1] = __float_as_uint(lnear ? Rd : Ld);
+            ++sp;
+        }
+        if (gL || gR) {
+            node = gL && (lnear || !gR) ? nr.lref : nr.rref;
+            continue;
+        }
+        bool found = false;
+        while (sp > 0 && !found) {
+            --sp;
+            node = st[2 * sp];
+            found = __uint_as_float(st[2 * sp + 1]) <= tbest; // query.cuh:106
+        }
+        if (!found)
+            break;
+    }
+}
+
+// tests the last (up to 64) leaves of the wave's buffer; returns how many are
+// left.  A hit at t becomes a candidate of its ray, whose bound falls to a
+// little more than t (the rounding of box and triangle parameters: see the
+// hidden leaves above); any hit ends the ray with ANY.
+template <bool STATS, int DIM, bool ANY>
+__device__ __forceinline__ uint32_t ray_leaves(const TreeView& t, RayLds& W, uint32_t nleaf, float scale, Counts& cnt)
+{
+    const uint32_t lane = threadIdx.x & 63, k = min(64u, nleaf);
+    nleaf -= k;
+    if (lane < k) {
+        const uint32_t w = W.leaf[2 * (nleaf + lane)], slot = w >> 24;
+        const float key = __uint_as_float(W.leaf[2 * (nleaf + lane) + 1]), b = __uint_as_float(W.bound[slot]);
+        if (key <= b) {
+            if (STATS)
+                cnt.leaf += 1;
+            const v3 o = W.origin(slot);
+            float th, uh, vh;
+            uint32_t id;
+            if (ray_leaf<DIM>(t, w & REF_MASK, o, W.dir(slot), th, uh, vh, id) && th < b) {
+                th += 0.0f; // -0 counts as 0
+                atomicMin(&W.best[slot], pack_best(th, id, key > th));
+                if (ANY)
+                    W.bound[slot] = 0x7FC00000u; // NaN: no key is below it
+                else
+                    atomicMin(&W.bound[slot],
+                              __float_as_uint(th * 1.0001f +
+                                              1e-5f * fmx(scale, fmx(dm::fabs_(o.x),
+                                                                     fmx(dm::fabs_(o.y), dm::fabs_(o.z))))));
+            }
+        }
+    }
+    return nleaf;
+}
+
+// query_device(ray_intersect) (query.cuh:79-169) for the rays of a wave, a
+// slot per bit of `all` (RayLds::start): W.best receives (t, triangle).  Run
+// by the whole wave.  A ray with a negative or NaN max_dist hits nothing.
+template <bool STATS, int DIM, bool ANY>
+__device__ __forceinline__ void ray_wave(const TreeView& t, uint64_t all, float max_dist, RayLds& W, Counts& cnt,
+                                         bool& overflow)
+{
+    const uint32_t lane = threadIdx.x & 63, side = lane & 1u;
+    const bool valid = ((all >> lane) & 1ull) && max_dist >= 0.0f;
+    uint64_t todo = __builtin_amdgcn_ballot_w64(valid);
+    uint32_t size = 0, nleaf = 0;
+    const float scale = scene_scale(t);
+    if (t.n_leaves == 1) { // the only leaf is tested without its box, as in the reference
+        list_push(W.leaf, nleaf, valid && lane < 32u, lane << 24, 0.0f);
+        if (nleaf)
+            nleaf = ray_leaves<STATS, DIM, ANY>(t, W, nleaf, scale, cnt);
+        list_push(W.leaf, nleaf, valid && lane >= 32u, lane << 24, 0.0f);
+        todo = 0ull;
+    }
+    const uint32_t cap_iters = 128u * t.n_leaves + 65536u;
+    for (uint32_t it = 0;; ++it) {
+        if (nleaf >= RAY_LEAF_RUN || (nleaf > 0u && todo == 0ull && size < 32u)) {
+            nleaf = ray_leaves<STATS, DIM, ANY>(t, W, nleaf, scale, cnt);
+            continue;
+        }
+        if (size == 0u && todo == 0ull)
+            break;
+        if (it >= cap_iters) {
+            overflow = true;
+            break;
+        }
+        if (size < 32u && todo != 0ull)
+            pool_feed(W, size, todo, RAY_ADD);
+        const uint32_t k = pool_take(size, W.cap);
+        size -= k;
+        uint32_t slot = 0, ref = 0;
+        float dist = F_INF;
+        bool go = false;
+        if ((lane >> 1) < k) {
+            const uint32_t at = size + (lane >> 1), w = W.pool[at], node = w & REF_MASK;
+            slot = w >> 24;
+            const float b = __uint_as_float(W.bound[slot]);
+            if (__uint_as_float((uint32_t)W.pkey[at] << 16) <= b && node < t.n_leaves - 1) {
+                const ChildRec c = load_child(t.tnode, node, side);
+                ref = c.ref;
+                go = box_ray(c.box, W.origin(slot), W.inv(slot), b, dist);
+                if (STATS) {
+                    cnt.node += side;
+                    cnt.box += 1;
+                }
+            }
+        }
+        dist = go ? dist : F_INF;
+        uint32_t first, count;
+        const bool leaf = as_leaf(ref, side, first, count);
+        const float other = pair_other(dist);
+        const bool lt = dist < other, eq = dist == other, near = lt || (eq && !side);
+        pool_push(W, size, go && !leaf && !near, (slot << 24) | (ref & REF_MASK), dist);
+        pool_push(W, size, go && !leaf && near, (slot << 24) | (ref & REF_MASK), dist);
+        list_push(W.leaf, nleaf, go && leaf, (slot << 24) | first, dist);
+        for (uint32_t j = 1; (t.flags & TREE_RUNS) && __ballot(go && leaf && j < count); ++j) {
+            if (nleaf >= LEAF_RUN)
+                nleaf = ray_leaves<STATS, DIM, ANY>(t, W, nleaf, scale, cnt);
+            list_push(W.leaf, nleaf, go && leaf && j < count, (slot << 24) | (first + j), dist);
+        }
+    }
+    if (ANY || t.n_leaves == 1)
+        return;
+    float d = F_INF;
+    uint32_t id = INVALID;
+    bool alone = valid && unpack_best(W.best[lane], d, id);
+    for (uint64_t left = __ballot(alone); left; left = __ballot(alone)) {
+        const uint32_t r = rank_in(left);
+        if (alone && r < W.cap / 128u) {
+            lane_ray<DIM>(t, W.origin(lane), W.dir(lane), W.inv(lane), max_dist, W.pool + 128 * r, d, id);
+            W.best[lane] = pack_best(d + 0.0f, id);
             alone = false;
         }
     }
@@ -830,19 +944,19 @@ __device__ __forceinline__ void for_chunks(uint32_t n, uint32_t qpw, uint32_t* c
 inline uint32_t nblocks(uint32_t n, uint32_t bs) { return (n + bs - 1) / bs; }
 
 // grid of a search launch: a wave per chunk, or (persist) as many waves as
-// are resident (lds bytes of LDS and at most `per_simd` waves on a SIMD)
+// are resident (wave_words words of LDS each, at most `per_simd` on a SIMD)
 struct SearchGrid {
     dim3 grid, block;
     uint32_t qpw;
     size_t lds;
     bool persist;
 };
-inline SearchGrid search_grid(uint32_t n, uint32_t block, uint32_t depth, bool capped, uint32_t n_cu,
-                              uint32_t per_simd, bool may_persist, bool n_on_device)
+inline SearchGrid search_grid(uint32_t n, uint32_t block, uint32_t wave_words, uint32_t n_cu, uint32_t per_simd,
+                              bool may_persist, bool n_on_device)
 {
     SearchGrid g;
     const uint32_t wpb = block / 64;
-    g.lds = sizeof(uint32_t) * wpb * wave_lds_words(pool_cap(depth), capped);
+    g.lds = sizeof(uint32_t) * wpb * wave_words;
     const uint32_t per_cu = std::max(1u, std::min((uint32_t)(LDS_PER_CU / g.lds), per_simd * 4u / wpb));
     const uint32_t resident = n_cu * per_cu;
     g.qpw = n_on_device ? 0u : queries_per_wave(n, resident * wpb); // 0: from the count on the device

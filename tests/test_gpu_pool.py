@@ -79,7 +79,7 @@ def test_closest_silhouette_does_not_depend_on_the_launch(name, leaf_size):
             np.testing.assert_array_equal(e1, e0)
         # hints too small, about right, too large, zero and none
         r = np.random.default_rng(3)
-        seed = np.where(np.isfinite(d0), d0, 1.0) * r.choice([0.0, 0.5, 1.0, 1.25, np.inf], len(d0))
+        seed = np.where(np.isfinite(d0), d0, 1.0) * r.choice([0.0, 0.5, 1.0, 1.25, 1e30], len(d0))
         for n in (65, len(q)):
             e1, d1 = np_(sc.closest_silhouette(q[:n], flip=flip, seed_radius=seed[:n].astype(np.float32)))
             np.testing.assert_array_equal(d1, d0[:n])
@@ -91,3 +91,32 @@ def test_closest_silhouette_does_not_depend_on_the_launch(name, leaf_size):
         np.testing.assert_array_equal(d1[within], d0[within])
         np.testing.assert_array_equal(e1[within], e0[within])
         assert np.all(d1[~within] > cap[~within])
+
+
+@pytest.mark.parametrize("name", ["ico", "ico_far", "box_far", "two"])
+@pytest.mark.parametrize("leaf_size", [1, 8])
+def test_rays_do_not_depend_on_the_launch(name, leaf_size):
+    import oracle
+    import snch_lbvh_amd as S
+    from snch_lbvh_amd import workloads as W
+
+    V, F = _meshes()[name]
+    n = 70000
+    o, d = _points(V, n, 13), W.unit_directions(n, 14)
+    d[::7] = np.eye(3, dtype=np.float32)[np.arange(len(d[::7])) % 3]  # along the axes: infinite reciprocals
+    r = np.random.default_rng(4)
+    tmax = r.choice(np.float32([np.inf, 0.5, 0.0, -1.0, np.nan]), n, p=[0.5, 0.3, 0.1, 0.05, 0.05])
+    sc = S.Scene(V, F).build_bvh(leaf_size=leaf_size)
+    for tm in (None, tmax):
+        cut = lambda k: None if tm is None else tm[:k]  # noqa: E731
+        full = [x.cpu().numpy() for x in sc.ray_intersect(o, d, cut(n))]
+        for k in (1, 2, 31, 32, 33, 64, 65, 1000):
+            part = [x.cpu().numpy() for x in sc.ray_intersect(o[:k], d[:k], cut(k))]
+            for a, b in zip(part, full):
+                np.testing.assert_array_equal(a, b[:k])
+            any_hit = sc.ray_intersect(o[:k], d[:k], cut(k), any_hit=True)[0].cpu().numpy()
+            np.testing.assert_array_equal(any_hit, full[0][:k])
+        if leaf_size == 1:  # the oracle visits a node's children in the same order
+            hit, t = oracle.ray(oracle.build_tree(V, F), o[:4000], d[:4000], cut(4000))[:2]
+            np.testing.assert_array_equal(full[0][:4000], hit.astype(bool))
+            np.testing.assert_array_equal(full[1][:4000], t)
