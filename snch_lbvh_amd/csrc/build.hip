@@ -297,9 +297,11 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
     b.lo = mk(F_INF, F_INF, F_INF);
     b.hi = mk(-F_INF, -F_INF, -F_INF);
     uint32_t e0 = 0, my = 0;
-    v3 c = mk(0.0f, 0.0f, 0.0f);
+    v3 c = mk(0.0f, 0.0f, 0.0f), p0 = c, p1 = c, p2 = c;
     if (i < nF) {
-        const v3 p0 = ld3(V, F[3 * i]), p1 = ld3(V, F[3 * i + 1]), p2 = ld3(V, F[3 * i + 2]);
+        p0 = ld3(V, F[3 * i]);
+        p1 = ld3(V, F[3 * i + 1]);
+        p2 = ld3(V, F[3 * i + 2]);
         b = box_of_point(p0);
         box_expand(b, p1);
         box_expand(b, p2);
@@ -320,6 +322,7 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
     r.axis = mk(0.0f, 0.0f, 0.0f);
     r.half_angle = F_PI;
     r.radius = 0.0f;
+    uint32_t slab = SLAB_ALL;
     bool all_two = true;
     v3 nn[3][2];
 #pragma unroll
@@ -428,12 +431,17 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
                         cmin = smin(cmin, clamp11(dot3(r.axis, nn[k][jj])));
                 }
                 r.half_angle = smax(0.0f, dm::acosf_(cmin));
+                // the owned edges end in the triangle's vertices
+                const float h0 = dot3(r.axis, sub(p0, c)), h1 = dot3(r.axis, sub(p1, c)), h2 = dot3(r.axis, sub(p2, c));
+                const float m = smax(smax(dm::fabs_(c.x), dm::fabs_(c.y)), dm::fabs_(c.z)) + r.radius;
+                if (conservative)
+                    slab = pack_slab(fmn(h0, fmn(h1, h2)), fmx(h0, fmx(h1, h2)), r.radius, 1e-6f * m);
             }
         }
-        // the leaf record: box and cone in three float4 (no padding lanes)
+        // the leaf record: box and cone in three float4
         leafrec[3 * i] = make_float4(b.lo.x, b.lo.y, b.lo.z, b.hi.x);
         leafrec[3 * i + 1] = make_float4(b.hi.y, b.hi.z, r.axis.x, r.axis.y);
-        leafrec[3 * i + 2] = make_float4(r.axis.z, r.half_angle, r.radius, 0.0f);
+        leafrec[3 * i + 2] = make_float4(r.axis.z, r.half_angle, r.radius, __uint_as_float(slab));
     }
     // scene AABB of the primitive's mesh
     float v[6] = {b.lo.x, b.lo.y, b.lo.z, b.hi.x, b.hi.y, b.hi.z};
@@ -836,13 +844,15 @@ __device__ __forceinline__ box3 ldbox(const float4* nb, uint32_t n)
     b.hi = mk(c.x, c.y, c.z);
     return b;
 }
-__device__ __forceinline__ cone3 ldcone(const float4* nc, uint32_t n)
+// a cone and its slab
+__device__ __forceinline__ cone3 ldcone(const float4* nc, uint32_t n, uint32_t& slab)
 {
     const float4 a = nc[2 * n], c = nc[2 * n + 1];
     cone3 r;
     r.axis = mk(a.x, a.y, a.z);
     r.half_angle = a.w;
     r.radius = c.x;
+    slab = __float_as_uint(c.y);
     return r;
 }
 
@@ -895,19 +905,24 @@ __device__ __forceinline__ uint32_t child_ref(const MeshIds& id, uint32_t node, 
 // of internal node p
 template <int DIM>
 __device__ __forceinline__ void refit_write(const MeshIds& id, uint32_t p, uint2 ch, const box3& lb, const box3& rb,
-                                            const cone3& lc, const cone3& rc, int conservative,
+                                            const cone3& lc, const cone3& rc, uint32_t ls, uint32_t rs, int conservative,
                                             const uint2* __restrict__ range, uint32_t leaf_size, box3& pb,
-                                            cone3& pc, float4* nbox, float4* ncone, float4* __restrict__ tnode,
+                                            cone3& pc, uint32_t& ps, float4* nbox, float4* ncone, float4* __restrict__ tnode,
                                             float4* __restrict__ tcone, bool own = true)
 {
     pb = box_merge(lb, rb);
     pc = DIM == 3 ? cone_merge(lc, rc, box_centroid(lb), box_centroid(rb), box_centroid(pb), conservative != 0)
                   : cone_merge2d(lc, rc, box_centroid(lb), box_centroid(rb), box_centroid(pb), conservative != 0);
+    // 16 us of the 1M-triangle build's 150 in k_refit; wide cones, which are
+    // most of the levels above the cuts, are left out (5 us)
+    ps = SLAB_ALL;
+    if (DIM == 3 && conservative && pc.half_angle < SLAB_MAX_ANGLE)
+        ps = slab_merge(pc, pb, lc, ls, lb, rc, rs, rb);
     if (own) { // the node's own box and cone in the reference layout (else they live in its parent's record)
         nbox[2 * p] = make_float4(pb.lo.x, pb.lo.y, pb.lo.z, 0.0f);
         nbox[2 * p + 1] = make_float4(pb.hi.x, pb.hi.y, pb.hi.z, 0.0f);
         ncone[2 * p] = make_float4(pc.axis.x, pc.axis.y, pc.axis.z, pc.half_angle);
-        ncone[2 * p + 1] = make_float4(pc.radius, 0.0f, 0.0f, 0.0f);
+        ncone[2 * p + 1] = make_float4(pc.radius, __uint_as_float(ps), 0.0f, 0.0f);
     }
     const uint32_t r = p - id.off; // internal record: (off - m) + (p - nb)
     tnode[4 * r + 0] = make_float4(lb.lo.x, lb.lo.y, lb.lo.z, lb.hi.x);
@@ -918,8 +933,8 @@ __device__ __forceinline__ void refit_write(const MeshIds& id, uint32_t p, uint2
     tcone[4 * r + 2] = make_float4(rc.axis.x, rc.axis.y, rc.axis.z, rc.half_angle);
     // the sines and cosines (the halves before these) are filled by
     // tcone_trig once the merges are done: off the chain of dependent merges
-    reinterpret_cast<float2*>(tcone)[8 * r + 3] = make_float2(lc.radius, 0.0f);
-    reinterpret_cast<float2*>(tcone)[8 * r + 7] = make_float2(rc.radius, 0.0f);
+    reinterpret_cast<float2*>(tcone)[8 * r + 3] = make_float2(lc.radius, __uint_as_float(ls));
+    reinterpret_cast<float2*>(tcone)[8 * r + 7] = make_float2(rc.radius, __uint_as_float(rs));
 }
 
 // sin and cos of both children's half angles of internal record r, read
@@ -1029,7 +1044,7 @@ __device__ __forceinline__ void collect_mid_members(uint32_t k0, uint32_t stride
 }
 
 template <int DIM>
-__global__ __launch_bounds__(RB) void k_refit(const float4* __restrict__ V, const int32_t* __restrict__ F,
+__global__ __launch_bounds__(RB, 6) void k_refit(const float4* __restrict__ V, const int32_t* __restrict__ F,
                                               const uint32_t* __restrict__ estart,
                                               const uint32_t* __restrict__ sidx, const float4* __restrict__ leafrec,
                                               const uint32_t* __restrict__ parent,
@@ -1040,7 +1055,8 @@ __global__ __launch_bounds__(RB) void k_refit(const float4* __restrict__ V, cons
                                               float4* __restrict__ tleaf, uint32_t* __restrict__ cuts,
                                               uint32_t cut_cap, const uint32_t* __restrict__ midtops,
                                               uint32_t midtop_cap, uint32_t* __restrict__ mids, uint32_t mid_cap,
-                                              uint32_t* __restrict__ members, const uint32_t* __restrict__ flags)
+                                              uint32_t* __restrict__ members, const uint32_t* __restrict__ flags,
+                                              uint32_t* slabs)
 {
     static_assert(RT == 1024, "10-bit local positions");
     collect_mid_members(blockIdx.x * RB + threadIdx.x, gridDim.x * RB, midtops, midtop_cap, parent, range, flags,
@@ -1053,6 +1069,9 @@ __global__ __launch_bounds__(RB) void k_refit(const float4* __restrict__ V, cons
     __shared__ uint16_t queue[RT];
     __shared__ RoundQueue rq;
     __shared__ uint32_t s_cut;
+    // The slabs of the live nodes stay in memory (slabs[first + slot]): a
+    // twelfth row of nd would leave two workgroups per CU (k_refit 199 us at
+    // 1M triangles with cuts of 960 leaves instead, 165 this way)
     const uint32_t t = threadIdx.x;
     const uint32_t count = min(cuts[cut_cap], cut_cap);
     if (t < 3)
@@ -1117,7 +1136,7 @@ __global__ __launch_bounds__(RB) void k_refit(const float4* __restrict__ V, cons
             const uint32_t node = D.nb + (D.n - 1) + (j - D.off);
             const float4 r0 = leafrec[3 * orig], r1 = leafrec[3 * orig + 1], r2 = leafrec[3 * orig + 2];
             const float4 b0 = make_float4(r0.x, r0.y, r0.z, 0.0f), b1 = make_float4(r0.w, r1.x, r1.y, 0.0f);
-            const float4 c0 = make_float4(r1.z, r1.w, r2.x, r2.y), c1 = make_float4(r2.z, 0.0f, 0.0f, 0.0f);
+            const float4 c0 = make_float4(r1.z, r1.w, r2.x, r2.y), c1 = make_float4(r2.z, r2.w, 0.0f, 0.0f);
             if (node == root) { // a cut of one leaf; other leaves live in their parents' records
                 nbox[2 * node] = b0;
                 nbox[2 * node + 1] = b1;
@@ -1132,6 +1151,7 @@ __global__ __launch_bounds__(RB) void k_refit(const float4* __restrict__ V, cons
                 cc.axis = mk(c0.x, c0.y, c0.z);
                 cc.half_angle = c0.w;
                 cc.radius = c1.x;
+                slabs[j] = __float_as_uint(r2.w);
                 nd.put(u, b, cc);
             }
             const uint32_t es = estart[orig], ec = estart[orig + 1] - es;
@@ -1161,12 +1181,16 @@ __global__ __launch_bounds__(RB) void k_refit(const float4* __restrict__ V, cons
                 const uint2 ch = make_uint2(cut_child_global(id, lc, first), cut_child_global(id, rc, first));
                 box3 lb, rb, pb;
                 cone3 lc3, rc3, pc;
+                // the children's slabs, read while the boxes and cones merge
+                const uint32_t lsl = slabs[first + ls], rsl = slabs[first + rs];
+                uint32_t psl;
                 nd.get(ls, lb, lc3);
                 nd.get(rs, rb, rc3);
                 const uint32_t p = D.nb + (first + k - D.off);
-                refit_write<DIM>(id, p, ch, lb, rb, lc3, rc3, conservative, range, leaf_size, pb, pc, nbox, ncone,
-                                 tnode, tcone, p == root);
+                refit_write<DIM>(id, p, ch, lb, rb, lc3, rc3, lsl, rsl, conservative, range, leaf_size, pb, pc, psl,
+                                 nbox, ncone, tnode, tcone, p == root);
                 nd.put(ls, pb, pc);
+                slabs[first + ls] = psl;
                 const uint32_t kp = lpar[k];
                 if (kp != NO_PARENT && (atomicOr(&larr[kp >> 5], 1u << (kp & 31u)) >> (kp & 31u)) & 1u)
                     rq.push(queue, qe, round, kp);
@@ -1212,7 +1236,7 @@ constexpr uint32_t NO_MEMBER = 0xFFFFu;
 constexpr uint32_t SET_ROUNDS = 128;      // a set is at most 64 levels deep
 static_assert(RM / (RT + 1) * 64 <= MID_CAP, "mid-set bound");
 
-// LDS arrays of a set, `cap` entries each (box: 11 rows, boxes in LDS only)
+// LDS arrays of a set, `cap` entries each (box: 12 rows, boxes in LDS only)
 struct SetLds {
     uint32_t* node;  // member's node id
     uint2* ch;       // its children's node ids
@@ -1222,17 +1246,19 @@ struct SetLds {
     uint16_t* queue;
     float* box;
     uint32_t cap;
-    __device__ __forceinline__ void put(uint32_t k, const box3& b, const cone3& c) const
+    __device__ __forceinline__ void put(uint32_t k, const box3& b, const cone3& c, uint32_t slab) const
     {
         float* v = box + k;
+        v[11 * cap] = __uint_as_float(slab);
         v[0 * cap] = b.lo.x; v[1 * cap] = b.lo.y; v[2 * cap] = b.lo.z;
         v[3 * cap] = b.hi.x; v[4 * cap] = b.hi.y; v[5 * cap] = b.hi.z;
         v[6 * cap] = c.axis.x; v[7 * cap] = c.axis.y; v[8 * cap] = c.axis.z;
         v[9 * cap] = c.half_angle; v[10 * cap] = c.radius;
     }
-    __device__ __forceinline__ void get(uint32_t k, box3& b, cone3& c) const
+    __device__ __forceinline__ void get(uint32_t k, box3& b, cone3& c, uint32_t& slab) const
     {
         const float* v = box + k;
+        slab = __float_as_uint(v[11 * cap]);
         b.lo = mk(v[0 * cap], v[1 * cap], v[2 * cap]);
         b.hi = mk(v[3 * cap], v[4 * cap], v[5 * cap]);
         c.axis = mk(v[6 * cap], v[7 * cap], v[8 * cap]);
@@ -1302,22 +1328,23 @@ __device__ void refit_set(const SetLds& s, uint32_t n, uint32_t lo_thr, uint32_t
             const MeshIds id{D.off, D.n, D.nb};
             box3 lb, rb, pb;
             cone3 lc, rc, pc;
+            uint32_t lsl, rsl, psl;
             if (BOX_LDS && (ci & 0xFFFFu) != NO_MEMBER) {
-                s.get(min(ci & 0xFFFFu, s.cap - 1), lb, lc);
+                s.get(min(ci & 0xFFFFu, s.cap - 1), lb, lc, lsl);
             } else {
                 lb = ldbox(nbox, ch.x);
-                lc = ldcone(ncone, ch.x);
+                lc = ldcone(ncone, ch.x, lsl);
             }
             if (BOX_LDS && (ci >> 16) != NO_MEMBER) {
-                s.get(min(ci >> 16, s.cap - 1), rb, rc);
+                s.get(min(ci >> 16, s.cap - 1), rb, rc, rsl);
             } else {
                 rb = ldbox(nbox, ch.y);
-                rc = ldcone(ncone, ch.y);
+                rc = ldcone(ncone, ch.y, rsl);
             }
-            refit_write<DIM>(id, p, ch, lb, rb, lc, rc, conservative, range, leaf_size, pb, pc, nbox, ncone, tnode,
-                             tcone);
+            refit_write<DIM>(id, p, ch, lb, rb, lc, rc, lsl, rsl, conservative, range, leaf_size, pb, pc, psl, nbox,
+                             ncone, tnode, tcone);
             if (BOX_LDS)
-                s.put(k, pb, pc);
+                s.put(k, pb, pc, psl);
             const uint32_t pk = s.word[k] >> 16;
             if (pk < n && (atomicSub(&s.word[pk], 1u) & 0xFFFFu) == 1u)
                 push(qe, round, pk);
@@ -1345,7 +1372,7 @@ __global__ __launch_bounds__(MB) void k_refit_mid(const uint32_t* __restrict__ p
     __shared__ uint32_t node[MID_CAP], cidx[MID_CAP], word[MID_CAP], mesh[MID_CAP];
     __shared__ uint2 ch[MID_CAP];
     __shared__ uint16_t queue[MID_CAP];
-    __shared__ float box[11 * MID_CAP];
+    __shared__ float box[12 * MID_CAP];
     __shared__ RoundQueue rq;
     const SetLds s{node, ch, cidx, word, mesh, queue, box, MID_CAP};
     const uint32_t t = threadIdx.x;
@@ -1375,7 +1402,7 @@ __global__ __launch_bounds__(MB) void k_refit_mid(const uint32_t* __restrict__ p
 constexpr uint32_t TOP_BOX = 2048;
 constexpr uint32_t TOP_TOPO = 6016;
 constexpr uint32_t TOP_SMEM = TOP_TOPO * 26;
-static_assert(TOP_BOX * (26 + 44) <= TOP_SMEM, "LDS layouts of k_refit_top");
+static_assert(TOP_BOX * (26 + 48) <= TOP_SMEM, "LDS layouts of k_refit_top");
 
 template <int DIM>
 __global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__ parent,
@@ -1402,7 +1429,7 @@ __global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__
         s.word = s.cidx + cap;
         s.mesh = s.word + cap;
         s.box = reinterpret_cast<float*>(s.mesh + cap);
-        s.queue = reinterpret_cast<uint16_t*>(s.box + (boxes ? 11 * cap : 0));
+        s.queue = reinterpret_cast<uint16_t*>(s.box + (boxes ? 12 * cap : 0));
         return s;
     };
     if ((n <= TOP_BOX && force == 0) || (n <= TOP_TOPO && force <= 1)) {
@@ -1443,8 +1470,10 @@ __global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__
             const uint2 ch = child[p];
             box3 pb;
             cone3 pc;
-            refit_write<DIM>(id, p, ch, ldbox(nbox, ch.x), ldbox(nbox, ch.y), ldcone(ncone, ch.x),
-                             ldcone(ncone, ch.y), conservative, range, leaf_size, pb, pc, nbox, ncone, tnode, tcone);
+            uint32_t lsl, rsl, psl;
+            const cone3 lc = ldcone(ncone, ch.x, lsl), rc = ldcone(ncone, ch.y, rsl);
+            refit_write<DIM>(id, p, ch, ldbox(nbox, ch.x), ldbox(nbox, ch.y), lc, rc, lsl, rsl, conservative, range,
+                             leaf_size, pb, pc, psl, nbox, ncone, tnode, tcone);
             const uint32_t par = parent[p];
             if (par == INVALID || !id.internal(par))
                 break;
@@ -1496,6 +1525,7 @@ hipError_t build_tree(snch_scene* s, uint32_t flags, uint32_t leaf_size, hipStre
             return e;            \
     } while (0)
     SNCH_TRY(w.leafbox.ensure(sizeof(float4) * 3 * N)); // the leaf records (box + cone)
+    SNCH_TRY(w.slabs.ensure(sizeof(uint32_t) * N)); // slab of the live node in each slot (k_refit)
     SNCH_TRY(w.scene_bits.ensure(sizeof(int) * 8 * M));
     SNCH_TRY(w.boxpart.ensure(sizeof(float) * 8 * blocks(N)));
     SNCH_TRY(w.codes.ensure(sizeof(uint32_t) * N));
@@ -1592,7 +1622,8 @@ hipError_t build_tree(snch_scene* s, uint32_t flags, uint32_t leaf_size, hipStre
                            w.parent.as<uint32_t>(), w.child.as<uint2>(), w.range.as<uint2>(),
                            desc, M, N, conservative, leaf_size, s->nbox.as<float4>(), s->ncone.as<float4>(),
                            s->tnode.as<float4>(), s->tcone.as<float4>(), s->tleaf.as<float4>(), cuts, cut_cap,
-                           midtops, top_cap, mids, mid_cap, w.members.as<uint32_t>(), w.flags.as<uint32_t>());
+                           midtops, top_cap, mids, mid_cap, w.members.as<uint32_t>(), w.flags.as<uint32_t>(),
+                           w.slabs.as<uint32_t>());
         if (any_big)
             hipLaunchKernelGGL(k_refit_mid<DIM>, dim3(std::min(mid_cap, 2u * n_cu)), dim3(MB), 0, st,
                                w.parent.as<uint32_t>(), w.child.as<uint2>(), w.range.as<uint2>(),

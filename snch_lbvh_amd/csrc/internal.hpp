@@ -40,7 +40,7 @@ struct BatchConfig {
 
 struct BuildScratch {
     DeviceBuffer leafbox /* leaf records: box + cone, 3 float4 */, scene_bits, boxpart, codes, idx, codes_alt, idx_alt, hist, parent, child, range,
-        flags, top, tops, status, mids, midtops, members;
+        flags, top, tops, status, mids, midtops, members, slabs;
 };
 
 } // namespace snch

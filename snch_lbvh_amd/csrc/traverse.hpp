@@ -51,11 +51,12 @@ __device__ __forceinline__ ChildRec load_child(const float4* __restrict__ tnode,
 struct ConeRec {
     v3 axis;
     float half_angle, sin_ha, cos_ha, radius;
+    uint32_t slab;
 };
 __device__ __forceinline__ ConeRec load_cone(const float4* __restrict__ tcone, uint32_t i, uint32_t side)
 {
     const float4 a = tcone[4 * i + 2 * side], b = tcone[4 * i + 2 * side + 1];
-    return ConeRec{mk(a.x, a.y, a.z), a.w, b.x, b.y, b.z};
+    return ConeRec{mk(a.x, a.y, a.z), a.w, b.x, b.y, b.z, __float_as_uint(b.w)};
 }
 
 // a child the traversal treats as a leaf: a true leaf, or a run of sorted
@@ -164,14 +165,17 @@ __device__ __forceinline__ bool overlap_dim(const float4& C, float radius, v3 p,
                     : cone_overlap2d(mk(C.x, C.y, 0.0f), C.w, radius, p, b, md);
 }
 
-// the cone test of a child whose box lies at squared distance md (query.cuh:366-367)
+// the cone test of a child whose box lies at squared distance md
+// (query.cuh:366-367), without the children no edge of which can be a
+// silhouette (cone_slab_clear)
 template <int DIM>
 __device__ __forceinline__ bool cone_hit(const TreeView& t, const ConeRec& c, v3 p, const box3& b, float md)
 {
     if (!cone_valid(c.half_angle))
         return false;
     if (DIM == 3 && (t.flags & TREE_FAST_CONE))
-        return cone_overlap_fast(c.axis, c.half_angle, c.sin_ha, c.cos_ha, c.radius, p, b, md);
+        return !cone_slab_clear(c.axis, c.half_angle, c.sin_ha, c.cos_ha, c.radius, c.slab, p, b) &&
+               cone_overlap_fast(c.axis, c.half_angle, c.sin_ha, c.cos_ha, c.radius, p, b, md);
     return overlap_dim<DIM>(make_float4(c.axis.x, c.axis.y, c.axis.z, c.half_angle), c.radius, p, b, md);
 }
 

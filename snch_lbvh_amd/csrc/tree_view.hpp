@@ -23,8 +23,9 @@ namespace snch {
 //             c as one leaf holding that run of sorted leaves (as_leaf).
 //   tcone[i]  4 x float4 = 64 B per internal node: the children's normal
 //             cones, 32 B each, read only by the silhouette query:
-//               [0] L.axis L.half_angle  [1] sin, cos of L.half_angle, L.radius, 0
-//               [2] R.axis R.half_angle  [3] sin, cos of R.half_angle, R.radius, 0
+//               [0] L.axis L.half_angle  [1] sin, cos of L.half_angle, L.radius, L.slab
+//               [2] R.axis R.half_angle  [3] sin, cos of R.half_angle, R.radius, R.slab
+//             slab: the extent of the child's edges along the axis (pack_slab)
 //   tleaf[j]  3 x float4 = 48 B per leaf, in Morton (sorted) order:
 //               [k] vertex k xyz, w = (original triangle, first owned edge,
 //               owned edge count) for k = 0, 1, 2
@@ -51,7 +52,7 @@ struct MeshDesc {
     uint32_t off, n, eoff, nb;
 };
 
-constexpr uint32_t TREE_FAST_CONE = 1u; // TreeView::flags: cone_overlap_fast may replace cone_overlap
+constexpr uint32_t TREE_FAST_CONE = 1u; // TreeView::flags: cone_overlap_fast may replace cone_overlap, and slabs hold
 constexpr uint32_t TREE_RUNS = 2u;      // children may be leaf runs (built with leaf size > 1)
 
 struct TreeView {
