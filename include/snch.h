@@ -66,7 +66,8 @@ typedef struct snch_query_opts {
     uint32_t block_size; /* threads per block: 64, 128, 256 or 512; 0 = default (64).  Outputs
                             are the same. */
     uint32_t coherent;   /* visiting order: 0 = Morton order of the query points when
-                            n >= SNCH_ORDER_MIN_QUERIES, 1 = always Morton order,
+                            n >= SNCH_ORDER_MIN_QUERIES (closest point: and the tree
+                            has more than 65,536 leaves), 1 = always Morton order,
                             2 = input order.  Results are written in input order and
                             do not depend on the visiting order. */
     uint64_t *stats;     /* optional DEVICE uint64[5], accumulated: child box tests, leaf

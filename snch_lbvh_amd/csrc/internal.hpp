@@ -157,6 +157,8 @@ hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q,
                                      const float* seed, bool capped, uint32_t* sil, float* dist, uint32_t block,
                                      uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t* ctr,
                                      uint32_t n_cu, hipStream_t st, uint32_t* err = nullptr);
+// whether a launch of that shape is persistent (it uses ctr then)
+bool silhouette_persists(uint32_t n, uint32_t block, uint32_t depth, bool hard, uint32_t n_cu);
 hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* o, const float* d,
                       const float* tmax, uint32_t n, int any_hit, uint8_t* hit, float* tout, float* uv, uint32_t* idx,
                       uint64_t* stats, uint32_t* ctr, uint32_t n_cu, hipStream_t st);

@@ -37,7 +37,7 @@ constexpr int OVF = 64; // private overflow entries per lane (generic queries)
 // ------------------------------------------------------------ closest point
 template <bool STATS, int DIM>
 __global__ __launch_bounds__(512, 6) void k_closest_point(TreeView t, const float* __restrict__ q, uint32_t n,
-                                                          uint32_t qpw, uint32_t cap, uint32_t* __restrict__ out_idx,
+                                                          uint32_t deal, uint32_t cap, uint32_t* __restrict__ out_idx,
                                                           float* __restrict__ out_dist,
                                                           const uint32_t* __restrict__ perm, uint32_t* ctr,
                                                           uint32_t* __restrict__ err, unsigned long long* stats)
@@ -47,11 +47,11 @@ __global__ __launch_bounds__(512, 6) void k_closest_point(TreeView t, const floa
     WaveLds W(smem + (threadIdx.x >> 6) * wave_lds_words(cap), cap);
     if (t.n_dev)
         n = min(n, *t.n_dev);
-    if (qpw == 0u)
-        qpw = queries_per_wave(n, gridDim.x * (blockDim.x >> 6));
+    if (deal == 0u)
+        deal = deal_queries(n, gridDim.x * (blockDim.x >> 6), CP_RUNS);
     bool ovf = false;
     Counts cnt;
-    for_chunks(n, qpw, ctr, [&](uint32_t slot, bool valid) {
+    for_chunks(n, deal, ctr, [&](uint32_t slot, bool valid) {
         const uint32_t qi = valid ? (perm ? min(perm[slot], n - 1) : slot) : 0u;
         if (valid)
             W.start(lane, load_point<DIM>(q, qi));
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(512, 6) void k_closest_point(TreeView t, const floa
 template <bool STATS, int DIM, bool ANY>
 __global__ __launch_bounds__(64, 6) void k_ray(TreeView t, const float4* __restrict__ V, const int32_t* __restrict__ F,
                                                const float* __restrict__ o, const float* __restrict__ d,
-                                               const float* __restrict__ tmax, uint32_t n, uint32_t qpw,
+                                               const float* __restrict__ tmax, uint32_t n, uint32_t deal,
                                                uint8_t* __restrict__ out_hit, float* __restrict__ out_t,
                                                float* __restrict__ out_uv, uint32_t* __restrict__ out_idx,
                                                uint32_t* ctr, uint32_t* __restrict__ err, unsigned long long* stats)
@@ -86,11 +86,11 @@ __global__ __launch_bounds__(64, 6) void k_ray(TreeView t, const float4* __restr
     RayLds W(smem);
     if (t.n_dev)
         n = min(n, *t.n_dev);
-    if (qpw == 0u)
-        qpw = queries_per_wave(n, gridDim.x);
+    if (deal == 0u)
+        deal = deal_queries(n, gridDim.x, RAY_RUNS);
     bool ovf = false;
     Counts cnt;
-    for_chunks(n, qpw, ctr, [&](uint32_t qi, bool valid) {
+    for_chunks(n, deal, ctr, [&](uint32_t qi, bool valid) {
         float max_dist = F_INF;
         v3 ro = mk(0.0f, 0.0f, 0.0f), rd = ro;
         if (valid) {
@@ -428,16 +428,17 @@ hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint
     if (n == 0)
         return hipSuccess;
     auto* sp = reinterpret_cast<unsigned long long*>(stats);
-    const SearchGrid g = search_grid(n, block, wave_lds_words(pool_cap(depth)), n_cu, 6, ctr != nullptr, t.n_dev != nullptr);
+    const SearchGrid g = search_grid(n, block, wave_lds_words(pool_cap(depth)), n_cu, 6, ctr != nullptr,
+                                      t.n_dev != nullptr, CP_RUNS);
     uint32_t* c = g.persist ? ctr : nullptr;
     if (c)
         hipLaunchKernelGGL(k_clear_chunks, dim3(1), dim3(64), 0, st, c);
     SNCH_DISPATCH_DIM(dim, {
         if (stats)
-            hipLaunchKernelGGL((k_closest_point<true, DIM>), g.grid, g.block, g.lds, st, t, q, n, g.qpw,
+            hipLaunchKernelGGL((k_closest_point<true, DIM>), g.grid, g.block, g.lds, st, t, q, n, g.deal,
                                pool_cap(depth), idx, dist, perm, c, traversal_error_word(), sp);
         else
-            hipLaunchKernelGGL((k_closest_point<false, DIM>), g.grid, g.block, g.lds, st, t, q, n, g.qpw,
+            hipLaunchKernelGGL((k_closest_point<false, DIM>), g.grid, g.block, g.lds, st, t, q, n, g.deal,
                                pool_cap(depth), idx, dist, perm, c, traversal_error_word(), sp);
     });
     return hipGetLastError();
@@ -450,12 +451,12 @@ hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t
     if (n == 0)
         return hipSuccess;
     auto* sp = reinterpret_cast<unsigned long long*>(stats);
-    const SearchGrid g = search_grid(n, 64, RayLds::WORDS, n_cu, 6, ctr != nullptr, t.n_dev != nullptr);
+    const SearchGrid g = search_grid(n, 64, RayLds::WORDS, n_cu, 6, ctr != nullptr, t.n_dev != nullptr, RAY_RUNS);
     uint32_t* c = g.persist ? ctr : nullptr;
     if (c)
         hipLaunchKernelGGL(k_clear_chunks, dim3(1), dim3(64), 0, st, c);
 #define SNCH_RAY(S_, A_)                                                                                             \
-    hipLaunchKernelGGL((k_ray<S_, DIM, A_>), g.grid, g.block, 0, st, t, V, F, o, d, tmax, n, g.qpw, hit, tout, uv, idx, \
+    hipLaunchKernelGGL((k_ray<S_, DIM, A_>), g.grid, g.block, 0, st, t, V, F, o, d, tmax, n, g.deal, hit, tout, uv, idx, \
                        c, traversal_error_word(), sp)
     SNCH_DISPATCH_DIM(dim, {
         if (any_hit) {

@@ -7,11 +7,11 @@ namespace {
 
 // MODE 0: plain search.  MODE 1: seed[qi] is a pruning hint.  MODE 2: a hard
 // cap (sil_wave).  A large launch is persistent: as many waves as are
-// resident take 64-query chunks of the visiting order as they get free, each
-// XCD from its own contiguous range first (its L2 holds that region's nodes).
+// resident take chunks of 64 queries as they get free, each XCD from its own
+// range of chunks first (its L2 holds that region's nodes).
 template <bool STATS, int DIM, int MODE>
 __global__ __launch_bounds__(512, STATS ? 4 : 6) void k_silhouette(TreeView t, const float* __restrict__ q, uint32_t n,
-                                                                   uint32_t qpw, uint32_t cap_items, int flip,
+                                                                   uint32_t deal, uint32_t cap_items, int flip,
                                                                    const float* __restrict__ seed,
                                                                    uint32_t* __restrict__ out_e,
                                                                    float* __restrict__ out_d,
@@ -24,11 +24,11 @@ __global__ __launch_bounds__(512, STATS ? 4 : 6) void k_silhouette(TreeView t, c
     WaveLds W(smem + (threadIdx.x >> 6) * wave_lds_words(cap_items, MODE == 2), cap_items);
     if (t.n_dev)
         n = min(n, *t.n_dev);
-    if (qpw == 0u)
-        qpw = queries_per_wave(n, gridDim.x * (blockDim.x >> 6));
+    if (deal == 0u)
+        deal = deal_queries(n, gridDim.x * (blockDim.x >> 6), SIL_RUNS);
     bool ovf = false;
     Counts cnt;
-    for_chunks(n, qpw, ctr, [&](uint32_t slot, bool valid) {
+    for_chunks(n, deal, ctr, [&](uint32_t slot, bool valid) {
         const uint32_t qi = valid ? (perm ? min(perm[slot], n - 1) : slot) : 0u;
         if (valid)
             W.start(lane, load_point<DIM>(q, qi));
@@ -57,6 +57,11 @@ __global__ void k_clear_sil_chunks(uint32_t* __restrict__ ctr)
 
 } // namespace
 
+bool silhouette_persists(uint32_t n, uint32_t block, uint32_t depth, bool hard, uint32_t n_cu)
+{
+    return search_grid(n, block, wave_lds_words(pool_cap(depth), hard), n_cu, 6, true, false, SIL_RUNS).persist;
+}
+
 hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q, uint32_t n, int flip,
                                      const float* seed, bool capped, uint32_t* sil, float* dist, uint32_t block,
                                      uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t* ctr,
@@ -68,12 +73,13 @@ hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q,
     if (!err)
         err = traversal_error_word();
     const bool hard = seed && capped;
-    const SearchGrid g = search_grid(n, block, wave_lds_words(pool_cap(depth), hard), n_cu, 6, ctr != nullptr, t.n_dev != nullptr);
+    const SearchGrid g = search_grid(n, block, wave_lds_words(pool_cap(depth), hard), n_cu, 6, ctr != nullptr,
+                                      t.n_dev != nullptr, SIL_RUNS);
     uint32_t* c = g.persist ? ctr : nullptr;
     if (c)
         hipLaunchKernelGGL(k_clear_sil_chunks, dim3(1), dim3(64), 0, st, c);
 #define SNCH_SIL(S_, M_)                                                                                             \
-    hipLaunchKernelGGL((k_silhouette<S_, DIM, M_>), g.grid, g.block, g.lds, st, t, q, n, g.qpw, pool_cap(depth), flip, \
+    hipLaunchKernelGGL((k_silhouette<S_, DIM, M_>), g.grid, g.block, g.lds, st, t, q, n, g.deal, pool_cap(depth), flip, \
                        seed, sil, dist, perm, c, err, sp)
     SNCH_DISPATCH_DIM(dim, {
         if (!seed) {

@@ -907,26 +907,47 @@ __device__ __forceinline__ uint32_t take_chunk(uint32_t* ctr, uint32_t nchunks, 
 }
 constexpr uint32_t CHUNK_CTR_WORDS = 8;
 
-// queries per wave of a launch over n: 64 consecutive ones of the visiting
-// order, or fewer when that would leave resident waves without work
-__host__ __device__ __forceinline__ uint32_t queries_per_wave(uint32_t n, uint32_t waves)
+// How the queries of a launch over n are dealt to its waves: the queries per wave
+// (64, or fewer where that would leave resident waves without work), and in bits
+// 8 and up the logarithm of the run length, the queries in sequence in the
+// visiting order that one wave gets.  Neighbours cost alike, and the costliest
+// lie together (around the centre of a sphere): a wave that gets 64 of them in
+// one run works on long after the others are done, while runs of one spread
+// them over all waves.  Runs share tree records between their queries, though.
+// Run length 1 where each resident wave has at most one chunk, twice that for
+// each doubling of the chunks per wave, up to 2^most.  For 2^22 queries: closest
+// point, 2^20 / 20,480 triangles, in runs of 1 / 4 / 64: 20.7 / 20.2 / 22.7 and
+// 3.7 / 3.4 / 4.2 ms; silhouette, torus of 2^20 / sphere of 327,680, in runs of
+// 1 / 16 / 64: 55 / 25 / 26 and 64 / 363 / 586 ms.  Rays cost alike and come in
+// the caller's order, often an image's: runs of 1 / 16 / 64: 1.16 / 1.01 / 0.98
+// ms, so 2^least = 2^most = 64.
+struct Runs {
+    uint32_t least, most;
+};
+constexpr Runs CP_RUNS{0, 2}, SIL_RUNS{0, 4}, RAY_RUNS{6, 6};
+__host__ __device__ __forceinline__ uint32_t deal_queries(uint32_t n, uint32_t waves, Runs r)
 {
     const uint32_t w = waves > 0u ? waves : 1u, k = n / w + (n % w ? 1u : 0u);
-    return k < 1u ? 1u : k > 64u ? 64u : k;
+    if (k <= 64u)
+        return k < 1u ? 1u : k;
+    uint32_t run = r.least;
+    while (run < r.most && (k >> (6u + run)) > 0u)
+        ++run;
+    return 64u | run << 8;
 }
 
-// Calls f(slot, valid) with the queries of each chunk of this wave.  Chunks of
-// 64 are consecutive queries of the visiting order; smaller ones take every
-// nchunks-th query, so that costly neighbours (the centre of a sphere) land in
-// different waves.  One chunk per wave where there are waves enough; else
-// (ctr, a persistent launch) the waves take chunks as they get free.
+// Calls f(slot, valid) with the queries of each chunk of this wave.  One chunk
+// per wave where there are waves enough; else (ctr, a persistent launch) the
+// waves take chunks as they get free.
 template <class F>
-__device__ __forceinline__ void for_chunks(uint32_t n, uint32_t qpw, uint32_t* ctr, F f)
+__device__ __forceinline__ void for_chunks(uint32_t n, uint32_t deal, uint32_t* ctr, F f)
 {
     const uint32_t lane = threadIdx.x & 63, wpb = blockDim.x >> 6, w = threadIdx.x >> 6;
+    const uint32_t qpw = deal & 255u, run = deal >> 8;
     const uint32_t waves = gridDim.x * wpb, nchunks = n / qpw + (n % qpw ? 1u : 0u);
+    const uint32_t first = ((lane >> run) * nchunks << run) + (lane & ((1u << run) - 1u));
     auto chunk = [&](uint32_t c) {
-        const uint32_t slot = qpw < 64u ? lane * nchunks + c : c * 64u + lane;
+        const uint32_t slot = first + (c << run);
         f(slot, lane < qpw && slot < n);
     };
     if (nchunks <= waves || !ctr) {
@@ -947,20 +968,20 @@ inline uint32_t nblocks(uint32_t n, uint32_t bs) { return (n + bs - 1) / bs; }
 // are resident (wave_words words of LDS each, at most `per_simd` on a SIMD)
 struct SearchGrid {
     dim3 grid, block;
-    uint32_t qpw;
+    uint32_t deal; // deal_queries, or 0: from the count on the device
     size_t lds;
     bool persist;
 };
 inline SearchGrid search_grid(uint32_t n, uint32_t block, uint32_t wave_words, uint32_t n_cu, uint32_t per_simd,
-                              bool may_persist, bool n_on_device)
+                              bool may_persist, bool n_on_device, Runs runs)
 {
     SearchGrid g;
     const uint32_t wpb = block / 64;
     g.lds = sizeof(uint32_t) * wpb * wave_words;
     const uint32_t per_cu = std::max(1u, std::min((uint32_t)(LDS_PER_CU / g.lds), per_simd * 4u / wpb));
     const uint32_t resident = n_cu * per_cu;
-    g.qpw = n_on_device ? 0u : queries_per_wave(n, resident * wpb); // 0: from the count on the device
-    const uint32_t blocks = nblocks(nblocks(n, g.qpw ? g.qpw : 1u), wpb);
+    g.deal = n_on_device ? 0u : deal_queries(n, resident * wpb, runs);
+    const uint32_t blocks = nblocks(nblocks(n, g.deal ? g.deal & 255u : 1u), wpb);
     g.persist = may_persist && blocks > resident;
     g.grid = dim3(g.persist ? resident : blocks);
     g.block = dim3(block);

@@ -43,7 +43,7 @@ def test_closest_point_does_not_depend_on_the_launch(name, leaf_size):
     V, F = _meshes()[name]
     q = _points(V, 70000, 11)
     sc = S.Scene(V, F).build_bvh(leaf_size=leaf_size)
-    i0, d0 = (x.cpu().numpy() for x in sc.closest_point(q))  # 64 queries a wave, Morton order
+    i0, d0 = (x.cpu().numpy() for x in sc.closest_point(q))  # the default launch
     for n in (1, 2, 8, 9, 63, 64, 65, 1000):
         i1, d1 = (x.cpu().numpy() for x in sc.closest_point(q[:n]))
         np.testing.assert_array_equal(d1, d0[:n])
