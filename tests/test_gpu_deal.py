@@ -50,3 +50,26 @@ def test_largest_pools(block_size, cap):
     else:
         e1, d1 = sc.closest_silhouette(q, block_size=block_size, stack_depth=32)
     assert torch.equal(d0, d1) and torch.equal(e0, e1)
+
+
+@pytest.mark.parametrize("sizes", [(1, 70, 1), (5001, 0, 63), (450001, 10, 129)])
+@pytest.mark.parametrize("queries_per_wave", [64, 256])
+def test_batch(sizes, queries_per_wave):
+    import torch
+
+    import snch_lbvh_amd as S
+    from snch_lbvh_amd import workloads as W
+
+    meshes = [W.cut_torus(24, 12), W.cut_torus(8, 6), (W.icosphere(2, 0.05, seed=2))]
+    lo, hi = W.padded_box(meshes[0][0], 0.2)
+    q = torch.from_numpy(W.uniform_points(sum(sizes), lo, hi, 7)).cuda()
+    off = np.cumsum([0, *sizes])
+    b = S.BatchScene(meshes).build_bvh()
+    tune = {"block_size": 128, "stack_depth": 8, "queries_per_wave": queries_per_wave}
+    for name in ("closest_point", "closest_silhouette"):
+        i, d = getattr(b, name)(q, off, tune=tune)
+        for m, (V, F) in enumerate(meshes):
+            s = slice(int(off[m]), int(off[m + 1]))
+            if sizes[m]:
+                i1, d1 = getattr(S.Scene(V, F).build_bvh(), name)(q[s])
+                assert torch.equal(d[s], d1) and torch.equal(i[s], i1)
