@@ -89,6 +89,9 @@ struct snch_scene {
     float last_phase_ms[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     // repeat builds replay the launch sequence captured on the second build
     // with the same (flags, leaf size); every buffer it names is sized by then
+    hipEvent_t build_ev[2] = {nullptr, nullptr}; // around a build
+    uint32_t* errors_host = nullptr;             // pinned: the error words after a build
+    std::vector<char> views_host;                // what batch.views holds
     hipGraphExec_t build_exec = nullptr;
     uint32_t build_key = 0, eager_key = 0, eager_builds = 0;
     // the per-handle query scratch (qscratch, batch) is reused by every call:
@@ -181,5 +184,6 @@ uint32_t* traversal_error_word(); // [0] traversal overflow, [1] sort wait bound
 // (current), resolved once per device
 hipError_t noalloc_init(int device, uint32_t** out);
 // SNCH_OK, or the error code and message of a sticky device error (cleared)
-int check_device_errors(const char* fn);
+// copied: the words, copied in stream order (null: they are copied here)
+int check_device_errors(const char* fn, const uint32_t* copied = nullptr);
 } // namespace snch
