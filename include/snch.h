@@ -75,7 +75,7 @@ typedef struct snch_query_opts {
                             visited, cone records read (silhouette query only) */
     const uint32_t *order; /* optional DEVICE permutation of [0, n) (e.g. from
                               snch_query_order): the visiting order; overrides coherent */
-    uint32_t stack_depth;      /* LDS of a wavefront's pool of pending nodes, 40 nodes per unit:
+    uint32_t stack_depth;      /* LDS of a wavefront's pool of pending nodes, 40 nodes per unit and at least 640:
                                   closest point 8 or 16 (0 = 16), closest silhouette (3D) and
                                   batched queries 8, 16, 24 or 32 (0 = 16).  Outputs are the same. */
     uint32_t queries_per_wave; /* batched queries: queries a wavefront takes from the work

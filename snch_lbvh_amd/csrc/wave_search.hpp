@@ -52,16 +52,20 @@ __device__ __forceinline__ void flush_counts(const Counts& c, unsigned long long
 // wave as slow as its slowest lane, a lane as slow as its chain of dependent
 // loads) every lane has work until the wave's last query ends, a node's two
 // children share one 64-B line per pair of lanes, and leaf code runs on full
-// waves.  Queries enter as the pool runs low, POOL_ADD at a time: with all 64
-// in flight at once the pool fills and pops one item at a time.
+// waves.  Queries enter as the pool runs low, CP_ADD or SIL_ADD at a time: with
+// all 64 in flight at once the pool fills and pops one item at a time.
 //
-// Measured, one lane per query with a stack -> pool.  Closest point: 2^22
-// queries on 2^20 triangles 46 -> 24 ms, 65,536 on 20,480 triangles 2.1 ->
-// 0.18 ms, 1,000 on 20,480 triangles 0.83 -> 0.03 ms (there a launch lasted as
-// long as the longest chain of dependent loads, about 2 us a node).  Closest
-// silhouette: 2^22 on 2^20 triangles 69 -> 36 ms (POOL_ADD 4: 43, 8: 41, 12:
-// 38, 16: 37, 24: 35), 10,007 on 90,000 triangles 4.3 -> 0.18 ms.  Pairs that
-// keep their near child in registers instead of the pool: 50 to 58 ms.
+// Measured, one lane per query with a stack -> pool (each with all that is in
+// this file now).  Closest point: 2^22 queries on 2^20 triangles 46 -> 19 ms,
+// 65,536 on 20,480 triangles 2.1 -> 0.12 ms, 1,000 0.83 -> 0.03 ms (there a
+// launch lasted as long as the longest chain of dependent loads, about 2 us a
+// node).  Closest silhouette: 2^22 on 2^20 triangles 68 -> 22.5 ms, 10,007 on
+// 90,000 triangles 4.3 -> 0.13 ms.  Pairs that keep their near child in
+// registers instead of the pool: half as long again.  For those 2^22 queries:
+// SIL_ADD 12 / 20 / 26 / 32 / 40 / 64: 26.7 / 25.7 / 24.7 / 22.6 / 24.5 / 25.0
+// ms; CP_ADD 16 to 24: within 1%; runs of 24 / 32 / 40 / 48 / 64 leaves: closest
+// point 22.0 / 21.0 / 20.1 / 19.7 / 19.3, silhouette 25.2 / 25.2 / 25.7 / 25.9 /
+// 25.9 (and 6% more of 10,007 with 64).
 //
 // The answer is that of the search one lane would make alone, near child
 // first, each node's leaves at once, which skips a box as soon as its lower
@@ -74,9 +78,9 @@ __device__ __forceinline__ void flush_counts(const Counts& c, unsigned long long
 // rounding, which leaves no such candidate out, and where a hidden leaf has
 // the smallest distance the lane repeats the search alone, from the widened
 // bound (a few dozen nodes).
-constexpr uint32_t POOL_ADD = 20;
-constexpr uint32_t LEAF_RUN = 40;            // leaves that are worth a step of the wave
-constexpr uint32_t LEAF_CAP = LEAF_RUN + 64; // buffer entries: below LEAF_RUN before a step, which adds at most 64
+constexpr uint32_t CP_ADD = 20, SIL_ADD = 32;
+constexpr uint32_t CP_LEAF_RUN = 64, SIL_LEAF_RUN = 40; // leaves that are worth a step of the wave
+constexpr uint32_t LEAF_CAP = 64 + 64; // buffer entries: below a run's before a step, which adds at most 64
 
 // smaller is better: the distance, then hidden candidates (so that an answer
 // tells whether any attains it), then the smaller id (distances are not
@@ -160,8 +164,9 @@ __device__ __forceinline__ float scene_scale(const TreeView& t)
 // allow).  A fuller pool pops
 // fewer items at a time (pool_take): closest silhouette on the torus below,
 // with 8-byte items, 62 ms with 480, 53 with 512, 42 with 640 (5 waves per
-// SIMD), 45 with 800 (4 waves).
-constexpr uint32_t pool_cap(uint32_t depth) { return 40 * depth; }
+// SIMD), 45 with 800 (4 waves).  Fewer than 640 starve it for no more waves
+// (320: 95 ms, closest point 142), so depth 8 gets 640 as well.
+constexpr uint32_t pool_cap(uint32_t depth) { return 40 * (depth > 16u ? depth : 16u); }
 // words of dynamic LDS of a wave
 constexpr uint32_t wave_lds_words(uint32_t cap, bool capped = false)
 {
@@ -313,7 +318,7 @@ __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds&
     // evaluates leaves; the bound only guards against a malformed tree
     const uint32_t cap_iters = 128u * t.n_leaves + 65536u;
     for (uint32_t it = 0;; ++it) {
-        if (nleaf >= LEAF_RUN || (nleaf > 0u && todo == 0ull && size < 32u)) {
+        if (nleaf >= CP_LEAF_RUN || (nleaf > 0u && todo == 0ull && size < 32u)) {
             nleaf = cp_leaves<STATS, DIM>(t, W, nleaf, scale, cnt);
             continue;
         }
@@ -324,7 +329,7 @@ __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds&
             break;
         }
         if (size < 32u && todo != 0ull)
-            pool_feed(W, size, todo, POOL_ADD);
+            pool_feed(W, size, todo, CP_ADD);
         const uint32_t k = pool_take(size, W.cap), side = lane & 1u;
         size -= k;
         uint32_t slot = 0, ref = 0;
@@ -365,7 +370,7 @@ __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds&
         pool_push(W, size, go && !leaf && near, (slot << 24) | (ref & REF_MASK), md);
         list_push(W.leaf, nleaf, go && leaf, (slot << 24) | first, md);
         for (uint32_t j = 1; (t.flags & TREE_RUNS) && __ballot(go && leaf && j < count); ++j) {
-            if (nleaf >= LEAF_RUN)
+            if (nleaf >= CP_LEAF_RUN)
                 nleaf = cp_leaves<STATS, DIM>(t, W, nleaf, scale, cnt);
             list_push(W.leaf, nleaf, go && leaf && j < count, (slot << 24) | (first + j), md);
         }
@@ -563,7 +568,7 @@ __device__ __forceinline__ void sil_wave(const TreeView& t, uint64_t all, bool f
     // malformed tree
     const uint32_t cap_iters = 128u * t.n_leaves + 65536u;
     for (uint32_t it = 0;; ++it) {
-        if (nleaf >= LEAF_RUN || (nleaf > 0u && todo == 0ull && size < 32u)) {
+        if (nleaf >= SIL_LEAF_RUN || (nleaf > 0u && todo == 0ull && size < 32u)) {
             nleaf = sil_leaves<STATS, DIM>(t, W, nleaf, scale, flip, cnt);
             continue;
         }
@@ -587,7 +592,7 @@ __device__ __forceinline__ void sil_wave(const TreeView& t, uint64_t all, bool f
             break;
         }
         if (size < 32u && todo != 0ull)
-            pool_feed(W, size, todo, POOL_ADD);
+            pool_feed(W, size, todo, SIL_ADD);
         const uint32_t k = pool_take(size, W.cap), side = lane & 1u;
         size -= k;
         uint32_t slot = 0, ref = 0;
@@ -620,7 +625,7 @@ __device__ __forceinline__ void sil_wave(const TreeView& t, uint64_t all, bool f
         pool_push(W, size, down && near, (slot << 24) | (ref & REF_MASK), md);
         list_push(W.leaf, nleaf, go && leaf, (slot << 24) | first, md);
         for (uint32_t j = 1; (t.flags & TREE_RUNS) && __ballot(go && leaf && j < count); ++j) {
-            if (nleaf >= LEAF_RUN)
+            if (nleaf >= SIL_LEAF_RUN)
                 nleaf = sil_leaves<STATS, DIM>(t, W, nleaf, scale, flip, cnt);
             list_push(W.leaf, nleaf, go && leaf && j < count, (slot << 24) | (first + j), md);
         }
@@ -863,7 +868,7 @@ __device__ __forceinline__ void ray_wave(const TreeView& t, uint64_t all, float 
         pool_push(W, size, go && !leaf && near, (slot << 24) | (ref & REF_MASK), dist);
         list_push(W.leaf, nleaf, go && leaf, (slot << 24) | first, dist);
         for (uint32_t j = 1; (t.flags & TREE_RUNS) && __ballot(go && leaf && j < count); ++j) {
-            if (nleaf >= LEAF_RUN)
+            if (nleaf >= RAY_LEAF_RUN)
                 nleaf = ray_leaves<STATS, DIM, ANY>(t, W, nleaf, scale, cnt);
             list_push(W.leaf, nleaf, go && leaf && j < count, (slot << 24) | (first + j), dist);
         }
