@@ -718,8 +718,10 @@ int snch_closest_silhouette_ex(const snch_scene* s, const float* q, uint32_t n, 
     if (own_order)
         SNCH_HIP(query_order(s->view(), (int)s->dim, q, n, s->qscratch, st, &perm),
                  "snch_closest_silhouette: ordering");
-    if (persist)
+    if (persist) {
         SNCH_HIP(s->chunk_ctr.ensure(sizeof(uint32_t) * 32), "snch_closest_silhouette: allocation");
+        SNCH_HIP(clear_chunks(s->chunk_ctr.as<uint32_t>(), st), "snch_closest_silhouette: counters");
+    }
     SNCH_HIP(launch_closest_silhouette(s->view(), (int)s->dim, q, n, flip, seed, capped, out_sil, out_dist, block,
                                        depth, perm, opts ? opts->stats : nullptr,
                                        persist ? s->chunk_ctr.as<uint32_t>() : nullptr, s->n_cu(), st),

@@ -144,7 +144,7 @@ hipError_t query_order(const TreeView& t, int dim, const float* q, uint32_t n, Q
 size_t query_order_scratch_bytes(uint32_t n);
 hipError_t query_order_in(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* words, hipStream_t st,
                           const uint32_t** perm, uint32_t* err);
-// ctr (nullable; 8 words, rewritten at launch by a kernel: graph capture is
+// ctr (nullable; 8 words, zero at launch: clear_chunks, a kernel, so that capture is
 // fine): lets a large launch be persistent, and is needed where the number of
 // queries is on the device (t.n_dev)
 hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* idx, float* dist,
@@ -160,6 +160,8 @@ hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q,
                                      const float* seed, bool capped, uint32_t* sil, float* dist, uint32_t block,
                                      uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t* ctr,
                                      uint32_t n_cu, hipStream_t st, uint32_t* err = nullptr);
+// zeroes a launch's ctr
+hipError_t clear_chunks(uint32_t* ctr, hipStream_t st);
 // whether a launch of that shape is persistent (it uses ctr then)
 bool silhouette_persists(uint32_t n, uint32_t block, uint32_t depth, bool hard, uint32_t n_cu);
 hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* o, const float* d,

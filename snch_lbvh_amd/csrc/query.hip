@@ -415,12 +415,6 @@ hipError_t query_order_in(const TreeView& t, int dim, const float* q, uint32_t n
     return hipGetLastError();
 }
 
-__global__ void k_clear_chunks(uint32_t* __restrict__ ctr)
-{
-    if (threadIdx.x < CHUNK_CTR_WORDS)
-        ctr[threadIdx.x] = 0u;
-}
-
 hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* idx, float* dist,
                                 uint32_t block, uint32_t depth, const uint32_t* perm, uint64_t* stats, uint32_t* ctr,
                                 uint32_t n_cu, hipStream_t st)
@@ -431,8 +425,6 @@ hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint
     const SearchGrid g = search_grid(n, block, wave_lds_words(pool_cap(depth)), n_cu, 6, ctr != nullptr,
                                       t.n_dev != nullptr, CP_RUNS);
     uint32_t* c = g.persist ? ctr : nullptr;
-    if (c)
-        hipLaunchKernelGGL(k_clear_chunks, dim3(1), dim3(64), 0, st, c);
     SNCH_DISPATCH_DIM(dim, {
         if (stats)
             hipLaunchKernelGGL((k_closest_point<true, DIM>), g.grid, g.block, g.lds, st, t, q, n, g.deal,
@@ -453,8 +445,6 @@ hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t
     auto* sp = reinterpret_cast<unsigned long long*>(stats);
     const SearchGrid g = search_grid(n, 64, RayLds::WORDS, n_cu, 6, ctr != nullptr, t.n_dev != nullptr, RAY_RUNS);
     uint32_t* c = g.persist ? ctr : nullptr;
-    if (c)
-        hipLaunchKernelGGL(k_clear_chunks, dim3(1), dim3(64), 0, st, c);
 #define SNCH_RAY(S_, A_)                                                                                             \
     hipLaunchKernelGGL((k_ray<S_, DIM, A_>), g.grid, g.block, 0, st, t, V, F, o, d, tmax, n, g.deal, hit, tout, uv, idx, \
                        c, traversal_error_word(), sp)

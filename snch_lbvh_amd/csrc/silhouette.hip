@@ -49,7 +49,7 @@ __global__ __launch_bounds__(512, STATS ? 4 : 6) void k_silhouette(TreeView t, c
         flush_counts(cnt, stats);
 }
 
-__global__ void k_clear_sil_chunks(uint32_t* __restrict__ ctr)
+__global__ void k_clear_chunks(uint32_t* __restrict__ ctr)
 {
     if (threadIdx.x < CHUNK_CTR_WORDS)
         ctr[threadIdx.x] = 0u;
@@ -60,6 +60,12 @@ __global__ void k_clear_sil_chunks(uint32_t* __restrict__ ctr)
 bool silhouette_persists(uint32_t n, uint32_t block, uint32_t depth, bool hard, uint32_t n_cu)
 {
     return search_grid(n, block, wave_lds_words(pool_cap(depth), hard), n_cu, 6, true, false, SIL_RUNS).persist;
+}
+
+hipError_t clear_chunks(uint32_t* ctr, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_clear_chunks, dim3(1), dim3(64), 0, st, ctr);
+    return hipGetLastError();
 }
 
 hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q, uint32_t n, int flip,
@@ -76,8 +82,6 @@ hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q,
     const SearchGrid g = search_grid(n, block, wave_lds_words(pool_cap(depth), hard), n_cu, 6, ctr != nullptr,
                                       t.n_dev != nullptr, SIL_RUNS);
     uint32_t* c = g.persist ? ctr : nullptr;
-    if (c)
-        hipLaunchKernelGGL(k_clear_sil_chunks, dim3(1), dim3(64), 0, st, c);
 #define SNCH_SIL(S_, M_)                                                                                             \
     hipLaunchKernelGGL((k_silhouette<S_, DIM, M_>), g.grid, g.block, g.lds, st, t, q, n, g.deal, pool_cap(depth), flip, \
                        seed, sil, dist, perm, c, err, sp)

@@ -138,13 +138,15 @@ __global__ void k_walk_codes(Walks w, int cur, uint32_t cap, const float4* __res
         return;
     const uint32_t n = min(w.count[cur], cap);
     if (i >= n) {
-        codes[i] = 0xFFFFFFFFu;
+        codes[i] = 0xFFFFu;
         idx[i] = 0xFFFFFFFFu;
         return;
     }
     const uint32_t wk = w.live[cur][i];
     const float4 p = w.pos[wk], lo = nbox[0], hi = nbox[1];
-    codes[i] = morton3(mk((p.x - lo.x) / (hi.x - lo.x), (p.y - lo.y) / (hi.y - lo.y), (p.z - lo.z) / (hi.z - lo.z)));
+    // 32 cells per axis: two sort passes instead of four, 20 of a step's 700 us
+    codes[i] =
+        morton3(mk((p.x - lo.x) / (hi.x - lo.x), (p.y - lo.y) / (hi.y - lo.y), (p.z - lo.z) / (hi.z - lo.z))) >> 15;
     idx[i] = wk;
 }
 
@@ -156,11 +158,14 @@ __global__ void k_apply_order(Walks w, int cur, uint32_t cap, const uint32_t* __
         w.live[cur][i] = sorted[i];
 }
 
-__global__ void k_gather(Walks w, int cur, uint32_t cap)
+// ctr: the chunk counters of the three persistent launches that follow
+__global__ void k_gather(Walks w, int cur, uint32_t cap, uint32_t* __restrict__ ctr)
 {
     const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i == 0)
         w.count[cur ^ 1] = 0; // next list starts empty (a kernel, not a memset: graph safe)
+    if (i < 24)
+        ctr[i] = 0u;
     const uint32_t n = min(w.count[cur], cap);
     if (i >= n)
         return;
@@ -314,11 +319,12 @@ hipError_t enqueue_steps(snch_wost* s, uint32_t max_steps, float eps, uint64_t s
                            s->oidx.as<uint32_t>());
         bool in_alt = false;
         if ((e = radix_sort_pairs(s->ocodes.as<uint32_t>(), s->oidx.as<uint32_t>(), s->ocodes_alt.as<uint32_t>(),
-                                  s->oidx_alt.as<uint32_t>(), cap, 32, s->ohist, st, &in_alt)) != hipSuccess)
+                                  s->oidx_alt.as<uint32_t>(), cap, 16, s->ohist, st, &in_alt)) != hipSuccess)
             return e;
         hipLaunchKernelGGL(k_apply_order, dim3(nb), dim3(256), 0, st, s->w, cur, cap,
                            in_alt ? s->oidx_alt.as<uint32_t>() : s->oidx.as<uint32_t>());
-        hipLaunchKernelGGL(k_gather, dim3(nb), dim3(256), 0, st, s->w, cur, cap);
+        hipLaunchKernelGGL(k_gather, dim3(nb), dim3(256), 0, st, s->w, cur, cap,
+                           s->chunk_ctr.as<uint32_t>());
         // persistent launches over the walks still live (their count is on the device)
         if ((e = launch_closest_point(vd, 3, s->w.qpos, cap, s->w.cp_idx, s->w.cp_dist, 64, 16, nullptr, nullptr,
                                       s->chunk_ctr.as<uint32_t>(), n_cu, st)) != hipSuccess)
@@ -326,14 +332,14 @@ hipError_t enqueue_steps(snch_wost* s, uint32_t max_steps, float eps, uint64_t s
         // the silhouette within the star radius bound (the closest-point distance)
         if (has_n && (e = launch_closest_silhouette(vn, 3, s->w.qpos, cap, 0, s->w.cp_dist, true, s->w.sil_idx,
                                                     s->w.sil_dist, 64, 16, nullptr, nullptr,
-                                                    s->chunk_ctr.as<uint32_t>(), n_cu, st)) != hipSuccess)
+                                                    s->chunk_ctr.as<uint32_t>() + 8, n_cu, st)) != hipSuccess)
             return e;
         hipLaunchKernelGGL(k_star, dim3(nb), dim3(256), 0, st, s->w, cur, cap, s->dir->dV.as<float4>(),
                            s->dir->dF.as<int32_t>(), eps, seed, has_n);
         if (has_n) {
             if ((e = launch_ray(vn, 3, s->neu->dV.as<float4>(), s->neu->dF.as<int32_t>(), s->w.ray_o, s->w.ray_d,
                                 s->w.star_r, cap, 0, s->w.ray_hit, s->w.ray_t, nullptr, s->w.ray_idx, nullptr,
-                                s->chunk_ctr.as<uint32_t>(), n_cu, st)) != hipSuccess)
+                                s->chunk_ctr.as<uint32_t>() + 16, n_cu, st)) != hipSuccess)
                 return e;
             if ((e = launch_sample(vn, 3, s->neu->dV.as<float4>(), s->neu->dF.as<int32_t>(), s->w.qpos, s->w.sph_r,
                                    s->w.sph_u, cap, s->w.smp_idx, s->w.smp_pdf, nullptr, st)) != hipSuccess)
