@@ -923,13 +923,14 @@ constexpr uint32_t CHUNK_CTR_WORDS = 8;
 // each doubling of the chunks per wave, up to 2^most.  For 2^22 queries: closest
 // point, 2^20 / 20,480 triangles, in runs of 1 / 4 / 64: 20.7 / 20.2 / 22.7 and
 // 3.7 / 3.4 / 4.2 ms; silhouette, torus of 2^20 / sphere of 327,680, in runs of
-// 1 / 16 / 64: 55 / 25 / 26 and 64 / 363 / 586 ms.  Rays cost alike and come in
-// the caller's order, often an image's: runs of 1 / 16 / 64: 1.16 / 1.01 / 0.98
-// ms, so 2^least = 2^most = 64.
+// 1 / 16 / 64: 55 / 25 / 26 and 64 / 363 / 586 ms.  Rays come in the
+// caller's order: 2^22 random ones do not care (1.00 ms in runs of 4 to 64, 1.16
+// in runs of 1), 2048 x 2048 of an image do (0.38 ms in runs of 1 to 32, 0.58 in
+// runs of 64; 632 x 632: 0.11 and 0.18), so 2^least = 4 and 2^most = 16.
 struct Runs {
     uint32_t least, most;
 };
-constexpr Runs CP_RUNS{0, 2}, SIL_RUNS{0, 4}, RAY_RUNS{6, 6};
+constexpr Runs CP_RUNS{0, 2}, SIL_RUNS{0, 4}, RAY_RUNS{2, 4};
 __host__ __device__ __forceinline__ uint32_t deal_queries(uint32_t n, uint32_t waves, Runs r)
 {
     const uint32_t w = waves > 0u ? waves : 1u, k = n / w + (n % w ? 1u : 0u);
