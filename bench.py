@@ -25,11 +25,11 @@ HBM_PEAK_GBS = 8000.0
 # kernel's own visit counters (one extra launch with counters on):
 #   in 12 B (point) + out 8 B (distance + silhouette id)
 #   + nodes visited * 64 B (node record: both child boxes and references)
-#   + cone records read * 48 B (both child cones and radii)
+#   + cone records read * 64 B (both child cones, radii and edge slabs)
 #   + leaves evaluated * 32 B (edge range words of the leaf record)
 #   + silhouette-edge tests * 32 B (endpoints, id, flags; the 32 B of face
 #     normals read only for edges within the current bound are not counted)
-S_NODE, S_CONE, S_LEAF, S_EDGE, S_IN, S_OUT = 64, 48, 32, 32, 12, 8
+S_NODE, S_CONE, S_LEAF, S_EDGE, S_IN, S_OUT = 64, 64, 32, 32, 12, 8
 
 
 def parse():
@@ -584,11 +584,11 @@ def main():
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "bytes_per_query": per_q,
                 "definition": "algorithmic bytes = this kernel's own per-query visits (counters of the same launch) "
-                              "x record sizes as read; the reference traversal's visits would give "
+                              "x record sizes as read, most of them served by caches (traffic_frac is the HBM side); the reference traversal's visits would give "
                               "bytes_per_query_reference_order (it tests ~4x more boxes)",
                 "bytes_per_query_reference_order": ref_bytes,
                 "traffic_frac": (traffic / (kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBS) if traffic else None,
-                "kernel": "k_sil_persist<16, false, 3, false>", "kernel_ms": kernel_ms, "step_ms_events": step_ms,
+                "kernel": "k_silhouette<false, 3, 0>", "kernel_ms": kernel_ms, "step_ms_events": step_ms,
                 "query_order_ms": order_ms, "input_order_kernel_ms": input_order_ms, "shape_sweep_ms": sweep,
                 "visits_per_query": {"nodes": node, "cone_records": cone, "leaves": leaf, "edge_tests": edge}}
 
@@ -610,9 +610,8 @@ def main():
         out_e2 = torch.empty_like(out_e)
         out_d2 = torch.empty_like(out_d)
 
-        def seeded(seed_tensor, in_place=0):
-            # unsettled queries re-queued for whole waves (the default), or searched again in place
-            opts = S.QueryOpts(0, 0, None, None, 0, 0, 0, in_place)
+        def seeded(seed_tensor):
+            opts = S.QueryOpts(0, 0, None, None)
             S.check(S.lib().snch_closest_silhouette_ex(sc._h, S._ptr(q), n, 0, S._ptr(seed_tensor), S._ptr(out_e2),
                                                        S._ptr(out_d2), ctypes.byref(opts), S._stream()))
 
@@ -631,13 +630,11 @@ def main():
         best = min(margins, key=lambda r: margins[r]["ms_per_step"])
         best_rel, best_abs = margins[best]["rel"], margins[best]["abs"]
 
-        def lstep(in_place=0):
+        def lstep():
             mlp.seed_radius(q, rel=best_rel, abs_margin=best_abs, out=seed_r)
-            seeded(seed_r, in_place)
+            seeded(seed_r)
 
         lwall, lms = run_timed(lstep, args.steps, args.warmup)
-        assert torch.equal(out_e2, out_e) and torch.equal(out_d2, out_d), "seeded result differs"
-        pwall, _ = run_timed(lambda: lstep(1), max(2, args.steps // 3), 1)
         assert torch.equal(out_e2, out_e) and torch.equal(out_d2, out_d), "seeded result differs"
         st2 = torch.zeros(5, dtype=torch.int64, device=dev)
         sc.closest_silhouette(q, seed_radius=seed_r, stats=st2)
@@ -652,8 +649,7 @@ def main():
                    "loss_first_last": [float(losses[0]), float(losses[-1])],
                    "nodes_per_query": st2[3].item() / n, "seed_rel": best_rel, "seed_abs": best_abs,
                    "fallback_fraction": fallback, "margin_sweep": margins, "tau": args.tau,
-                   "unsettled": "re-queued for whole waves of the same launch",
-                   "in_place_ms_per_step": pwall * 1000.0 / max(2, args.steps // 3),
+                   "unsettled": "searched again by the same wave",
                    "exact_seed": {"value": n * max(2, args.steps // 3) / iwall, "nodes_per_query": st3[3].item() / n}}
 
     # other queries (reported beside the headline)
