@@ -549,7 +549,7 @@ int snch_scene_build(snch_scene* s, const snch_build_opts* opts, void* stream)
     for (hipEvent_t& ev : s->build_ev)
         if (!ev)
             SNCH_HIP(hipEventCreate(&ev), "hipEventCreate");
-    if (!s->errors_host)
+    if (s->built && !s->errors_host) // (pinning takes 0.1 ms: not for a scene that is built once)
         SNCH_HIP(hipHostMalloc(reinterpret_cast<void**>(&s->errors_host), 2 * sizeof(uint32_t), hipHostMallocDefault),
                  "snch_scene_build: pinned memory");
     const hipEvent_t e0 = s->build_ev[0], e1 = s->build_ev[1];
@@ -577,7 +577,7 @@ int snch_scene_build(snch_scene* s, const snch_build_opts* opts, void* stream)
     }
     (void)hipEventRecord(e1, st);
     const uint32_t* ew = traversal_error_word();
-    const bool copied = ew && hipMemcpyAsync(s->errors_host, ew, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, st) == hipSuccess;
+    const bool copied = ew && s->errors_host && hipMemcpyAsync(s->errors_host, ew, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, st) == hipSuccess;
     hipError_t es = hipStreamSynchronize(st);
     float ms = 0.0f;
     (void)hipEventElapsedTime(&ms, e0, e1);
