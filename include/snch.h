@@ -253,7 +253,7 @@ typedef struct snch_device_view {
     uint32_t dim;      /* 2 or 3 */
     uint32_t n_leaves; /* primitives of the mesh */
     uint32_t flags;    /* traversal options recorded by the build */
-    uint32_t qbase;    /* stack key quantisation base of the tree */
+    uint32_t qbase;    /* key quantisation base of the tree, for stacks of a user's own */
     const void *tnode, *tcone, *tleaf, *tedge, *nbox, *ncone; /* float4 records */
     const void *V;     /* vertices, float4 */
     const int32_t *F;  /* the mesh's primitives' vertex indices into V */

@@ -58,7 +58,7 @@ constexpr uint32_t TREE_RUNS = 2u;      // children may be leaf runs (built with
 struct TreeView {
     uint32_t n_leaves;
     uint32_t flags;
-    uint32_t qbase; // traversal-stack key quantisation base (bits >> 20 of D^2, less 247)
+    uint32_t qbase; // bits >> 20 of the squared scene diagonal, less 247 (part of the device view; no search here uses it)
     uint32_t pad_;
     const float4* __restrict__ tnode;
     const float4* __restrict__ tcone;
