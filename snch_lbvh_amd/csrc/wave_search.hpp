@@ -77,7 +77,11 @@ __device__ __forceinline__ void flush_counts(const Counts& c, unsigned long long
 // first decides.  So the pool prunes with bounds widened by more than that
 // rounding, which leaves no such candidate out, and where a hidden leaf has
 // the smallest distance the lane repeats the search alone, from the widened
-// bound (a few dozen nodes).
+// bound (a few dozen nodes).  Closest point also bounds an answer by the boxes'
+// minmaxdists, and there a leaf can be too far as well: the distance computed
+// for a sliver or a degenerate triangle may be any multiple of the true one, or
+// NaN, so that nothing within its box's minmaxdist is found.  A lane whose
+// bound ended below its answer's own therefore searches alone too (cp_wave).
 constexpr uint32_t CP_ADD = 20, SIL_ADD = 32;
 constexpr uint32_t CP_LEAF_RUN = 64, SIL_LEAF_RUN = 40; // leaves that are worth a step of the wave
 constexpr uint32_t LEAF_CAP = 64 + 64; // buffer entries: below a run's before a step, which adds at most 64
@@ -151,6 +155,18 @@ __device__ __forceinline__ float widened(float d, v3 p, float scale)
     const float delta = (DIM == 3 ? 5e-7f : 2.0f * BVH_OFFSET) +
                         1e-6f * fmx(scale, fmx(dm::fabs_(p.x), fmx(dm::fabs_(p.y), dm::fabs_(p.z))));
     const float u = d * 1.000002f + delta;
+    return u * u;
+}
+// the same by half as much: more than the rounding of a distance still (random
+// slivers and needles, 3e8 queries at 1e-6 to 1e4 times their size: no leaf is
+// hidden deeper), and less than that of a minmaxdist that equals the answer's
+// distance (1.5 % of the queries beside a rough mesh) widened in full
+template <int DIM>
+__device__ __forceinline__ float half_widened(float d, v3 p, float scale)
+{
+    const float delta = (DIM == 3 ? 2.5e-7f : BVH_OFFSET) +
+                        0.5e-6f * fmx(scale, fmx(dm::fabs_(p.x), fmx(dm::fabs_(p.y), dm::fabs_(p.z))));
+    const float u = d * 1.000001f + delta;
     return u * u;
 }
 __device__ __forceinline__ float scene_scale(const TreeView& t)
@@ -313,7 +329,10 @@ __device__ __forceinline__ uint32_t cp_leaves(const TreeView& t, WaveLds& W, uin
 // by the whole wave.  Every box has geometry on (in 2D, within BVH_OFFSET of)
 // each of its faces, so its minmaxdist bounds the answer from above: besides
 // the reference's test against the sibling (query.cuh:279, :297) it lowers
-// the query's bound before any leaf is reached.
+// the query's bound before any leaf is reached.  Where a box's leaves are farther
+// than it promises (slivers), the bound has passed over leaves that the answer
+// may be among: a query that ends with its bound below its answer, or without
+// an answer, is searched alone.
 template <bool STATS, int DIM>
 __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds& W, Counts& cnt, bool& overflow)
 {
@@ -396,15 +415,22 @@ __device__ __forceinline__ void cp_wave(const TreeView& t, uint32_t nq, WaveLds&
         }
     }
     // the pool is empty: its memory holds the stacks of the lone searches
-    float d = F_INF;
+    float d = F_INF, w = F_INF;
     uint32_t id = INVALID;
-    bool alone = lane < nq && unpack_best(W.best[lane], d, id);
+    bool alone = false;
+    if (lane < nq) {
+        const v3 p = W.point(lane);
+        const bool hidden = unpack_best(W.best[lane], d, id);
+        const float h = HwMath::sqrt(d);
+        alone = hidden || id == INVALID || __uint_as_float(W.bound[lane]) < half_widened<DIM>(h, p, scale);
+        if (id != INVALID)
+            w = widened<DIM>(HwMath::sqrt(widened<DIM>(h, p, scale)), p, scale);
+    }
     for (uint64_t todo = __ballot(alone); todo; todo = __ballot(alone)) {
         const uint32_t r = rank_in(todo);
         if (alone && r < W.cap / 128u) {
             const v3 p = W.point(lane);
-            lane_nearest<DIM>(t, p, widened<DIM>(HwMath::sqrt(__uint_as_float(W.bound[lane])), p, scale),
-                              W.pool + 128 * r, d, id);
+            lane_nearest<DIM>(t, p, w, W.pool + 128 * r, d, id);
             W.best[lane] = pack_best(d, id);
             alone = false;
         }
