@@ -592,12 +592,15 @@ int snch_scene_build(snch_scene* s, const snch_build_opts* opts, void* stream)
         return hip_fail(e, "snch_scene_build");
     if (es != hipSuccess)
         return hip_fail(es, "snch_scene_build: synchronize");
+    // memory holds this build's tree, also where the error words (which may be
+    // another call's) make the call fail: a scene built before answers from it,
+    // so its views say which leaf runs and radii it has
+    s->build_flags = flags;
+    ++s->build_gen;
+    SNCH_HIP(refresh_views(s, leaf), "snch_scene_build: views");
     if (const int rc = check_device_errors("snch_scene_build", copied ? s->errors_host : nullptr))
         return rc;
-    s->build_flags = flags;
-    SNCH_HIP(refresh_views(s, leaf), "snch_scene_build: views");
     s->built = true;
-    ++s->build_gen;
     s->last_build_ms = ms;
     return SNCH_OK;
 }
