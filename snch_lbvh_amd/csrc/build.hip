@@ -434,11 +434,12 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
                         cmin = smin(cmin, clamp11(dot3(r.axis, nn[k][jj])));
                 }
                 r.half_angle = smax(0.0f, dm::acosf_(cmin));
-                // the owned edges end in the triangle's vertices
+                // the owned edges end in the triangle's vertices, within the radius
                 const float h0 = dot3(r.axis, sub(p0, c)), h1 = dot3(r.axis, sub(p1, c)), h2 = dot3(r.axis, sub(p2, c));
                 const float m = smax(smax(dm::fabs_(c.x), dm::fabs_(c.y)), dm::fabs_(c.z)) + r.radius;
                 if (conservative)
-                    slab = pack_slab(fmn(h0, fmn(h1, h2)), fmx(h0, fmx(h1, h2)), r.radius, 1e-6f * m);
+                    slab = pack_slab(fmx(fmn(h0, fmn(h1, h2)), -r.radius), fmn(fmx(h0, fmx(h1, h2)), r.radius),
+                                     r.radius, 1e-6f * m);
             }
         }
         // the leaf record: box and cone in three float4

@@ -272,10 +272,12 @@ SNCH_HD bool cone_overlap_fast(v3 axis, float half_angle, float sin_ha, float co
     return av * il * h <= sin_ha * s + cos_ha * d + tol;
 }
 
-// The extent of a cone's owned edges along its axis, relative to the centre
-// its radius is measured from: the middle and half width of an interval, in 16
-// bits each, as fractions of the radius (which bounds the extent: that whole
-// interval is SLAB_ALL).  `slack` covers the rounding of lo and hi; the square
+// The extent of a cone's owned edges along its axis, relative to the centre of
+// its box: the middle and half width of an interval, in 16 bits each, as
+// fractions of the cone's radius; SLAB_ALL where that cannot hold them (all of
+// the box).  The radius is only the unit: it does not bound the edges, since a
+// cone whose sibling owns no edges keeps its radius while the box and its centre
+// change.  `slack` covers the rounding of lo and hi; the square
 // roots and reciprocals (AM) need not be correctly rounded, their errors are
 // far below the 1e-5 of the radius added here.
 constexpr uint32_t SLAB_ALL = 0xFFFF0000u;
@@ -283,32 +285,33 @@ constexpr float SLAB_MAX_ANGLE = 0.75f; // wider cones keep SLAB_ALL: their test
 template <class AM = HwMath>
 SNCH_HD uint32_t pack_slab(float lo, float hi, float radius, float slack)
 {
-    lo = fmx(lo, -radius);
-    hi = fmn(hi, radius);
     const float inv = AM::rcp(radius);
-    const float m = (float)(int)(0.5f * (lo + hi) * inv * 32767.0f);
+    const float m = (float)(int)fmn(fmx(0.5f * (lo + hi) * inv, -1.0f) * 32767.0f, 32767.0f);
     const float mid = m * (radius * (1.0f / 32767.0f));
     const float h = (fmx(hi - mid, mid - lo) + slack) * inv * 65535.0f + 2.0f; // 2: more than 1e-5 of the radius
     return hi >= lo && radius > 1e-30f && h < 65535.0f ? ((uint32_t)h << 16) | ((uint32_t)(int)m & 0xFFFFu) : SLAB_ALL;
 }
-SNCH_HD void unpack_slab(uint32_t w, float radius, float& mid, float& half)
+// reach: the distance from the box's centre to its corners
+SNCH_HD void unpack_slab(uint32_t w, float radius, float reach, float& mid, float& half)
 {
-    mid = (float)(int16_t)(w & 0xFFFFu) * (radius * (1.0f / 32767.0f));
-    half = (float)(w >> 16) * (radius * (1.0f / 65535.0f));
+    const bool all = w >= SLAB_ALL;
+    mid = all ? 0.0f : (float)(int16_t)(w & 0xFFFFu) * (radius * (1.0f / 32767.0f));
+    half = all ? reach : (float)(w >> 16) * (radius * (1.0f / 65535.0f));
 }
 // the interval along `axis`, from centre `c`, of a child's edges: the child's
-// box and, when its axis has unit length, its slab and radius
+// box and, when its axis has unit length, its slab and its box's reach
 template <class AM = HwMath>
 SNCH_HD void slab_child(const cone3& k, uint32_t slab, const box3& kb, v3 axis, v3 c, float& lo, float& hi)
 {
     const v3 kc = box_centroid(kb);
     const float at = dot3(axis, mk(kc.x - c.x, kc.y - c.y, kc.z - c.z));
-    const float w = dot3(cabs3(axis), mk(kb.hi.x - kc.x, kb.hi.y - kc.y, kb.hi.z - kc.z));
+    const v3 ext = sub(kb.hi, kc);
+    const float w = dot3(cabs3(axis), ext), reach = AM::sqrt(sqlen3(ext));
     const float ct = dot3(axis, k.axis), st = AM::sqrt(sqlen3(cross3(axis, k.axis)));
     float mid, half;
-    unpack_slab(slab, k.radius, mid, half);
+    unpack_slab(slab, k.radius, reach, mid, half);
     const bool unit = dm::fabs_(sqlen3(k.axis) - 1.0f) < 1e-5f;
-    const float m = ct * mid, x = unit ? dm::fabs_(ct) * half + st * k.radius : F_INF;
+    const float m = ct * mid, x = unit ? dm::fabs_(ct) * half + st * reach : F_INF;
     const bool valid = cone_valid(k.half_angle); // else it owns no edges
     lo = valid ? fmn(lo, at + fmx(-w, m - x)) : lo;
     hi = valid ? fmx(hi, at + fmn(w, m + x)) : hi;
@@ -344,11 +347,11 @@ SNCH_HD bool cone_slab_clear(v3 axis, float half_angle, float sin_ha, float cos_
 {
     const v3 c = box_centroid(b);
     const v3 v = mk(c.x - o.x, c.y - o.y, c.z - o.z);
-    const float l2 = dot3(v, v), s = dot3(axis, v);
+    const float l2 = dot3(v, v), s = dot3(axis, v), reach = AM::sqrt(sqlen3(sub(b.hi, c)));
     float mid, half;
-    unpack_slab(slab, radius, mid, half);
-    const float h = dm::fabs_(s + mid) - half, q = AM::sqrt(fmx(l2 - s * s, 0.0f)) + radius;
-    return half_angle < F_PI_2 && cos_ha * h - sin_ha * q > 1.05e-3f + 2e-3f * (AM::sqrt(l2) + radius);
+    unpack_slab(slab, radius, reach, mid, half);
+    const float h = dm::fabs_(s + mid) - half, q = AM::sqrt(fmx(l2 - s * s, 0.0f)) + reach;
+    return half_angle < F_PI_2 && cos_ha * h - sin_ha * q > 1.05e-3f + 2e-3f * (AM::sqrt(l2) + reach);
 }
 
 // Rodrigues rotation (cone.cuh:288-302).  When the axes are (anti)parallel the
