@@ -425,13 +425,15 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
                 // increases over [-1, 1] (checked for every float), so the
                 // maximum of the angles is the angle of the smallest cosine,
                 // bit for bit, for one arccos instead of up to six
-                float cmin = 1.0f;
+                float cmin = 1.0f, smax2 = 0.0f; // and the largest squared sine
 #pragma unroll
                 for (uint32_t k = 0; k < 3; ++k) {
                     if (k >= my)
                         break;
-                    for (int jj = 0; jj < 2; ++jj)
+                    for (int jj = 0; jj < 2; ++jj) {
                         cmin = smin(cmin, clamp11(dot3(r.axis, nn[k][jj])));
+                        smax2 = smax(smax2, sqlen3(cross3(r.axis, nn[k][jj])));
+                    }
                 }
                 r.half_angle = smax(0.0f, dm::acosf_(cmin));
                 // the owned edges end in the triangle's vertices, within the radius
@@ -439,7 +441,8 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
                 const float m = smax(smax(dm::fabs_(c.x), dm::fabs_(c.y)), dm::fabs_(c.z)) + r.radius;
                 if (conservative)
                     slab = pack_slab(fmx(fmn(h0, fmn(h1, h2)), -r.radius), fmn(fmx(h0, fmx(h1, h2)), r.radius),
-                                     r.radius, 1e-6f * m);
+                                     r.radius, 1e-6f * m,
+                                     smax2 < 0.09f ? excess_units(asin_bound(HwMath::sqrt(smax2)) - r.half_angle + 1e-6f) : 0u);
             }
         }
         // the leaf record: box and cone in three float4

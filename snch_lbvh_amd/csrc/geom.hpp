@@ -273,48 +273,74 @@ SNCH_HD bool cone_overlap_fast(v3 axis, float half_angle, float sin_ha, float co
 }
 
 // The extent of a cone's owned edges along its axis, relative to the centre of
-// its box: the middle and half width of an interval, in 16 bits each, as
-// fractions of the cone's radius; SLAB_ALL where that cannot hold them (all of
-// the box).  The radius is only the unit: it does not bound the edges, since a
-// cone whose sibling owns no edges keeps its radius while the box and its centre
-// change.  `slack` covers the rounding of lo and hi; the square
+// its box: the middle and half width of an interval, in 13 bits each (bits 0 and
+// 19 up), as fractions of the cone's radius; SLAB_ALL where that cannot hold
+// them (all of the box).  The radius is only the unit: it does not bound the
+// edges, since a cone whose sibling owns no edges keeps its radius while the box
+// and its centre change.  `slack` covers the rounding of lo and hi; the square
 // roots and reciprocals (AM) need not be correctly rounded, their errors are
-// far below the 1e-5 of the radius added here.
-constexpr uint32_t SLAB_ALL = 0xFFFF0000u;
+// far below the 1e-4 of the radius added here.
+// Bits 13 to 18: by how much the edges' face normals may lie outside the cone's
+// half angle, in SLAB_UNIT radians; SLAB_LOST: too far.  Half angles and merges
+// take small angles from the arccos of a rounded cosine, which loses up to 7e-4
+// each time, and a chain of merges adds that up (a smooth patch of 2^18 leaves:
+// 1.3e-3; 2.3e-3 after seven merges that each tilt by 3e-4).
+constexpr uint32_t SLAB_ALL = 0xFFF80000u, SLAB_LOST = 63u;
+constexpr float SLAB_UNIT = 1e-4f;
 constexpr float SLAB_MAX_ANGLE = 0.75f; // wider cones keep SLAB_ALL: their test hardly ever holds
 template <class AM = HwMath>
-SNCH_HD uint32_t pack_slab(float lo, float hi, float radius, float slack)
+SNCH_HD uint32_t pack_slab(float lo, float hi, float radius, float slack, uint32_t excess = 0u)
 {
     const float inv = AM::rcp(radius);
-    const float m = (float)(int)fmn(fmx(0.5f * (lo + hi) * inv, -1.0f) * 32767.0f, 32767.0f);
-    const float mid = m * (radius * (1.0f / 32767.0f));
-    const float h = (fmx(hi - mid, mid - lo) + slack) * inv * 65535.0f + 2.0f; // 2: more than 1e-5 of the radius
-    return hi >= lo && radius > 1e-30f && h < 65535.0f ? ((uint32_t)h << 16) | ((uint32_t)(int)m & 0xFFFFu) : SLAB_ALL;
+    const float m = (float)(int)fmn(fmx(0.5f * (lo + hi) * inv, -1.0f) * 4095.0f, 4095.0f);
+    const float mid = m * (radius * (1.0f / 4095.0f));
+    const float h = (fmx(hi - mid, mid - lo) + slack) * inv * 8191.0f + 2.0f; // 2: more than 1e-4 of the radius
+    return (hi >= lo && radius > 1e-30f && h < 8191.0f ? ((uint32_t)h << 19) | ((uint32_t)(int)m & 0x1FFFu) : SLAB_ALL) |
+           excess << 13;
 }
 // reach: the distance from the box's centre to its corners
 SNCH_HD void unpack_slab(uint32_t w, float radius, float reach, float& mid, float& half)
 {
     const bool all = w >= SLAB_ALL;
-    mid = all ? 0.0f : (float)(int16_t)(w & 0xFFFFu) * (radius * (1.0f / 32767.0f));
-    half = all ? reach : (float)(w >> 16) * (radius * (1.0f / 65535.0f));
+    mid = all ? 0.0f : (float)((int32_t)(w << 19) >> 19) * (radius * (1.0f / 4095.0f));
+    half = all ? reach : (float)(w >> 19) * (radius * (1.0f / 8191.0f));
 }
-// the interval along `axis`, from centre `c`, of a child's edges: the child's
-// box and, when its axis has unit length, its slab and its box's reach
+SNCH_HD uint32_t slab_excess(uint32_t w) { return (w >> 13) & SLAB_LOST; }
+// an excess of e radians, in units (rounded up).  Below 5e-6: none, the margin of
+// cone_slab_clear covers 64 levels of that
+SNCH_HD uint32_t excess_units(float e)
+{
+    return e <= 5e-6f ? 0u : e < SLAB_UNIT * (SLAB_LOST - 1u) ? (uint32_t)(e * (1.0f / SLAB_UNIT)) + 1u : SLAB_LOST;
+}
+// arcsine of 0 <= x < 0.3, at most 2e-6 too large
+SNCH_HD float asin_bound(float x)
+{
+    const float x2 = x * x;
+    return x * (1.0f + x2 * (0.16666667f + x2 * (0.075f + 0.056f * x2)));
+}
+// A child in a merged cone `r` with box centre `c`: its box and, when its axis
+// has unit length, its slab and its box's reach give the interval of its edges
+// along r's axis; the sine of the angle between the axes gives its excess there.
+// (An angle above 0.3 is as exact as its cosine: its error is left to the caller.)
 template <class AM = HwMath>
-SNCH_HD void slab_child(const cone3& k, uint32_t slab, const box3& kb, v3 axis, v3 c, float& lo, float& hi)
+SNCH_HD void slab_child(const cone3& k, uint32_t slab, const box3& kb, const cone3& r, v3 c, float off_unit, float& lo,
+                        float& hi, uint32_t& excess)
 {
     const v3 kc = box_centroid(kb);
-    const float at = dot3(axis, mk(kc.x - c.x, kc.y - c.y, kc.z - c.z));
+    const float at = dot3(r.axis, mk(kc.x - c.x, kc.y - c.y, kc.z - c.z));
     const v3 ext = sub(kb.hi, kc);
-    const float w = dot3(cabs3(axis), ext), reach = AM::sqrt(sqlen3(ext));
-    const float ct = dot3(axis, k.axis), st = AM::sqrt(sqlen3(cross3(axis, k.axis)));
+    const float w = dot3(cabs3(r.axis), ext), reach = AM::sqrt(sqlen3(ext));
+    const float ct = dot3(r.axis, k.axis), st = AM::sqrt(sqlen3(cross3(r.axis, k.axis)));
     float mid, half;
     unpack_slab(slab, k.radius, reach, mid, half);
-    const bool unit = dm::fabs_(sqlen3(k.axis) - 1.0f) < 1e-5f;
+    const bool unit = off_unit < 1e-5f;
     const float m = ct * mid, x = unit ? dm::fabs_(ct) * half + st * reach : F_INF;
     const bool valid = cone_valid(k.half_angle); // else it owns no edges
     lo = valid ? fmn(lo, at + fmx(-w, m - x)) : lo;
     hi = valid ? fmx(hi, at + fmn(w, m + x)) : hi;
+    const float add = st < 0.3f ? asin_bound(st) + (k.half_angle - r.half_angle) + 1e-6f : (2e-7f + off_unit) * 3.4f;
+    const uint32_t e = unit ? slab_excess(slab) + excess_units(add) : SLAB_LOST;
+    excess = valid && e > excess ? e : excess;
 }
 // the slab of a merged cone r of box b
 template <class AM = HwMath>
@@ -323,24 +349,32 @@ SNCH_HD uint32_t slab_merge(const cone3& r, const box3& b, const cone3& k0, uint
 {
     const v3 c = box_centroid(b);
     float lo = F_INF, hi = -F_INF;
-    slab_child<AM>(k0, s0, b0, r.axis, c, lo, hi);
-    slab_child<AM>(k1, s1, b1, r.axis, c, lo, hi);
+    uint32_t excess = 0u;
+    // how far the axes are from unit length (one that belongs to no edges does not matter)
+    auto off = [](const cone3& k) { return cone_valid(k.half_angle) ? dm::fabs_(sqlen3(k.axis) - 1.0f) : 0.0f; };
+    const float off_unit = fmx(off(r), fmx(off(k0), off(k1)));
+    slab_child<AM>(k0, s0, b0, r, c, off_unit, lo, hi, excess);
+    slab_child<AM>(k1, s1, b1, r, c, off_unit, lo, hi, excess);
     const float m = fmx(fmx(fmx(dm::fabs_(b.lo.x), dm::fabs_(b.hi.x)), fmx(dm::fabs_(b.lo.y), dm::fabs_(b.hi.y))),
                         fmx(dm::fabs_(b.lo.z), dm::fabs_(b.hi.z)));
-    return pack_slab<AM>(lo, hi, r.radius, 1e-6f * m);
+    return pack_slab<AM>(lo, hi, r.radius, 1e-6f * m, excess < SLAB_LOST ? excess : SLAB_LOST);
 }
 // No edge of the cone can pass the silhouette predicate seen from o, because
 // every point x of its edges lies on one side of all its face planes by more
 // than that predicate's tolerance: with a = the axis, h = the least |a.(x - o)|
-// over the slab and q the greatest distance of x from the axis through o,
-// |n.(x - o)| >= cos(ha) h - sin(ha) q for every normal n of the cone.  The
-// predicate treats |n.(x - o)| <= 1e-3 as grazing, and distances up to 1e-3
-// apart: hence the margin, and 2e-3 of the distance for the rounding of these
-// sums and of the cone itself (a normal may lie up to 8e-4 outside its half
-// angle, which is the arccos of a cosine rounded near 1).  The view-cone test (cone_overlap) takes all of the bounding sphere for the
-// edges; a patch of surface is a thin slab of it.  On the 1M-triangle torus
-// 898 -> 540 nodes per query, 2^22 queries 36 -> 26 ms, walk on stars 64 -> 49
-// ms; rough meshes (noise above the edge length) gain nothing and pay about 2 %.
+// over the slab, q the greatest distance of x from the axis through o and t the
+// half angle with its excess, |n.(x - o)| >= cos(t) h - sin(t) q for every
+// normal n.  The predicate treats |n.(x - o)| <= 1e-3 as grazing, and distances
+// up to 1e-3 apart: hence the margin.  An excess e takes at most
+// sqrt(h^2 + q^2) e <= 1.42 (l + reach) e away; 5e-4 more of that length covers
+// the excess that is not counted (64 levels of 5e-6) and the rounding of these
+// sums.  The view-cone test (cone_overlap) takes all of the bounding sphere for
+// the edges; a patch of surface is a thin slab of it.  On the 1M-triangle torus
+// 808 -> 495 nodes per query, 2^22 queries 34.0 -> 20.7 ms, walk on stars 61 ->
+// 46 ms (2^17 walks); rough meshes (noise above the edge length) gain nothing and
+// pay about 2 %.  One margin for all cones, without the excess of each: 2e-3 of
+// the length (too little for a chain of tilted merges) 22.0 ms, 4e-3 23.2, 8e-3
+// 24.1, 2e-2 27.8.
 template <class AM = HwMath>
 SNCH_HD bool cone_slab_clear(v3 axis, float half_angle, float sin_ha, float cos_ha, float radius, uint32_t slab, v3 o,
                              const box3& b)
@@ -348,10 +382,12 @@ SNCH_HD bool cone_slab_clear(v3 axis, float half_angle, float sin_ha, float cos_
     const v3 c = box_centroid(b);
     const v3 v = mk(c.x - o.x, c.y - o.y, c.z - o.z);
     const float l2 = dot3(v, v), s = dot3(axis, v), reach = AM::sqrt(sqlen3(sub(b.hi, c)));
+    const uint32_t e = slab_excess(slab);
     float mid, half;
     unpack_slab(slab, radius, reach, mid, half);
     const float h = dm::fabs_(s + mid) - half, q = AM::sqrt(fmx(l2 - s * s, 0.0f)) + reach;
-    return half_angle < F_PI_2 && cos_ha * h - sin_ha * q > 1.05e-3f + 2e-3f * (AM::sqrt(l2) + reach);
+    return half_angle < F_PI_2 && e < SLAB_LOST &&
+           cos_ha * h - sin_ha * q > 1.05e-3f + (5e-4f + 1.42f * SLAB_UNIT * (float)e) * (AM::sqrt(l2) + reach);
 }
 
 // Rodrigues rotation (cone.cuh:288-302).  When the axes are (anti)parallel the
