@@ -275,6 +275,20 @@ struct LeafEdgeLds {
     uint32_t faces[64];
 };
 
+constexpr uint32_t NO_SLAB = 0xFFFFFFFFu; // of a leaf's excess: its cone is wide or empty
+
+// the slab of a leaf's cone: the owned edges end in the triangle's vertices and
+// lie within the cone's radius of the centre c of its box
+__device__ __forceinline__ uint32_t leaf_slab(const cone3& r, v3 c, v3 p0, v3 p1, v3 p2, uint32_t excess)
+{
+    if (excess == NO_SLAB)
+        return SLAB_ALL;
+    const float h0 = dot3(r.axis, sub(p0, c)), h1 = dot3(r.axis, sub(p1, c)), h2 = dot3(r.axis, sub(p2, c));
+    const float m = fmx(fmx(dm::fabs_(c.x), dm::fabs_(c.y)), dm::fabs_(c.z)) + r.radius;
+    return pack_slab(fmx(fmn(h0, fmn(h1, h2)), -r.radius), fmn(fmx(h0, fmx(h1, h2)), r.radius), r.radius, 1e-6f * m,
+                     excess);
+}
+
 // Leaf box and leaf cone of each triangle (scene.cuh:870-961) and the packed
 // silhouette-edge records.  A triangle owns 0..3 edges; rather than looping
 // over them per lane (three divergent iterations per wave), the wave lists
@@ -300,11 +314,11 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
     b.lo = mk(F_INF, F_INF, F_INF);
     b.hi = mk(-F_INF, -F_INF, -F_INF);
     uint32_t e0 = 0, my = 0;
-    v3 c = mk(0.0f, 0.0f, 0.0f), p0 = c, p1 = c, p2 = c;
+    v3 c = mk(0.0f, 0.0f, 0.0f);
+    float edge2 = 0.0f;
     if (i < nF) {
-        p0 = ld3(V, F[3 * i]);
-        p1 = ld3(V, F[3 * i + 1]);
-        p2 = ld3(V, F[3 * i + 2]);
+        const v3 p0 = ld3(V, F[3 * i]), p1 = ld3(V, F[3 * i + 1]), p2 = ld3(V, F[3 * i + 2]);
+        edge2 = fmx(sqlen3(sub(p1, p0)), fmx(sqlen3(sub(p2, p1)), sqlen3(sub(p0, p2))));
         b = box_of_point(p0);
         box_expand(b, p1);
         box_expand(b, p2);
@@ -325,7 +339,7 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
     r.axis = mk(0.0f, 0.0f, 0.0f);
     r.half_angle = F_PI;
     r.radius = 0.0f;
-    uint32_t slab = SLAB_ALL;
+    uint32_t excess = NO_SLAB; // of the cone's slab, which k_refit computes where it has the vertices
     bool all_two = true;
     v3 nn[3][2];
 #pragma unroll
@@ -436,22 +450,16 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
                     }
                 }
                 r.half_angle = smax(0.0f, dm::acosf_(cmin));
-                // the owned edges end in the triangle's vertices, within the radius
-                const float h0 = dot3(r.axis, sub(p0, c)), h1 = dot3(r.axis, sub(p1, c)), h2 = dot3(r.axis, sub(p2, c));
-                const float m = smax(smax(dm::fabs_(c.x), dm::fabs_(c.y)), dm::fabs_(c.z)) + r.radius;
                 if (conservative)
-                    slab = pack_slab(fmx(fmn(h0, fmn(h1, h2)), -r.radius), fmn(fmx(h0, fmx(h1, h2)), r.radius),
-                                     r.radius, 1e-6f * m,
-                                     smax2 < 0.09f ? excess_units(asin_bound(HwMath::sqrt(smax2)) - r.half_angle + 1e-6f) : 0u);
+                    excess = smax2 < 0.09f ? excess_units(asin_bound(HwMath::sqrt(smax2)) - r.half_angle + 1e-6f) : 0u;
             }
         }
         // the leaf record: box and cone in three float4
         leafrec[3 * i] = make_float4(b.lo.x, b.lo.y, b.lo.z, b.hi.x);
         leafrec[3 * i + 1] = make_float4(b.hi.y, b.hi.z, r.axis.x, r.axis.y);
-        leafrec[3 * i + 2] = make_float4(r.axis.z, r.half_angle, r.radius, __uint_as_float(slab));
+        leafrec[3 * i + 2] = make_float4(r.axis.z, r.half_angle, r.radius, __uint_as_float(excess));
     }
     // scene AABB of the primitive's mesh, and its longest edge
-    const float edge2 = fmx(sqlen3(sub(p1, p0)), fmx(sqlen3(sub(p2, p1)), sqlen3(sub(p0, p2))));
     float v[7] = {b.lo.x, b.lo.y, b.lo.z, b.hi.x, b.hi.y, b.hi.z, edge2};
     const int slot_of[7] = {0, 1, 2, 3, 4, 5, 7};
     reduce_scene_box<7, 3>(v, mesh, i < nF, scene_bits, slot_of, part);
@@ -911,52 +919,56 @@ __device__ __forceinline__ uint32_t child_ref(const MeshIds& id, uint32_t node, 
     return cnt <= leaf_size ? ref | (cnt << RUN_SHIFT) : ref;
 }
 
-// the parent box and cone of two children (bvh.cuh:520-604), and the records
-// of internal node p
+// the parent cone of two children (bvh.cuh:520-604) with the merged box pb
 template <int DIM>
-__device__ __forceinline__ void refit_write(const MeshIds& id, uint32_t p, uint2 ch, const box3& lb, const box3& rb,
-                                            const cone3& lc, const cone3& rc, uint32_t ls, uint32_t rs, int conservative,
-                                            const uint2* __restrict__ range, uint32_t leaf_size, box3& pb,
-                                            cone3& pc, uint32_t& ps, float4* nbox, float4* ncone, float4* __restrict__ tnode,
-                                            float4* __restrict__ tcone, bool own = true)
+__device__ __forceinline__ cone3 node_cone(const box3& lb, const box3& rb, const box3& pb, const cone3& lc,
+                                           const cone3& rc, int conservative)
 {
-    pb = box_merge(lb, rb);
-    pc = DIM == 3 ? cone_merge(lc, rc, box_centroid(lb), box_centroid(rb), box_centroid(pb), conservative != 0)
-                  : cone_merge2d(lc, rc, box_centroid(lb), box_centroid(rb), box_centroid(pb), conservative != 0);
-    // 16 us of the 1M-triangle build's 150 in k_refit; wide cones, which are
-    // most of the levels above the cuts, are left out (5 us)
-    ps = SLAB_ALL;
-    if (DIM == 3 && conservative && pc.half_angle < SLAB_MAX_ANGLE)
-        ps = slab_merge(pc, pb, lc, ls, lb, rc, rs, rb);
-    if (own) { // the node's own box and cone in the reference layout (else they live in its parent's record)
-        nbox[2 * p] = make_float4(pb.lo.x, pb.lo.y, pb.lo.z, 0.0f);
-        nbox[2 * p + 1] = make_float4(pb.hi.x, pb.hi.y, pb.hi.z, 0.0f);
-        ncone[2 * p] = make_float4(pc.axis.x, pc.axis.y, pc.axis.z, pc.half_angle);
-        ncone[2 * p + 1] = make_float4(pc.radius, __uint_as_float(ps), 0.0f, 0.0f);
-    }
+    return DIM == 3 ? cone_merge(lc, rc, box_centroid(lb), box_centroid(rb), box_centroid(pb), conservative != 0)
+                    : cone_merge2d(lc, rc, box_centroid(lb), box_centroid(rb), box_centroid(pb), conservative != 0);
+}
+// its slab; wide cones, most of the levels above the cuts, have none
+template <int DIM>
+__device__ __forceinline__ uint32_t node_slab(const cone3& pc, const box3& pb, const cone3& lc, uint32_t ls,
+                                              const box3& lb, const cone3& rc, uint32_t rs, const box3& rb,
+                                              int conservative)
+{
+    return DIM == 3 && conservative && pc.half_angle < SLAB_MAX_ANGLE ? slab_merge(pc, pb, lc, ls, lb, rc, rs, rb)
+                                                                      : SLAB_ALL;
+}
+// the traversal records of internal node p: its children's boxes and references
+__device__ __forceinline__ void write_boxes(const MeshIds& id, uint32_t p, uint2 ch, const box3& lb, const box3& rb,
+                                            const uint2* __restrict__ range, uint32_t leaf_size,
+                                            float4* __restrict__ tnode)
+{
     const uint32_t r = p - id.off; // internal record: (off - m) + (p - nb)
     tnode[4 * r + 0] = make_float4(lb.lo.x, lb.lo.y, lb.lo.z, lb.hi.x);
     tnode[4 * r + 1] = make_float4(lb.hi.y, lb.hi.z, __uint_as_float(child_ref(id, ch.x, range, leaf_size)), 0.0f);
     tnode[4 * r + 2] = make_float4(rb.lo.x, rb.lo.y, rb.lo.z, rb.hi.x);
     tnode[4 * r + 3] = make_float4(rb.hi.y, rb.hi.z, __uint_as_float(child_ref(id, ch.y, range, leaf_size)), 0.0f);
-    tcone[4 * r + 0] = make_float4(lc.axis.x, lc.axis.y, lc.axis.z, lc.half_angle);
-    tcone[4 * r + 2] = make_float4(rc.axis.x, rc.axis.y, rc.axis.z, rc.half_angle);
-    // the sines and cosines (the halves before these) are filled by
-    // tcone_trig once the merges are done: off the chain of dependent merges
-    reinterpret_cast<float2*>(tcone)[8 * r + 3] = make_float2(lc.radius, __uint_as_float(ls));
-    reinterpret_cast<float2*>(tcone)[8 * r + 7] = make_float2(rc.radius, __uint_as_float(rs));
 }
-
-// sin and cos of both children's half angles of internal record r, read
-// back from the record
-__device__ __forceinline__ void tcone_trig(float4* __restrict__ tcone, uint32_t r)
+// and, of internal record r, their cones, the sines and cosines of the half
+// angles, and slabs
+__device__ __forceinline__ void write_cones(uint32_t r, const cone3& lc, uint32_t ls, const cone3& rc, uint32_t rs,
+                                            float4* __restrict__ tcone)
 {
-    const float hl = tcone[4 * r + 0].w, hr = tcone[4 * r + 2].w;
-    float ls, lcs, rs, rcs;
-    dm::sincosf_(hl, &ls, &lcs);
-    dm::sincosf_(hr, &rs, &rcs);
-    reinterpret_cast<float2*>(tcone)[8 * r + 2] = make_float2(ls, lcs);
-    reinterpret_cast<float2*>(tcone)[8 * r + 6] = make_float2(rs, rcs);
+    float sn, cs;
+    dm::sincosf_(lc.half_angle, &sn, &cs);
+    tcone[4 * r + 0] = make_float4(lc.axis.x, lc.axis.y, lc.axis.z, lc.half_angle);
+    tcone[4 * r + 1] = make_float4(sn, cs, lc.radius, __uint_as_float(ls));
+    dm::sincosf_(rc.half_angle, &sn, &cs);
+    tcone[4 * r + 2] = make_float4(rc.axis.x, rc.axis.y, rc.axis.z, rc.half_angle);
+    tcone[4 * r + 3] = make_float4(sn, cs, rc.radius, __uint_as_float(rs));
+}
+// a node's own box, cone and slab in the reference layout (for nodes that a
+// later launch reads or that have no parent; others live in their parent's records)
+__device__ __forceinline__ void write_own(uint32_t p, const box3& pb, const cone3& pc, uint32_t slab, float4* nbox,
+                                          float4* ncone)
+{
+    nbox[2 * p] = make_float4(pb.lo.x, pb.lo.y, pb.lo.z, 0.0f);
+    nbox[2 * p + 1] = make_float4(pb.hi.x, pb.hi.y, pb.hi.z, 0.0f);
+    ncone[2 * p] = make_float4(pc.axis.x, pc.axis.y, pc.axis.z, pc.half_angle);
+    ncone[2 * p + 1] = make_float4(pc.radius, __uint_as_float(slab), 0.0f, 0.0f);
 }
 
 // box + cone of live nodes in LDS, structure of arrays over RT slots.  A node
@@ -1079,9 +1091,9 @@ __global__ __launch_bounds__(RB, 6) void k_refit(const float4* __restrict__ V, c
     __shared__ uint16_t queue[RT];
     __shared__ RoundQueue rq;
     __shared__ uint32_t s_cut;
-    // The slabs of the live nodes stay in memory (slabs[first + slot]): a
-    // twelfth row of nd would leave two workgroups per CU (k_refit 199 us at
-    // 1M triangles with cuts of 960 leaves instead, 165 this way)
+    // No row of nd for the slabs: it would leave two workgroups per CU.  Leaves'
+    // slabs are in memory (slabs[sorted position]), and a merged node's takes the
+    // place of its word of lnode.
     const uint32_t t = threadIdx.x;
     const uint32_t count = min(cuts[cut_cap], cut_cap);
     if (t < 3)
@@ -1146,24 +1158,16 @@ __global__ __launch_bounds__(RB, 6) void k_refit(const float4* __restrict__ V, c
             const uint32_t node = D.nb + (D.n - 1) + (j - D.off);
             const float4 r0 = leafrec[3 * orig], r1 = leafrec[3 * orig + 1], r2 = leafrec[3 * orig + 2];
             const float4 b0 = make_float4(r0.x, r0.y, r0.z, 0.0f), b1 = make_float4(r0.w, r1.x, r1.y, 0.0f);
-            const float4 c0 = make_float4(r1.z, r1.w, r2.x, r2.y), c1 = make_float4(r2.z, r2.w, 0.0f, 0.0f);
+            const float4 c0 = make_float4(r1.z, r1.w, r2.x, r2.y), c1 = make_float4(r2.z, 0.0f, 0.0f, 0.0f);
             if (node == root) { // a cut of one leaf; other leaves live in their parents' records
                 nbox[2 * node] = b0;
                 nbox[2 * node + 1] = b1;
                 ncone[2 * node] = c0;
-                ncone[2 * node + 1] = c1;
             }
-            {
-                box3 b;
-                b.lo = mk(b0.x, b0.y, b0.z);
-                b.hi = mk(b1.x, b1.y, b1.z);
-                cone3 cc;
-                cc.axis = mk(c0.x, c0.y, c0.z);
-                cc.half_angle = c0.w;
-                cc.radius = c1.x;
-                slabs[j] = __float_as_uint(r2.w);
-                nd.put(u, b, cc);
-            }
+            const box3 lb{mk(b0.x, b0.y, b0.z), mk(b1.x, b1.y, b1.z)};
+            const cone3 cc{mk(c0.x, c0.y, c0.z), c0.w, c1.x};
+            nd.put(u, lb, cc);
+            uint32_t slab = SLAB_ALL;
             const uint32_t es = estart[orig], ec = estart[orig + 1] - es;
             const uint32_t lo = orig - D.off, les = es - D.eoff;
             if (DIM == 3) {
@@ -1171,49 +1175,85 @@ __global__ __launch_bounds__(RB, 6) void k_refit(const float4* __restrict__ V, c
                 tleaf[3 * j + 0] = make_float4(a.x, a.y, a.z, __uint_as_float(lo));
                 tleaf[3 * j + 1] = make_float4(b.x, b.y, b.z, __uint_as_float(les));
                 tleaf[3 * j + 2] = make_float4(d.x, d.y, d.z, __uint_as_float(ec));
+                slab = leaf_slab(cc, box_centroid(lb), mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), mk(d.x, d.y, d.z),
+                                 __float_as_uint(r2.w));
             } else {
                 const float4 a = V[F[2 * orig]], b = V[F[2 * orig + 1]];
                 tleaf[3 * j + 0] = make_float4(a.x, a.y, 0.0f, __uint_as_float(lo));
                 tleaf[3 * j + 1] = make_float4(b.x, b.y, 0.0f, __uint_as_float(les));
                 tleaf[3 * j + 2] = make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(ec));
             }
+            slabs[j] = slab;
+            if (node == root)
+                ncone[2 * node + 1] = make_float4(c1.x, __uint_as_float(slab), 0.0f, 0.0f);
         }
         // topology, leaf slots and the ready nodes
         uint32_t qs = 0, qe = __syncthreads_or(bad ? 1 : 0) ? 0u : rq.n[0];
+        // Nothing but slabs waits for a merged node's record and slab, so the rounds,
+        // a chain of dependent merges, are kept to the boxes and cones: once the
+        // nodes of a round (never more than those of the round before) fit half of
+        // the threads, the rounds use one half of them in turn, and each thread
+        // writes its node's record (`due`) in the next round, beside the other
+        // half's merges.  1M triangles: k_refit 166 us with slabs merged in the
+        // rounds and sines in a pass after them, 136 this way (181 with the
+        // record read back for the slab instead of kept in registers), 139 before
+        // there were slabs.
+        struct {
+            uint32_t k = INVALID, wd; // local position, and its word of lnode
+            box3 lb;                  // the left child (the right child's slot of nd stays as it is)
+            cone3 lc, pc;
+        } due;
+        auto write_due = [&] {
+            const uint32_t lc = due.wd & 0x7FFu, rc = (due.wd >> 11) & 0x7FFu;
+            const uint2 ch = make_uint2(cut_child_global(id, lc, first), cut_child_global(id, rc, first));
+            const uint32_t p = D.nb + (first + due.k - D.off);
+            // a child's slab: a leaf's is in memory, an internal node's takes its word of lnode
+            auto slab_of = [&](uint32_t c) { return c & (1u << 10) ? slabs[first + (c & 0x3FFu)] : lnode[c]; };
+            const uint32_t lsl = slab_of(lc), rsl = slab_of(rc);
+            box3 rb;
+            cone3 rcone;
+            nd.get(rc & 0x3FFu, rb, rcone);
+            const box3 pb = box_merge(due.lb, rb);
+            const uint32_t ps = node_slab<DIM>(due.pc, pb, due.lc, lsl, due.lb, rcone, rsl, rb, conservative);
+            lnode[due.k] = ps;
+            write_boxes(id, p, ch, due.lb, rb, range, leaf_size, tnode);
+            write_cones(p - id.off, due.lc, lsl, rcone, rsl, tcone);
+            if (p == root)
+                write_own(p, pb, due.pc, ps, nbox, ncone);
+            due.k = INVALID;
+        };
         for (uint32_t round = 1; qs < qe && round < RT; ++round) {
             if (t == 0)
                 rq.n[(round + 1) % 3] = 0u;
-            for (uint32_t i = qs + t; i < qe; i += RB) {
+            const bool halves = qe - qs <= RB / 2;
+            if (due.k != INVALID)
+                write_due();
+            const uint32_t i = qs + (halves && (round & 1u) ? t ^ (RB / 2) : t); // qe - qs <= RT / 2 = RB
+            if (i < qe) {
                 const uint32_t k = queue[i];
-                const uint32_t wd = lnode[k];
-                const uint32_t lc = wd & 0x7FFu, rc = (wd >> 11) & 0x7FFu;
-                const uint32_t ls = wd >> 22, rs = rc & 0x3FFu; // the right child's first leaf is its position
-                const uint2 ch = make_uint2(cut_child_global(id, lc, first), cut_child_global(id, rc, first));
-                box3 lb, rb, pb;
-                cone3 lc3, rc3, pc;
-                // the children's slabs, read while the boxes and cones merge
-                const uint32_t lsl = slabs[first + ls], rsl = slabs[first + rs];
-                uint32_t psl;
-                nd.get(ls, lb, lc3);
-                nd.get(rs, rb, rc3);
-                const uint32_t p = D.nb + (first + k - D.off);
-                refit_write<DIM>(id, p, ch, lb, rb, lc3, rc3, lsl, rsl, conservative, range, leaf_size, pb, pc, psl,
-                                 nbox, ncone, tnode, tcone, p == root);
-                nd.put(ls, pb, pc);
-                slabs[first + ls] = psl;
+                due.k = k;
+                due.wd = lnode[k];
+                const uint32_t ls = due.wd >> 22, rs = (due.wd >> 11) & 0x3FFu; // the right child's first leaf is its position
+                box3 rb;
+                cone3 rc;
+                nd.get(ls, due.lb, due.lc);
+                nd.get(rs, rb, rc);
+                const box3 pb = box_merge(due.lb, rb);
+                due.pc = node_cone<DIM>(due.lb, rb, pb, due.lc, rc, conservative);
+                nd.put(ls, pb, due.pc);
                 const uint32_t kp = lpar[k];
                 if (kp != NO_PARENT && (atomicOr(&larr[kp >> 5], 1u << (kp & 31u)) >> (kp & 31u)) & 1u)
                     rq.push(queue, qe, round, kp);
+                if (!halves)
+                    write_due();
             }
             __syncthreads();
             const uint32_t added = rq.n[round % 3];
             qs = qe;
             qe += added;
         }
-        // every merged node is in queue[0, qe); the barrier above orders its
-        // record's writes before these reads
-        for (uint32_t i = t; i < qe; i += RB)
-            tcone_trig(tcone, D.nb + (first + queue[i] - D.off) - id.off);
+        if (due.k != INVALID)
+            write_due();
         // clear for the next cut (after the barrier that ends this one's rounds)
         if (t < 3)
             rq.n[t] = 0u;
@@ -1256,19 +1296,18 @@ struct SetLds {
     uint16_t* queue;
     float* box;
     uint32_t cap;
-    __device__ __forceinline__ void put(uint32_t k, const box3& b, const cone3& c, uint32_t slab) const
+    __device__ __forceinline__ uint32_t& slab(uint32_t k) const { return reinterpret_cast<uint32_t*>(box)[11 * cap + k]; }
+    __device__ __forceinline__ void put(uint32_t k, const box3& b, const cone3& c) const
     {
         float* v = box + k;
-        v[11 * cap] = __uint_as_float(slab);
         v[0 * cap] = b.lo.x; v[1 * cap] = b.lo.y; v[2 * cap] = b.lo.z;
         v[3 * cap] = b.hi.x; v[4 * cap] = b.hi.y; v[5 * cap] = b.hi.z;
         v[6 * cap] = c.axis.x; v[7 * cap] = c.axis.y; v[8 * cap] = c.axis.z;
         v[9 * cap] = c.half_angle; v[10 * cap] = c.radius;
     }
-    __device__ __forceinline__ void get(uint32_t k, box3& b, cone3& c, uint32_t& slab) const
+    __device__ __forceinline__ void get(uint32_t k, box3& b, cone3& c) const
     {
         const float* v = box + k;
-        slab = __float_as_uint(v[11 * cap]);
         b.lo = mk(v[0 * cap], v[1 * cap], v[2 * cap]);
         b.hi = mk(v[3 * cap], v[4 * cap], v[5 * cap]);
         c.axis = mk(v[6 * cap], v[7 * cap], v[8 * cap]);
@@ -1326,47 +1365,75 @@ __device__ void refit_set(const SetLds& s, uint32_t n, uint32_t lo_thr, uint32_t
             push(0u, 0u, k);
     __syncthreads();
     uint32_t qs = 0, qe = min(rq.n[0], n);
+    // records and slabs one round later, as in k_refit
+    struct {
+        uint32_t k = INVALID; // member
+        box3 lb, rb;
+        cone3 lc, rc, pc;
+    } due;
+    auto write_due = [&] {
+        const uint32_t k = due.k, p = s.node[k], ci = s.cidx[k];
+        const uint2 ch = s.ch[k];
+        const MeshDesc D = desc[min(s.mesh[k], M - 1)];
+        const MeshIds id{D.off, D.n, D.nb};
+        auto slab_of = [&](uint32_t member, uint32_t node) {
+            return BOX_LDS && member != NO_MEMBER ? s.slab(min(member, s.cap - 1)) : __float_as_uint(ncone[2 * node + 1].y);
+        };
+        const uint32_t lsl = slab_of(ci & 0xFFFFu, ch.x), rsl = slab_of(ci >> 16, ch.y);
+        const uint32_t ps = node_slab<DIM>(due.pc, box_merge(due.lb, due.rb), due.lc, lsl, due.lb, due.rc, rsl, due.rb, conservative);
+        if (BOX_LDS) {
+            s.slab(k) = ps;
+            write_own(p, box_merge(due.lb, due.rb), due.pc, ps, nbox, ncone);
+        } else {
+            reinterpret_cast<float*>(ncone + 2 * (size_t)p)[5] = __uint_as_float(ps);
+        }
+        write_boxes(id, p, ch, due.lb, due.rb, range, leaf_size, tnode);
+        write_cones(p - id.off, due.lc, lsl, due.rc, rsl, tcone);
+        due.k = INVALID;
+    };
     for (uint32_t round = 1; qs < qe && round < SET_ROUNDS; ++round) {
         if (t == 0)
             rq.n[(round + 1) % 3] = 0u;
-        for (uint32_t i = qs + t; i < qe; i += NT) {
+        const bool halves = qe - qs <= NT / 2;
+        if (due.k != INVALID)
+            write_due();
+        for (uint32_t i = qs + (halves && (round & 1u) ? t ^ (NT / 2) : t); i < qe; i += NT) {
             const uint32_t k = s.queue[i];
-            const uint32_t p = s.node[k];
             const uint2 ch = s.ch[k];
             const uint32_t ci = s.cidx[k];
-            const MeshDesc D = desc[min(s.mesh[k], M - 1)];
-            const MeshIds id{D.off, D.n, D.nb};
-            box3 lb, rb, pb;
-            cone3 lc, rc, pc;
-            uint32_t lsl, rsl, psl;
+            uint32_t unused;
             if (BOX_LDS && (ci & 0xFFFFu) != NO_MEMBER) {
-                s.get(min(ci & 0xFFFFu, s.cap - 1), lb, lc, lsl);
+                s.get(min(ci & 0xFFFFu, s.cap - 1), due.lb, due.lc);
             } else {
-                lb = ldbox(nbox, ch.x);
-                lc = ldcone(ncone, ch.x, lsl);
+                due.lb = ldbox(nbox, ch.x);
+                due.lc = ldcone(ncone, ch.x, unused);
             }
             if (BOX_LDS && (ci >> 16) != NO_MEMBER) {
-                s.get(min(ci >> 16, s.cap - 1), rb, rc, rsl);
+                s.get(min(ci >> 16, s.cap - 1), due.rb, due.rc);
             } else {
-                rb = ldbox(nbox, ch.y);
-                rc = ldcone(ncone, ch.y, rsl);
+                due.rb = ldbox(nbox, ch.y);
+                due.rc = ldcone(ncone, ch.y, unused);
             }
-            refit_write<DIM>(id, p, ch, lb, rb, lc, rc, lsl, rsl, conservative, range, leaf_size, pb, pc, psl, nbox,
-                             ncone, tnode, tcone);
+            due.k = k;
+            const box3 pb = box_merge(due.lb, due.rb);
+            due.pc = node_cone<DIM>(due.lb, due.rb, pb, due.lc, due.rc, conservative);
             if (BOX_LDS)
-                s.put(k, pb, pc, psl);
+                s.put(k, pb, due.pc);
+            else
+                write_own(s.node[k], pb, due.pc, SLAB_ALL, nbox, ncone);
             const uint32_t pk = s.word[k] >> 16;
             if (pk < n && (atomicSub(&s.word[pk], 1u) & 0xFFFFu) == 1u)
                 push(qe, round, pk);
+            if (!halves)
+                write_due();
         }
         __syncthreads(); // this round's boxes (LDS or memory) precede the next round's reads
         const uint32_t added = rq.n[round % 3];
         qs = qe;
         qe = min(qe + added, n);
     }
-    // the sin and cos of the children's half angles, once every record is written
-    for (uint32_t k = t; k < n; k += NT)
-        tcone_trig(tcone, s.node[k] - desc[min(s.mesh[k], M - 1)].off);
+    if (due.k != INVALID)
+        write_due();
 }
 
 // One workgroup per mid set (a grid-stride loop over the sets), boxes in LDS.
@@ -1478,12 +1545,13 @@ __global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__
             continue;
         for (uint32_t guard = 0; guard < SET_ROUNDS; ++guard) {
             const uint2 ch = child[p];
-            box3 pb;
-            cone3 pc;
-            uint32_t lsl, rsl, psl;
+            uint32_t lsl, rsl;
             const cone3 lc = ldcone(ncone, ch.x, lsl), rc = ldcone(ncone, ch.y, rsl);
-            refit_write<DIM>(id, p, ch, ldbox(nbox, ch.x), ldbox(nbox, ch.y), lc, rc, lsl, rsl, conservative, range,
-                             leaf_size, pb, pc, psl, nbox, ncone, tnode, tcone);
+            const box3 lb = ldbox(nbox, ch.x), rb = ldbox(nbox, ch.y), pb = box_merge(lb, rb);
+            const cone3 pc = node_cone<DIM>(lb, rb, pb, lc, rc, conservative);
+            write_own(p, pb, pc, node_slab<DIM>(pc, pb, lc, lsl, lb, rc, rsl, rb, conservative), nbox, ncone);
+            write_boxes(id, p, ch, lb, rb, range, leaf_size, tnode);
+            write_cones(p - id.off, lc, lsl, rc, rsl, tcone);
             const uint32_t par = parent[p];
             if (par == INVALID || !id.internal(par))
                 break;
@@ -1492,11 +1560,6 @@ __global__ __launch_bounds__(1024) void k_refit_top(const uint32_t* __restrict__
                 break;
             p = par;
         }
-    }
-    __syncthreads(); // the records' writes precede their reads
-    for (uint32_t k = t; k < n; k += 1024) {
-        const uint32_t p = tops[k];
-        tcone_trig(tcone, p - desc[mesh_search<true>(desc, M, p)].off);
     }
 }
 
@@ -1535,7 +1598,7 @@ hipError_t build_tree(snch_scene* s, uint32_t flags, uint32_t leaf_size, hipStre
             return e;            \
     } while (0)
     SNCH_TRY(w.leafbox.ensure(sizeof(float4) * 3 * N)); // the leaf records (box + cone)
-    SNCH_TRY(w.slabs.ensure(sizeof(uint32_t) * N)); // slab of the live node in each slot (k_refit)
+    SNCH_TRY(w.slabs.ensure(sizeof(uint32_t) * N)); // slabs of the leaves in sorted order (k_refit)
     SNCH_TRY(w.scene_bits.ensure(sizeof(int) * 8 * M));
     SNCH_TRY(w.boxpart.ensure(sizeof(float) * 8 * blocks(N)));
     SNCH_TRY(w.codes.ensure(sizeof(uint32_t) * N));
