@@ -977,7 +977,9 @@ int snch_batch_autotune(snch_scene* s, uint32_t kind, const float* q, const uint
             float ms = 0.0f;
             if ((err = measure(c, &ms)) == hipSuccess) {
                 ++cur.n_tried;
-                if (ms < best_ms) {
+                // depth 8 launches what depth 16 does: a second sample, no better choice
+                const bool same = axis == 1 && pool_cap(c.stack_depth) == pool_cap(start);
+                if (ms < best_ms && !same) {
                     best_ms = ms;
                     cur.block_size = c.block_size;
                     cur.stack_depth = c.stack_depth;

@@ -146,6 +146,15 @@ hipError_t query_order(const TreeView& t, int dim, const float* q, uint32_t n, Q
 size_t query_order_scratch_bytes(uint32_t n);
 hipError_t query_order_in(const TreeView& t, int dim, const float* q, uint32_t n, uint32_t* words, hipStream_t st,
                           const uint32_t** perm, uint32_t* err);
+// pool items of a wave for a stack depth option: 640 for the default of 16
+// (6,400 B of LDS per wave: 25 waves on a CU, above the 6 per SIMD that 80 VGPRs
+// allow).  A fuller pool pops
+// fewer items at a time (pool_take): closest silhouette on the 1M-triangle torus,
+// with 8-byte items, 62 ms with 480, 53 with 512, 42 with 640 (5 waves per
+// SIMD), 45 with 800 (4 waves).  Fewer than 640 starve it for no more waves
+// (320: 95 ms, closest point 142), so depth 8 gets 640 as well.
+constexpr uint32_t pool_cap(uint32_t depth) { return 40 * (depth > 16u ? depth : 16u); }
+
 // ctr (nullable; 8 words, zero at launch: clear_chunks, a kernel, so that capture is
 // fine): lets a large launch be persistent, and is needed where the number of
 // queries is on the device (t.n_dev)

@@ -175,14 +175,6 @@ __device__ __forceinline__ float scene_scale(const TreeView& t)
     return fmx(fmx(fmx(dm::fabs_(b.lo.x), dm::fabs_(b.hi.x)), fmx(dm::fabs_(b.lo.y), dm::fabs_(b.hi.y))),
                fmx(dm::fabs_(b.lo.z), dm::fabs_(b.hi.z)));
 }
-// pool items of a wave for a stack depth option: 640 for the default of 16
-// (6.2 KB of LDS per wave: 26 waves on a CU, above the 6 per SIMD that 80 VGPRs
-// allow).  A fuller pool pops
-// fewer items at a time (pool_take): closest silhouette on the torus below,
-// with 8-byte items, 62 ms with 480, 53 with 512, 42 with 640 (5 waves per
-// SIMD), 45 with 800 (4 waves).  Fewer than 640 starve it for no more waves
-// (320: 95 ms, closest point 142), so depth 8 gets 640 as well.
-constexpr uint32_t pool_cap(uint32_t depth) { return 40 * (depth > 16u ? depth : 16u); }
 // words of dynamic LDS of a wave
 constexpr uint32_t wave_lds_words(uint32_t cap, bool capped = false)
 {
