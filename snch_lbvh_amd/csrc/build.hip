@@ -80,8 +80,7 @@ __device__ __forceinline__ uint32_t mesh_search(const MeshDesc* __restrict__ d, 
     return lo;
 }
 
-// scene-box accumulators (+inf, -inf) of every mesh, 8 ints per mesh; slot 7:
-// the longest primitive edge, squared (ray queries)
+// scene-box accumulators (+inf, -inf) of every mesh, 8 ints per mesh
 // (and clears the list counters k_morton and k_karras append to, and the
 // radix sort's digit totals and tile counters)
 __global__ void k_init_scene_box(int* bits, uint32_t M, uint32_t* list_a, uint32_t* list_b, uint32_t* list_c,
@@ -104,14 +103,13 @@ __global__ void k_init_scene_box(int* bits, uint32_t M, uint32_t* list_a, uint32
     bits[t] = k < 3 ? f2ord(F_INF) : f2ord(-F_INF);
 }
 
-// block reduction of a scene box and the longest edge (v: NMIN minima, then
-// maxima): wave butterfly, then, when the whole block
+// block reduction of a scene box: wave butterfly, then, when the whole block
 // holds one mesh (always for a single mesh), the block's box in its partial
-// record part[8 b, 8 b + 8) (box slots 0-5, the mesh, the edge) for k_box_final;
+// record part[8 b, 8 b + 8) (box slots 0-5, then the mesh) for k_box_final;
 // else atomics per wave or per lane and a record marked INVALID.  Thousands
 // of workgroups updating the same six words one after the other would
 // serialise on them.
-template <int NV, int NMIN>
+template <int NV>
 __device__ __forceinline__ void reduce_scene_box(float (&v)[NV], uint32_t mesh, bool valid, int* scene_bits,
                                                  const int* slot_of, float* __restrict__ part)
 {
@@ -126,12 +124,12 @@ __device__ __forceinline__ void reduce_scene_box(float (&v)[NV], uint32_t mesh, 
         for (int o = 32; o > 0; o >>= 1) {
 #pragma unroll
             for (int k = 0; k < NV; ++k)
-                v[k] = k < NMIN ? fmn(v[k], __shfl_xor(v[k], o, 64)) : fmx(v[k], __shfl_xor(v[k], o, 64));
+                v[k] = k < NV / 2 ? fmn(v[k], __shfl_xor(v[k], o, 64)) : fmx(v[k], __shfl_xor(v[k], o, 64));
         }
     } else if (valid) {
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
-            if (k < NMIN)
+            if (k < NV / 2)
                 atomicMin(scene_bits + 8 * mesh + slot_of[k], f2ord(v[k]));
             else
                 atomicMax(scene_bits + 8 * mesh + slot_of[k], f2ord(v[k]));
@@ -153,7 +151,7 @@ __device__ __forceinline__ void reduce_scene_box(float (&v)[NV], uint32_t mesh, 
             same = same && redu[q] && redm[q] == redm[0];
         if (k == 7)
             rec[6] = __uint_as_float(same ? redm[0] : INVALID);
-        if (NMIN == 2 && k == 6) { // slots of z in 2D
+        if (NV == 4 && k == 6) { // slots of z in 2D
             rec[2] = F_INF;
             rec[5] = -F_INF;
         }
@@ -161,13 +159,13 @@ __device__ __forceinline__ void reduce_scene_box(float (&v)[NV], uint32_t mesh, 
             if (same) {
                 float acc = red[0][k];
                 for (int q = 1; q < BT / 64; ++q)
-                    acc = k < NMIN ? fmn(acc, red[q][k]) : fmx(acc, red[q][k]);
+                    acc = k < NV / 2 ? fmn(acc, red[q][k]) : fmx(acc, red[q][k]);
                 rec[slot_of[k]] = acc;
             } else {
                 for (int q = 0; q < BT / 64; ++q) {
                     if (!redu[q])
                         continue;
-                    if (k < NMIN)
+                    if (k < NV / 2)
                         atomicMin(scene_bits + 8 * redm[q] + slot_of[k], f2ord(red[q][k]));
                     else
                         atomicMax(scene_bits + 8 * redm[q] + slot_of[k], f2ord(red[q][k]));
@@ -185,19 +183,18 @@ constexpr uint32_t WAVE_EMPTY = 0xFFFFFFFEu; // no record of a mesh in the wave
 __global__ __launch_bounds__(BF) void k_box_final(const float* __restrict__ part, uint32_t n_part,
                                                   int* __restrict__ scene_bits)
 {
-    __shared__ float red[BF / 64][7];
+    __shared__ float red[BF / 64][6];
     __shared__ uint32_t redm[BF / 64]; // the wave's mesh, WAVE_EMPTY, or INVALID (mixed: already applied)
     const uint32_t i = blockIdx.x * BF + threadIdx.x;
     const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    auto slot = [](int k) { return k < 6 ? k : 7; }; // of a record and of the accumulators
     uint32_t mesh = INVALID;
-    float v[7] = {F_INF, F_INF, F_INF, -F_INF, -F_INF, -F_INF, -F_INF};
+    float v[6] = {F_INF, F_INF, F_INF, -F_INF, -F_INF, -F_INF};
     if (i < n_part) {
         mesh = __float_as_uint(part[8 * i + 6]);
         if (mesh != INVALID) {
 #pragma unroll
-            for (int k = 0; k < 7; ++k)
-                v[k] = part[8 * i + slot(k)];
+            for (int k = 0; k < 6; ++k)
+                v[k] = part[8 * i + k];
         }
     }
     const uint64_t live = __ballot(mesh != INVALID);
@@ -207,26 +204,26 @@ __global__ __launch_bounds__(BF) void k_box_final(const float* __restrict__ part
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
 #pragma unroll
-            for (int k = 0; k < 7; ++k)
+            for (int k = 0; k < 6; ++k)
                 v[k] = k < 3 ? fmn(v[k], __shfl_xor(v[k], o, 64)) : fmx(v[k], __shfl_xor(v[k], o, 64));
         }
     } else if (mesh != INVALID) {
 #pragma unroll
-        for (int k = 0; k < 7; ++k) {
+        for (int k = 0; k < 6; ++k) {
             if (k < 3)
-                atomicMin(scene_bits + 8 * mesh + slot(k), f2ord(v[k]));
+                atomicMin(scene_bits + 8 * mesh + k, f2ord(v[k]));
             else
-                atomicMax(scene_bits + 8 * mesh + slot(k), f2ord(v[k]));
+                atomicMax(scene_bits + 8 * mesh + k, f2ord(v[k]));
         }
     }
     if (lane == 0) {
 #pragma unroll
-        for (int k = 0; k < 7; ++k)
+        for (int k = 0; k < 6; ++k)
             red[w][k] = v[k];
         redm[w] = uni ? m0 : INVALID;
     }
     __syncthreads();
-    if (threadIdx.x < 7) {
+    if (threadIdx.x < 6) {
         const int k = threadIdx.x;
         uint32_t mb = WAVE_EMPTY;
         bool same = true;
@@ -244,18 +241,18 @@ __global__ __launch_bounds__(BF) void k_box_final(const float* __restrict__ part
                 if (redm[q] != WAVE_EMPTY)
                     acc = k < 3 ? fmn(acc, red[q][k]) : fmx(acc, red[q][k]);
             if (k < 3)
-                atomicMin(scene_bits + 8 * mb + slot(k), f2ord(acc));
+                atomicMin(scene_bits + 8 * mb + k, f2ord(acc));
             else
-                atomicMax(scene_bits + 8 * mb + slot(k), f2ord(acc));
+                atomicMax(scene_bits + 8 * mb + k, f2ord(acc));
         } else if (!same) {
             for (int q = 0; q < BF / 64; ++q) {
                 const uint32_t mq = redm[q];
                 if (mq == WAVE_EMPTY || mq == INVALID)
                     continue;
                 if (k < 3)
-                    atomicMin(scene_bits + 8 * mq + slot(k), f2ord(red[q][k]));
+                    atomicMin(scene_bits + 8 * mq + k, f2ord(red[q][k]));
                 else
-                    atomicMax(scene_bits + 8 * mq + slot(k), f2ord(red[q][k]));
+                    atomicMax(scene_bits + 8 * mq + k, f2ord(red[q][k]));
             }
         }
     }
@@ -315,10 +312,8 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
     b.hi = mk(-F_INF, -F_INF, -F_INF);
     uint32_t e0 = 0, my = 0;
     v3 c = mk(0.0f, 0.0f, 0.0f);
-    float edge2 = 0.0f;
     if (i < nF) {
         const v3 p0 = ld3(V, F[3 * i]), p1 = ld3(V, F[3 * i + 1]), p2 = ld3(V, F[3 * i + 2]);
-        edge2 = fmx(sqlen3(sub(p1, p0)), fmx(sqlen3(sub(p2, p1)), sqlen3(sub(p0, p2))));
         b = box_of_point(p0);
         box_expand(b, p1);
         box_expand(b, p2);
@@ -459,10 +454,10 @@ __global__ __launch_bounds__(BT) void k_leafgen(const float4* __restrict__ V, co
         leafrec[3 * i + 1] = make_float4(b.hi.y, b.hi.z, r.axis.x, r.axis.y);
         leafrec[3 * i + 2] = make_float4(r.axis.z, r.half_angle, r.radius, __uint_as_float(excess));
     }
-    // scene AABB of the primitive's mesh, and its longest edge
-    float v[7] = {b.lo.x, b.lo.y, b.lo.z, b.hi.x, b.hi.y, b.hi.z, edge2};
-    const int slot_of[7] = {0, 1, 2, 3, 4, 5, 7};
-    reduce_scene_box<7, 3>(v, mesh, i < nF, scene_bits, slot_of, part);
+    // scene AABB of the primitive's mesh
+    float v[6] = {b.lo.x, b.lo.y, b.lo.z, b.hi.x, b.hi.y, b.hi.z};
+    const int slot_of[6] = {0, 1, 2, 3, 4, 5};
+    reduce_scene_box<6>(v, mesh, i < nF, scene_bits, slot_of, part);
 }
 
 // scene<2>: leaf box (scene.cuh:420-433) and leaf cone from the owned
@@ -480,10 +475,8 @@ __global__ __launch_bounds__(BT) void k_leafgen2d(const float4* __restrict__ V, 
     box3 b;
     b.lo = mk(F_INF, F_INF, 0.0f);
     b.hi = mk(-F_INF, -F_INF, 0.0f);
-    float edge2 = 0.0f;
     if (i < nS) {
         const v3 p0 = ld3(V, S[2 * i]), p1 = ld3(V, S[2 * i + 1]);
-        edge2 = sqlen3(sub(p1, p0));
         b = seg_box(p0, p1);
         const v3 c = box_centroid(b);
         float ax = 0.0f, ay = 0.0f, ha = F_PI, rad = 0.0f;
@@ -556,9 +549,9 @@ __global__ __launch_bounds__(BT) void k_leafgen2d(const float4* __restrict__ V, 
         leafrec[3 * i + 1] = make_float4(b.hi.y, 0.0f, ax, ay);
         leafrec[3 * i + 2] = make_float4(0.0f, ha, rad, 0.0f);
     }
-    float v[5] = {b.lo.x, b.lo.y, b.hi.x, b.hi.y, edge2};
-    const int slot_of[5] = {0, 1, 3, 4, 7};
-    reduce_scene_box<5, 2>(v, mesh, i < nS, scene_bits, slot_of, part);
+    float v[4] = {b.lo.x, b.lo.y, b.hi.x, b.hi.y};
+    const int slot_of[4] = {0, 1, 3, 4};
+    reduce_scene_box<4>(v, mesh, i < nS, scene_bits, slot_of, part);
 }
 
 // bvh.cuh:269-277 and morton_code.cuh:85-92

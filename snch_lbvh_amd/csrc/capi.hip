@@ -746,7 +746,7 @@ int snch_ray_ex(const snch_scene* s, const float* o, const float* d, const float
 {
     SNCH_NEED_SINGLE(s, "snch_ray");
     SNCH_CHECK_ARG(n == 0 || (o && d && out_hit), "snch_ray: null pointer");
-    SNCH_HIP(launch_ray(s->view(), (int)s->dim, s->dV.as<float4>(), s->dF.as<int32_t>(), s->edge2(), o, d, tmax, n, any_hit,
+    SNCH_HIP(launch_ray(s->view(), (int)s->dim, s->dV.as<float4>(), s->dF.as<int32_t>(), o, d, tmax, n, any_hit,
                         out_hit, out_t, out_uv, out_idx, opts ? opts->stats : nullptr, nullptr, s->n_cu(),
                         static_cast<hipStream_t>(stream)),
              "snch_ray");

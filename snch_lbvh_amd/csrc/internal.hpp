@@ -102,8 +102,6 @@ struct snch_scene {
     mutable bool scratch_used = false;
     ~snch_scene();
     snch::TreeView view(uint32_t mesh = 0) const;
-    // the (first) mesh's longest edge, squared (device memory, from the last build)
-    const float* edge2() const { return scratch.scene_bits.as<float>() + 7; }
 };
 
 namespace snch {
@@ -175,11 +173,9 @@ hipError_t launch_closest_silhouette(const TreeView& t, int dim, const float* q,
 hipError_t clear_chunks(uint32_t* ctr, hipStream_t st);
 // whether a launch of that shape is persistent (it uses ctr then)
 bool silhouette_persists(uint32_t n, uint32_t block, uint32_t depth, bool hard, uint32_t n_cu);
-// edge2: the mesh's longest edge, squared (snch_scene::edge2)
-hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* edge2,
-                      const float* o, const float* d, const float* tmax, uint32_t n, int any_hit, uint8_t* hit,
-                      float* tout, float* uv, uint32_t* idx, uint64_t* stats, uint32_t* ctr, uint32_t n_cu,
-                      hipStream_t st);
+hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* o, const float* d,
+                      const float* tmax, uint32_t n, int any_hit, uint8_t* hit, float* tout, float* uv, uint32_t* idx,
+                      uint64_t* stats, uint32_t* ctr, uint32_t n_cu, hipStream_t st);
 hipError_t launch_sample(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* c,
                          const float* r, const float* u, uint32_t n, int32_t* idx, float* pdf, float* pt,
                          hipStream_t st);

@@ -71,11 +71,11 @@ __global__ __launch_bounds__(512, 6) void k_closest_point(TreeView t, const floa
 }
 
 // ------------------------------------------------------------ ray
-// edge2: the mesh's longest edge, squared.  out_uv: the hit's barycentrics (2D:
-// the segment parameter), from the hit test of the triangle found
+// out_uv: the hit's barycentrics (2D: the segment parameter), from the hit
+// test of the triangle found
 template <bool STATS, int DIM, bool ANY>
 __global__ __launch_bounds__(64, 6) void k_ray(TreeView t, const float4* __restrict__ V, const int32_t* __restrict__ F,
-                                               const float* __restrict__ edge2, const float* __restrict__ o, const float* __restrict__ d,
+                                               const float* __restrict__ o, const float* __restrict__ d,
                                                const float* __restrict__ tmax, uint32_t n, uint32_t deal,
                                                uint8_t* __restrict__ out_hit, float* __restrict__ out_t,
                                                float* __restrict__ out_uv, uint32_t* __restrict__ out_idx,
@@ -88,7 +88,6 @@ __global__ __launch_bounds__(64, 6) void k_ray(TreeView t, const float4* __restr
         n = min(n, *t.n_dev);
     if (deal == 0u)
         deal = deal_queries(n, gridDim.x, RAY_RUNS);
-    const float edge = HwMath::sqrt(*edge2) * 1.00001f;
     bool ovf = false;
     Counts cnt;
     for_chunks(n, deal, ctr, [&](uint32_t qi, bool valid) {
@@ -102,7 +101,7 @@ __global__ __launch_bounds__(64, 6) void k_ray(TreeView t, const float4* __restr
             // aabb.cuh:308-311 (2D: z slab inert)
             W.start(lane, ro, rd, mk(1.0f / rd.x, 1.0f / rd.y, 1.0f / rd.z), max_dist);
         }
-        ray_wave<STATS, DIM, ANY>(t, __ballot(valid), max_dist, edge, W, cnt, ovf);
+        ray_wave<STATS, DIM, ANY>(t, __ballot(valid), max_dist, W, cnt, ovf);
         if (!valid)
             return;
         float tbest;
@@ -437,10 +436,9 @@ hipError_t launch_closest_point(const TreeView& t, int dim, const float* q, uint
     return hipGetLastError();
 }
 
-hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* edge2,
-                      const float* o, const float* d, const float* tmax, uint32_t n, int any_hit, uint8_t* hit,
-                      float* tout, float* uv, uint32_t* idx, uint64_t* stats, uint32_t* ctr, uint32_t n_cu,
-                      hipStream_t st)
+hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t* F, const float* o, const float* d,
+                      const float* tmax, uint32_t n, int any_hit, uint8_t* hit, float* tout, float* uv, uint32_t* idx,
+                      uint64_t* stats, uint32_t* ctr, uint32_t n_cu, hipStream_t st)
 {
     if (n == 0)
         return hipSuccess;
@@ -448,7 +446,7 @@ hipError_t launch_ray(const TreeView& t, int dim, const float4* V, const int32_t
     const SearchGrid g = search_grid(n, 64, RayLds::WORDS, n_cu, 6, ctr != nullptr, t.n_dev != nullptr, RAY_RUNS);
     uint32_t* c = g.persist ? ctr : nullptr;
 #define SNCH_RAY(S_, A_)                                                                                             \
-    hipLaunchKernelGGL((k_ray<S_, DIM, A_>), g.grid, g.block, 0, st, t, V, F, edge2, o, d, tmax, n, g.deal, hit, tout, uv, idx, \
+    hipLaunchKernelGGL((k_ray<S_, DIM, A_>), g.grid, g.block, 0, st, t, V, F, o, d, tmax, n, g.deal, hit, tout, uv, idx, \
                        c, traversal_error_word(), sp)
     SNCH_DISPATCH_DIM(dim, {
         if (any_hit) {

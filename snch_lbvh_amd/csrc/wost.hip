@@ -337,7 +337,7 @@ hipError_t enqueue_steps(snch_wost* s, uint32_t max_steps, float eps, uint64_t s
         hipLaunchKernelGGL(k_star, dim3(nb), dim3(256), 0, st, s->w, cur, cap, s->dir->dV.as<float4>(),
                            s->dir->dF.as<int32_t>(), eps, seed, has_n);
         if (has_n) {
-            if ((e = launch_ray(vn, 3, s->neu->dV.as<float4>(), s->neu->dF.as<int32_t>(), s->neu->edge2(), s->w.ray_o, s->w.ray_d,
+            if ((e = launch_ray(vn, 3, s->neu->dV.as<float4>(), s->neu->dF.as<int32_t>(), s->w.ray_o, s->w.ray_d,
                                 s->w.star_r, cap, 0, s->w.ray_hit, s->w.ray_t, nullptr, s->w.ray_idx, nullptr,
                                 s->chunk_ctr.as<uint32_t>() + 16, n_cu, st)) != hipSuccess)
                 return e;
