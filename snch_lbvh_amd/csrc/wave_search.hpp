@@ -811,10 +811,24 @@ __device__ inline void lane_ray(const TreeView& t, v3 ro, v3 rd, v3 inv, float m
     }
 }
 
+// 2D: a segment is hit up to 1e-3 of its length past its ends, where its box ends
+// BVH_OFFSET past them: a ray may hit a segment longer than 1 (at most the
+// scene's diagonal) up to this much before it enters its box, by the distance
+// along the ray's reciprocals, and at most the time it takes across the scene.
+// 2^20 rays on 20,000 segments of a curve: 0.242 -> 0.249 ms, on 2,000 of a soup
+// 0.69 -> 0.74.
+__device__ __forceinline__ float past_end(v3 inv, float scale)
+{
+    auto finite = [](float x) { return dm::fabs_(x) < F_INF ? dm::fabs_(x) : 0.0f; };
+    const float length = 2.83f * scale, r = 1.01e-3f * length;
+    return fmn(r * fmx(finite(inv.x), finite(inv.y)),
+               (length + r + 4.0f * BVH_OFFSET) * 1.00001f * fmn(dm::fabs_(inv.x), dm::fabs_(inv.y)));
+}
+
 // tests the last (up to 64) leaves of the wave's buffer; returns how many are
 // left.  A hit at t becomes a candidate of its ray, whose bound falls to a
 // little more than t (the rounding of box and triangle parameters: see the
-// hidden leaves above); any hit ends the ray with ANY.  Where a ray grazes a
+// hidden leaves above; in 2D past_end too); any hit ends the ray with ANY.  Where a ray grazes a
 // sliver, rounding knows no such bound: a triangle is hit while its determinant
 // is FLT_EPSILON, and the parameter computed for it may be any amount before its
 // box.  The lone search reports such a hit if it happens to meet that leaf before
@@ -847,7 +861,8 @@ __device__ __forceinline__ uint32_t ray_leaves(const TreeView& t, RayLds& W, uin
                     atomicMin(&W.bound[slot],
                               __float_as_uint(th * 1.0001f +
                                               1e-5f * fmx(scale, fmx(dm::fabs_(o.x),
-                                                                     fmx(dm::fabs_(o.y), dm::fabs_(o.z))))));
+                                                                     fmx(dm::fabs_(o.y), dm::fabs_(o.z)))) +
+                                              (DIM == 2 ? past_end(W.inv(slot), scale) : 0.0f)));
             }
         }
     }
