@@ -366,13 +366,14 @@ SNCH_HD uint32_t slab_merge(const cone3& r, const box3& b, const cone3& k0, uint
 // half angle with its excess, |n.(x - o)| >= cos(t) h - sin(t) q for every
 // normal n.  The predicate treats |n.(x - o)| <= 1e-3 as grazing, and distances
 // up to 1e-3 apart: hence the margin.  An excess e takes at most
-// sqrt(h^2 + q^2) e <= 1.42 (l + reach) e away; 5e-4 more of that length covers
+// sqrt(h^2 + q^2) e <= 1.42 (|s| + q) e away (s: the centre's height over o); 5e-4
+// more of that length, which is at least that from o to any of the box, covers
 // the excess that is not counted (64 levels of 5e-6) and the rounding of these
 // sums.  The view-cone test (cone_overlap) takes all of the bounding sphere for
 // the edges; a patch of surface is a thin slab of it.  On the 1M-triangle torus
 // 808 -> 495 nodes per query, 2^22 queries 34.0 -> 20.7 ms, walk on stars 61 ->
 // 46 ms (2^17 walks); rough meshes (noise above the edge length) gain nothing and
-// pay about 2 %.  One margin for all cones, without the excess of each: 2e-3 of
+// pay about 1 %.  One margin for all cones, without the excess of each: 2e-3 of
 // the length (too little for a chain of tilted merges) 22.0 ms, 4e-3 23.2, 8e-3
 // 24.1, 2e-2 27.8.
 template <class AM = HwMath>
@@ -387,7 +388,7 @@ SNCH_HD bool cone_slab_clear(v3 axis, float half_angle, float sin_ha, float cos_
     unpack_slab(slab, radius, reach, mid, half);
     const float h = dm::fabs_(s + mid) - half, q = AM::sqrt(fmx(l2 - s * s, 0.0f)) + reach;
     return half_angle < F_PI_2 && e < SLAB_LOST &&
-           cos_ha * h - sin_ha * q > 1.05e-3f + (5e-4f + 1.42f * SLAB_UNIT * (float)e) * (AM::sqrt(l2) + reach);
+           cos_ha * h - sin_ha * q > 1.05e-3f + (5e-4f + 1.42f * SLAB_UNIT * (float)e) * (dm::fabs_(s) + q);
 }
 
 // Rodrigues rotation (cone.cuh:288-302).  When the axes are (anti)parallel the
