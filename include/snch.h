@@ -75,11 +75,13 @@ typedef struct snch_query_opts {
                             visited, cone records read (silhouette query only) */
     const uint32_t *order; /* optional DEVICE permutation of [0, n) (e.g. from
                               snch_query_order): the visiting order; overrides coherent */
-    uint32_t stack_depth;      /* LDS of a wavefront's pool of pending nodes, 40 nodes per unit and at least 640:
-                                  closest point 8 or 16 (0 = 16), closest silhouette (3D) and
-                                  batched queries 8, 16, 24 or 32 (0 = 16).  Outputs are the same. */
+    uint32_t stack_depth;      /* LDS of a wavefront's pool of pending nodes, 40 nodes per unit and at least 640
+                                  (so 8 launches what 16 does): closest point 8 or 16 (0 = 16),
+                                  closest silhouette (3D) and batched queries 8, 16, 24 or 32
+                                  (0 = 16).  Outputs are the same. */
     uint32_t queries_per_wave; /* batched queries: queries a wavefront takes from the work
-                                  queue at a time, a multiple of 64 up to 4096 (0 = 64) */
+                                  queue at a time, a multiple of 64 up to 4096 (0 = 64); where the
+                                  batch has too few for that to fill the GPU, in proportion fewer */
     uint32_t seed_is_cap;      /* closest silhouette: 1 = seed_radius is a hard search radius
                                   (the answer is exact when it lies within the radius; otherwise
                                   the returned distance exceeds the radius, possibly +inf) */
@@ -220,6 +222,7 @@ int snch_batch_closest_silhouette(const snch_scene *scene, const float *q, const
  * 256}, each axis swept with the others at their best so far; one warm-up
  * and one HIP-event-timed launch per configuration over all queries
  * (sample_per_mesh = 0) or the first sample_per_mesh queries of each mesh.
+ * Depth 8, which launches what 16 does, is timed but never chosen.
  * Leaves the scene built with the best leaf size.  Pass the result's
  * block_size, stack_depth and queries_per_wave in snch_query_opts.
  * Synchronises. */
@@ -322,8 +325,8 @@ int snch_wost_solve(snch_wost *wost, const float *x0, uint32_t n, uint32_t max_s
  * SNCH_NOALLOC_MAX_QUERIES is rejected with SNCH_ERR_INVALID.  Every call on a
  * GPU shares that GPU's array, so calls that overlap on one GPU (other
  * streams, other threads) race and must be serialised by the caller.  With a
- * seed radius, queries not settled within it are searched again at once by
- * their own lane (snch_query_opts.seed_retry = 1), which needs no queue. */
+ * seed radius, queries not settled within it enter their wavefront's search
+ * again without it, as in snch_closest_silhouette, which needs no queue. */
 #define SNCH_NOALLOC_MAX_QUERIES (1u << 22)
 int snch_closest_silhouette_noalloc(const snch_scene *scene, const float *q, uint32_t n, int flip,
                                     const float *seed_radius, uint32_t *out_sil, float *out_dist, void *stream);

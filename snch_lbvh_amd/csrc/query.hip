@@ -1,9 +1,10 @@
 // Query kernels for triangle scenes on gfx950: closest primitive, closest
 // silhouette, ray (closest hit / any hit) and SampleTriangleInSphere.
 //
-// One lane = one query (the reference: one thread per query through
-// query_device, query.cuh:79-423, and sample_object_in_sphere,
-// sample.cuh:23-92).  Differences in HOW, not WHAT:
+// The reference runs one thread per query (query_device, query.cuh:79-423, and
+// sample_object_in_sphere, sample.cuh:23-92).  Here the searches run up to 64
+// queries per wave from a pool; the sampler and the generic overlap and line
+// queries keep one lane per query.  Differences in HOW, not WHAT:
 //  * Node layout: one 64-B record per internal node holds both children's
 //    boxes and references, 32 B each; the silhouette query reads a cone record
 //    from a separate stream, so the closest-point and ray queries never touch

@@ -25,7 +25,8 @@ namespace snch {
 //             cones, 32 B each, read only by the silhouette query:
 //               [0] L.axis L.half_angle  [1] sin, cos of L.half_angle, L.radius, L.slab
 //               [2] R.axis R.half_angle  [3] sin, cos of R.half_angle, R.radius, R.slab
-//             slab: the extent of the child's edges along the axis (pack_slab)
+//             slab: the extent of the child's edges along the axis, and by how much
+//             their face normals may lie outside the half angle (pack_slab)
 //   tleaf[j]  3 x float4 = 48 B per leaf, in Morton (sorted) order:
 //               [k] vertex k xyz, w = (original triangle, first owned edge,
 //               owned edge count) for k = 0, 1, 2

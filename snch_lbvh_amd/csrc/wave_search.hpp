@@ -59,9 +59,10 @@ __device__ __forceinline__ void flush_counts(const Counts& c, unsigned long long
 // this file now).  Closest point: 2^22 queries on 2^20 triangles 46 -> 18.5 ms,
 // 65,536 on 20,480 triangles 2.1 -> 0.12 ms, 1,000 0.83 -> 0.03 ms (there a
 // launch lasted as long as the longest chain of dependent loads, about 2 us a
-// node).  Closest silhouette: 2^22 on 2^20 triangles 68 -> 22.5 ms, 10,007 on
+// node).  Closest silhouette: 2^22 on 2^20 triangles 68 -> 20.7 ms, 10,007 on
 // 90,000 triangles 4.3 -> 0.13 ms.  Pairs that keep their near child in
-// registers instead of the pool: half as long again.  For those 2^22 queries:
+// registers instead of the pool: half as long again.  For those 2^22 queries,
+// while they took 22.6 ms:
 // SIL_ADD 12 / 20 / 26 / 32 / 40 / 64: 26.7 / 25.7 / 24.7 / 22.6 / 24.5 / 25.0
 // ms; CP_ADD 16 to 24: within 1%; runs of 24 / 32 / 40 / 48 / 64 leaves: closest
 // point 22.0 / 21.0 / 20.1 / 19.7 / 19.3, silhouette 25.2 / 25.2 / 25.7 / 25.9 /
@@ -69,7 +70,8 @@ __device__ __forceinline__ void flush_counts(const Counts& c, unsigned long long
 //
 // The answer is that of the search one lane would make alone, near child
 // first, each node's leaves at once, which skips a box as soon as its lower
-// bound exceeds the best distance so far (lane_nearest below).  Where no
+// bound exceeds the best distance so far (lane_nearest below); rays that graze a
+// face within rounding excepted (ray_leaves).  Where no
 // rounding interferes that is the smallest (distance, id) of all leaves,
 // whatever the order.  But a leaf's computed distance can lie below its box's
 // computed lower bound by a few units in the last place of the coordinates
@@ -689,8 +691,13 @@ __device__ __forceinline__ void sil_wave(const TreeView& t, uint64_t all, bool f
 // ------------------------------------------------------------ rays
 
 // LDS of a wave's rays: as WaveLds, with the origin, the reciprocal and the
-// direction per query slot.  A ray visits few nodes (20 on the 1M-triangle
-// torus), so all 64 of a wave enter at once and a smaller pool does.
+// direction per query slot, and so a smaller pool, which does: a ray visits few
+// nodes (20 on the 1M-triangle torus).  2^22 random rays at that torus / a camera's
+// at the torus over a ground plane / random ones at 64 tori over it, in ms: as it
+// is 1.00 / 2.62 / 4.84; a pool of 256 1.00 / 6.62 / 4.89, of 512 (21 waves per CU)
+// 1.07 / 2.82 / 4.87; RAY_ADD 16 / 24 / 48 / 64: 1.00 / 2.86 / 5.22, 1.01 / 3.02 /
+// 5.30, 1.02 / 2.87 / 5.31, 1.02 / 2.90 / 5.38; RAY_LEAF_RUN 16 / 40: 1.01 / 2.53 /
+// 4.61, 1.01 / 2.77 / 5.21, but 2D rays (the soup of 2,000 segments: 0.72) 0.75 / 0.68.
 constexpr uint32_t RAY_LEAF_RUN = 24, RAY_ADD = 32;
 struct RayLds {
     unsigned long long* best; // (t, triangle)
